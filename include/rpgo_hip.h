@@ -326,9 +326,12 @@ int rpgo_pcm_batch_run(rpgo_ctx* ctx, const rpgo_pcm_batch* batch, const rpgo_pc
 int rpgo_pcm_batch_download_adj(rpgo_ctx* ctx, int32_t g, uint64_t* adj_bits);
 
 /* ------------------------------------------------------------------------
- * Robust solve: GNC-TLS over Levenberg-Marquardt / Gauss-Newton with a PCG
- * linear step (block-tridiagonal segment preconditioner along the odometry
- * chain plus a rigid-segment coarse level).  Replaces RobustSolver::optimize
+ * Robust solve: GNC-TLS over Levenberg-Marquardt / Gauss-Newton.  The linear
+ * step is a sparse block Cholesky solve in FP64 (the reference's own kind of
+ * step); graphs whose elimination fills in too much, singular systems and
+ * calls that choose a preconditioner (pcg_segment > 0 or pcg_coarse != 0) take
+ * a PCG (block-tridiagonal segment preconditioner along the odometry chain
+ * plus a rigid-segment coarse level).  Replaces RobustSolver::optimize
  * (src/RobustSolver.cpp:115-306): gtsam::GncOptimizer with known inliers
  * (:105-113, :130-180, :225-275) or plain LevenbergMarquardtOptimizer /
  * GaussNewtonOptimizer (:181-218, :276-296).  SE(3) poses only.
@@ -403,7 +406,8 @@ typedef struct {
 typedef struct {
   int32_t gnc_iterations;
   int32_t lm_iterations;
-  int32_t pcg_iterations;
+  int32_t pcg_iterations;       /* PCG iterations; a direct solve counts 1 and
+                                   each refinement of it 1              */
   int32_t linearizations;
   double mu_init;
   double mu_final;

@@ -3,6 +3,7 @@
 
 #include <cstring>
 
+#include "direct_plan.h"
 #include "rpgo_internal.h"
 
 namespace rpgo {
@@ -12,6 +13,20 @@ constexpr int kCoarseSegMax = 256;  // rigid segments of the coarse precondition
 constexpr int kCoarseSegSmall = 128;  // default below kCoarseLargeN poses
 constexpr int kCoarseLargeN = 10000;  // poses from which the default is kCoarseSegMax
 constexpr int kCoarseMax = 6 * kCoarseSegMax;
+// A direct solve is refined to this relative residual (or pcg_rel_tol where
+// that is smaller), in at most kDirectRefine steps.  A factorization's
+// residual is rounding spread over every mode, so the soft modes of a long
+// chain need it smaller than a PCG's: 50,000 poses with 1,600 loop closures
+// stopped 1.4e-7 (relative) from the converged steps at 1e-6, 5e-9 at 1e-10.
+constexpr double kDirectTol = 1e-10;
+constexpr int kDirectRefine = 3;
+// From this many poses the last step of a nonlinear solve gets one more
+// refinement.  The factor takes damping and diagonal rounded to one FP64
+// number, an error of about 1e-16 of the diagonal with the same sign at every
+// pose; along the softest mode of 50,000 poses that shortens a step by 8e-5,
+// 3e-8 of the poses when it is the last (earlier steps' errors are corrected
+// by the later ones).  Below, the bias is far under the solve's 1e-10.
+constexpr int kDirectFinishMin = 8192;
 
 struct GraphKey {
   int N = 0, S = 0, Sc = 0, nseg_c = 0;
@@ -57,6 +72,13 @@ struct SolverRun {
   hipGraphExec_t graph_exec = nullptr;  // captured PCG chunk
   GraphKey graph_key;
   bool use_graphs = true;
+  // direct solve (direct.hip): the plan of the current problem, its device
+  // copy, and the factor's storage
+  bool direct_ready = false;
+  DirectPlan plan;
+  double last_residual = 0.0;      // relative residual of the last direct solve
+  DevBuf d_meta, d_childs, d_origs, d_nb, d_maps, d_lvl;
+  DevBuf d_U, d_G, d_L, d_Y, d_part, d_bad;
   // pinned host buffers of this run's readbacks (scalars; one PCG chunk's
   // residual history), allocated on first use
   double* h_scalars = nullptr;
@@ -77,7 +99,18 @@ struct SolverRun {
   int read_scalars(hipStream_t st, int count, double* out);
   double* pinned_scalars();
   double* pinned_history();
-  int run(hipStream_t st, rpgo_solve_report* rep);
+  void retract(hipStream_t st);
+  void cost_partials(hipStream_t st, const double* xp, double* part);
+  int direct_setup(hipStream_t st, const int32_t* h_kind, const int32_t* h_fi, const int32_t* h_fj);
+  int direct_factor(hipStream_t st, double lambda);
+  int direct_backward(hipStream_t st, double* out);
+  int direct_check(hipStream_t st, double lambda);
+  int direct_refine(hipStream_t st);
+  int direct_step(hipStream_t st, double lambda, double* lin, double* cost_new, bool* ok);
+  int direct_finish(hipStream_t st, double lambda, double* cost_new);
+  bool last_step(double cur, double nw, int it) const;
+  int direct_cost(hipStream_t st, const double* xp, double* out);
+  int run(hipStream_t st, const rpgo_solve_problem* pr, rpgo_solve_report* rep);
   double* cost_buf() { return cost.as<double>(); }
   void release() {
     if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
@@ -89,7 +122,8 @@ struct SolverRun {
                       &Hjj, &Hij, &gi, &gj, &inc_off, &inc_cnt, &inc, &inc_q, &D, &Minv, &hdiag, &b64,
                       &chain, &Useg, &Ds, &Cs, &ext_off, &ext, &ext_q, &Pb, &Ac, &Lci, &LcT, &Ainv, &cres,
                       &ccor,
-                      &dx, &r, &zv, &p, &q, &hx, &sc})
+                      &dx, &r, &zv, &p, &q, &hx, &sc, &d_meta, &d_childs, &d_origs, &d_nb, &d_maps, &d_lvl,
+                      &d_U, &d_G, &d_L, &d_Y, &d_part, &d_bad})
       v->release();
   }
 };

@@ -28,6 +28,7 @@
 #include "replay64.h"
 #include "rpgo_internal.h"
 #include "rpgo_solver.h"
+#include "solver_device.h"
 
 namespace rpgo {
 
@@ -279,6 +280,28 @@ __global__ void k_factor_errors(int F, const int* __restrict__ kind, const int* 
   err[f] = 0.5 * quad6(e, info + (size_t)f * 36);
 }
 
+// The same with the weighted sum: part[b] = sum of w err over workgroup b's
+// factors (256 each), in a fixed order.
+__global__ void __launch_bounds__(256) k_factor_cost(int F, const int* __restrict__ kind, const int* __restrict__ fi,
+                                                     const int* __restrict__ fj, const double* __restrict__ z,
+                                                     const double* __restrict__ info, const double* __restrict__ w,
+                                                     const double* __restrict__ x, double* __restrict__ err, int chart,
+                                                     double* __restrict__ part) {
+  __shared__ double red[16];
+  const int f = blockIdx.x * 256 + threadIdx.x;
+  double c = 0.0;
+  if (f < F) {
+    double e[6];
+    const int k = kind[f];
+    factor_error(k, x + (size_t)fi[f] * 12, x + (size_t)(k == 0 ? fj[f] : fi[f]) * 12, z + (size_t)f * 12, e, chart);
+    c = 0.5 * quad6(e, info + (size_t)f * 36);
+    err[f] = c;
+    c *= w[f];
+  }
+  c = block_sum(c, red);
+  if (threadIdx.x == 0) part[blockIdx.x] = c;
+}
+
 // per-factor Gauss-Newton contributions: blocks, gradients and cost (FP64)
 // 64-thread workgroups (the launch shape): the register budget of one
 // wavefront per SIMD.  The products are formed in an order that keeps at
@@ -490,47 +513,6 @@ __global__ void k_assemble(int N, const int* __restrict__ off, const int* __rest
 // poses (block LDL^T, one thread per segment), dropping the loop-closure
 // blocks and the coupling across segment borders.  S = 1 is block-Jacobi.
 // ---------------------------------------------------------------------------
-
-// DPP row rotation of an FP64 value (both halves), all lanes of the row valid
-template <int N>
-__device__ __forceinline__ double row_ror_f64(double v) {
-  const int lo = __double2loint(v), hi = __double2hiint(v);
-  return __hiloint2double(__builtin_amdgcn_update_dpp(0, hi, 0x120 + N, 0xF, 0xF, false),
-                          __builtin_amdgcn_update_dpp(0, lo, 0x120 + N, 0xF, 0xF, false));
-}
-
-__device__ __forceinline__ double readlane_f64(double v, int lane) {
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                          __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
-
-// Sum over the 64 lanes of a converged wavefront, in every lane: rotations
-// within each row of 16 lanes by DPP (VALU, a few cycles each), then the four
-// row sums by v_readlane.  A six-step shuffle reduction went through the LDS
-// crossbar (ds_bpermute) at every step, on the critical path of each PCG
-// launch.
-__device__ __forceinline__ double wave_sum_pre(double v) {
-  v += row_ror_f64<8>(v);
-  v += row_ror_f64<4>(v);
-  v += row_ror_f64<2>(v);
-  v += row_ror_f64<1>(v);
-  return (readlane_f64(v, 0) + readlane_f64(v, 16)) + (readlane_f64(v, 32) + readlane_f64(v, 48));
-}
-
-// block-wide FP64 sum (all threads call it; the result is valid in thread 0)
-__device__ __forceinline__ double block_sum(double v, double* lds16) {
-  v = wave_sum_pre(v);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) lds16[wid] = v;
-  __syncthreads();
-  double t = 0.0;
-  if (threadIdx.x < 64) {
-    t = threadIdx.x < (blockDim.x >> 6) ? lds16[threadIdx.x] : 0.0;
-    t = wave_sum_pre(t);
-  }
-  return t;  // valid in thread 0
-}
 
 // chain[k] = 2 f + flip for the first odometry factor joining k and k+1
 // (flip = 1 when the factor runs k+1 -> k), -1 when none
@@ -1959,6 +1941,19 @@ int SolverRun::linearize(hipStream_t st) {
   return RPGO_OK;
 }
 
+// xn = x retracted by dx
+void SolverRun::retract(hipStream_t st) {
+  k_retract<<<grid_for(N, 128, 1 << 22), 128, 0, st>>>(N, x.as<double>(), dx.as<double>(), xn.as<double>(),
+                                                       prm.pose2_chart);
+}
+
+// factor errors at xp and the weighted cost's ceil(F / 256) partial sums
+void SolverRun::cost_partials(hipStream_t st, const double* xp, double* part) {
+  k_factor_cost<<<(unsigned)((F + 255) / 256), 256, 0, st>>>(F, kind.as<int>(), fi.as<int>(), fj.as<int>(),
+                                                             z.as<double>(), info.as<double>(), w.as<double>(), xp,
+                                                             err.as<double>(), prm.pose2_chart, part);
+}
+
 // y = (H + lambda damp) x
 void SolverRun::spmv(hipStream_t st, double lambda, const double* xin, double* yout) {
   k_spmv<<<grid_for(N, 128, 1 << 22), 128, 0, st>>>(
@@ -2230,13 +2225,18 @@ static bool lm_converged(const rpgo_solve_params& p, double cur, double nw) {
   return (dec / cur <= p.lm_relative_error_tol) || (dec <= p.lm_absolute_error_tol);
 }
 
+// Whether the accepted step that took the cost to nw ends the run
+bool SolverRun::last_step(double cur, double nw, int it) const {
+  return it >= prm.lm_max_iterations || lm_converged(prm, cur, nw);
+}
+
 // One LevenbergMarquardtOptimizer / GaussNewtonOptimizer run from x0 with the
 // current weights; leaves the result in x and its weighted cost in *cost_out.
 int SolverRun::nonlinear_solve(hipStream_t st, bool from_x0, double* cost_out, int* iters_out) {
   int rc;
   if (from_x0) RPGO_HIP_CHECK(hipMemcpyAsync(x.ptr, x0.ptr, sizeof(double) * 12 * N, hipMemcpyDeviceToDevice, st));
   double err;
-  if ((rc = total_cost(st, x.as<double>(), &err))) return rc;
+  if ((rc = direct_ready ? direct_cost(st, x.as<double>(), &err) : total_cost(st, x.as<double>(), &err))) return rc;
   double lambda = prm.lambda_initial;
   int it = 0;
   const bool gn = prm.solver == RPGO_SOLVER_GN;
@@ -2244,12 +2244,16 @@ int SolverRun::nonlinear_solve(hipStream_t st, bool from_x0, double* cost_out, i
     if ((rc = linearize(st))) return rc;
     if (gn) {
       int pit;
-      if ((rc = pcg(st, 0.0, &pit))) return rc;
-      k_retract<<<grid_for(N, 128, 1 << 22), 128, 0, st>>>(N, x.as<double>(), dx.as<double>(), xn.as<double>(),
-                                                           prm.pose2_chart);
-      double nerr;
-      if ((rc = total_cost(st, xn.as<double>(), &nerr))) return rc;
+      double nerr, lin;
+      bool solved = false;
+      if (direct_ready && (rc = direct_step(st, 0.0, &lin, &nerr, &solved))) return rc;
+      if (!solved) {
+        if ((rc = pcg(st, 0.0, &pit))) return rc;
+        retract(st);
+        if ((rc = total_cost(st, xn.as<double>(), &nerr))) return rc;
+      }
       ++it;
+      if (solved && last_step(err, nerr, it) && (rc = direct_finish(st, 0.0, &nerr))) return rc;
       if (polish && !(nerr < err)) break;  // refinement keeps the better iterate
       std::swap(x, xn);
       const bool conv = lm_converged(prm, err, nerr);
@@ -2257,16 +2261,20 @@ int SolverRun::nonlinear_solve(hipStream_t st, bool from_x0, double* cost_out, i
       if (conv) break;
       continue;
     }
-    bool accepted = false;
-    double nerr = err;
+    bool accepted = false, solved = false;
+    double nerr = err, lambda_step = lambda;
     while (true) {
       int pit;
-      if ((rc = pcg(st, lambda, &pit))) return rc;
       double lin;
-      if ((rc = model_decrease(st, &lin))) return rc;
-      k_retract<<<grid_for(N, 128, 1 << 22), 128, 0, st>>>(N, x.as<double>(), dx.as<double>(), xn.as<double>(),
-                                                           prm.pose2_chart);
-      if ((rc = total_cost(st, xn.as<double>(), &nerr))) return rc;
+      solved = false;
+      lambda_step = lambda;
+      if (direct_ready && (rc = direct_step(st, lambda, &lin, &nerr, &solved))) return rc;
+      if (!solved) {
+        if ((rc = pcg(st, lambda, &pit))) return rc;
+        if ((rc = model_decrease(st, &lin))) return rc;
+        retract(st);
+        if ((rc = total_cost(st, xn.as<double>(), &nerr))) return rc;
+      }
       const double fid = lin > 0.0 ? (err - nerr) / lin : -1.0;
       if (lin >= 0.0 && fid >= prm.min_model_fidelity) {
         accepted = true;
@@ -2280,6 +2288,7 @@ int SolverRun::nonlinear_solve(hipStream_t st, bool from_x0, double* cost_out, i
     ++it;
     if (!accepted) break;
     const bool conv = lm_converged(prm, err, nerr);
+    if (solved && last_step(err, nerr, it) && (rc = direct_finish(st, lambda_step, &nerr))) return rc;
     std::swap(x, xn);
     err = nerr;
     if (conv) break;
@@ -2298,10 +2307,11 @@ int SolverRun::compute_errors(hipStream_t st, const double* xp) {
   return RPGO_OK;
 }
 
-int SolverRun::run(hipStream_t st, rpgo_solve_report* rep) {
+int SolverRun::run(hipStream_t st, const rpgo_solve_problem* pr, rpgo_solve_report* rep) {
   int rc;
   stats = Stats{};
   if ((rc = build_incidence(st))) return rc;
+  if ((rc = direct_setup(st, pr->kind, pr->key_i, pr->key_j))) return rc;
   int lm_it = 0;
   double cost = 0.0;
   int gnc_it = 0;

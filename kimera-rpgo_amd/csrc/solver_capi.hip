@@ -171,7 +171,7 @@ static int solve_one(hipStream_t st, hipEvent_t ev0, hipEvent_t ev1, SolverRun& 
   RPGO_HIP_CHECK(hipStreamSynchronize(st));
   RPGO_HIP_CHECK(hipEventRecord(ev0, st));
   if (F > 0) {
-    if ((rc = S.run(st, rep))) return rc;
+    if ((rc = S.run(st, pr, rep))) return rc;
   } else {
     RPGO_HIP_CHECK(hipMemcpyAsync(S.x.ptr, S.x0.ptr, sizeof(double) * 12 * N, hipMemcpyDeviceToDevice, st));
   }

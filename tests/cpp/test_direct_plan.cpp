@@ -1,0 +1,279 @@
+// CPU check of the direct solve's elimination plan (csrc/direct_plan.h): the
+// factorization the plan describes, carried out on the host with every index
+// bounds-checked, solves random block systems of all the shapes the solver
+// takes (chains in any order, repeated and reversed factors, loop closures,
+// stars, disconnected poses, cliques), against a dense Cholesky solve.
+#include <random>
+
+#include "../../kimera-rpgo_amd/csrc/direct_plan.h"
+#include "harness.h"
+
+using namespace rpgo;
+
+namespace {
+
+struct Sys {
+  int N;
+  std::vector<int32_t> kind, fi, fj;
+  std::vector<std::vector<double>> D, H;  // 36 per pose, 36 per factor
+  std::vector<double> b;
+};
+
+Sys random_system(int N, const std::vector<std::pair<int, int>>& edges, unsigned seed) {
+  std::mt19937 rng(seed);
+  std::normal_distribution<double> g;
+  Sys s;
+  s.N = N;
+  s.D.assign(N, std::vector<double>(36, 0.0));
+  s.b.resize(6 * (size_t)N);
+  for (auto& v : s.b) v = g(rng);
+  for (int k = 0; k < N; ++k)
+    for (int i = 0; i < 6; ++i) s.D[k][i * 7] = 0.5;
+  for (auto& e : edges) {
+    s.kind.push_back(0);
+    s.fi.push_back(e.first);
+    s.fj.push_back(e.second);
+    double J[2][36];
+    for (auto& A : J)
+      for (double& v : A) v = g(rng);
+    auto prod = [&](const double* A, const double* B) {  // A^T B
+      std::vector<double> o(36, 0.0);
+      for (int i = 0; i < 6; ++i)
+        for (int j = 0; j < 6; ++j)
+          for (int m = 0; m < 6; ++m) o[i * 6 + j] += A[m * 6 + i] * B[m * 6 + j];
+      return o;
+    };
+    const auto ii = prod(J[0], J[0]), jj = prod(J[1], J[1]);
+    for (int q = 0; q < 36; ++q) {
+      s.D[e.first][q] += ii[q];
+      s.D[e.second][q] += jj[q];
+    }
+    s.H.push_back(prod(J[0], J[1]));
+    if (s.kind.size() % 7 == 3) {  // a prior now and then: no off-diagonal block
+      s.kind.push_back(1);
+      s.fi.push_back(e.first);
+      s.fj.push_back(e.first);
+      s.H.push_back(std::vector<double>(36, 1e300));
+    }
+  }
+  return s;
+}
+
+std::vector<double> dense_solve(const Sys& s) {
+  const int n = 6 * s.N;
+  std::vector<double> A((size_t)n * n, 0.0), x(s.b);
+  for (int k = 0; k < s.N; ++k)
+    for (int q = 0; q < 36; ++q) A[(size_t)(6 * k + q / 6) * n + 6 * k + q % 6] += s.D[k][q];
+  for (size_t f = 0; f < s.kind.size(); ++f)
+    if (s.kind[f] == 0)
+      for (int q = 0; q < 36; ++q) {
+        const int r = 6 * s.fi[f] + q / 6, c = 6 * s.fj[f] + q % 6;
+        A[(size_t)r * n + c] += s.H[f][q];
+        A[(size_t)c * n + r] += s.H[f][q];
+      }
+  for (int c = 0; c < n; ++c) {
+    for (int k = 0; k < c; ++k)
+      for (int r = c; r < n; ++r) A[(size_t)r * n + c] -= A[(size_t)r * n + k] * A[(size_t)c * n + k];
+    const double p = std::sqrt(A[(size_t)c * n + c]);
+    for (int r = c; r < n; ++r) A[(size_t)r * n + c] /= p;
+  }
+  for (int r = 0; r < n; ++r) {
+    for (int k = 0; k < r; ++k) x[r] -= A[(size_t)r * n + k] * x[k];
+    x[r] /= A[(size_t)r * n + r];
+  }
+  for (int r = n - 1; r >= 0; --r) {
+    for (int k = r + 1; k < n; ++k) x[r] -= A[(size_t)k * n + r] * x[k];
+    x[r] /= A[(size_t)r * n + r];
+  }
+  return x;
+}
+
+// The plan's factorization and both substitutions, front by front
+std::vector<double> plan_solve(const Sys& s, const DirectPlan& P, int& bad) {
+  std::vector<double> U(P.u_len, 0.0), G(36 * P.nb_pose.size(), 0.0), L(36 * (size_t)s.N, 0.0), y(6 * (size_t)s.N),
+      x(6 * (size_t)s.N, 0.0);
+  for (int p = 0; p < s.N; ++p) {
+    const FrontMeta& m = P.meta.at(p);
+    const int d = m.d;
+    std::vector<double> row(36 * (size_t)(d + 1), 0.0), f(6 * (size_t)(d + 1), 0.0), S((size_t)front_update_len(d), 0.0);
+    for (int q = 0; q < 36; ++q) row[q] = s.D.at(m.pose)[q];
+    for (int i = 0; i < 6; ++i) f[i] = s.b[6 * m.pose + i];
+    for (int o = 0; o < m.n_orig; ++o) {
+      const FrontOrig& a = P.origs.at(m.orig_off + o);
+      const int slot = a.slot_t >> 1;
+      if (slot < 1 || slot > d) { ++bad; continue; }
+      for (int i = 0; i < 6; ++i)
+        for (int j = 0; j < 6; ++j) row[36 * slot + i * 6 + j] += s.H.at(a.f)[(a.slot_t & 1) ? j * 6 + i : i * 6 + j];
+    }
+    for (int c = 0; c < m.n_child; ++c) {
+      const FrontChild& ch = P.childs.at(m.child_off + c);
+      for (int k = 0; k <= d; ++k) {
+        const int pk = P.maps.at(ch.map_off + k);
+        if (pk < 0) continue;
+        if (pk >= ch.d || (k == 0) != (pk == 0)) { ++bad; continue; }
+        const int64_t uc = ch.u_off + (int64_t)ch.d * (ch.d + 1) / 2 * 36 + 6 * pk;
+        for (int i = 0; i < 6; ++i) f[6 * k + i] += U.at(uc + i);
+        for (int l = 0; l <= k; ++l) {
+          const int pl = P.maps.at(ch.map_off + l);
+          if (pl < 0) continue;
+          if (pl > pk) { ++bad; continue; }
+          for (int q = 0; q < 36; ++q) {
+            const double v = U.at(ch.u_off + 36 * ((int64_t)pk * (pk + 1) / 2 + pl) + q);
+            if (l == 0) row[36 * k + q] += v;
+            else S[36 * ((int64_t)(k - 1) * k / 2 + l - 1) + q] += v;
+          }
+        }
+      }
+    }
+    double* Lp = &L[36 * (size_t)p];
+    for (int c = 0; c < 6; ++c)
+      for (int r = c; r < 6; ++r) {
+        double v = row[r * 6 + c];
+        for (int k = 0; k < c; ++k) v -= Lp[r * 6 + k] * Lp[c * 6 + k];
+        Lp[r * 6 + c] = r == c ? std::sqrt(v) : v / Lp[c * 7];
+      }
+    auto sub = [&](double* g) {  // g L^-T, a row of six
+      for (int j = 0; j < 6; ++j) {
+        for (int k = 0; k < j; ++k) g[j] -= g[k] * Lp[j * 6 + k];
+        g[j] /= Lp[j * 7];
+      }
+    };
+    sub(f.data());
+    for (int i = 0; i < 6; ++i) y[6 * p + i] = f[i];
+    double* Gp = d ? &G.at(36 * (size_t)m.nb_off) : nullptr;
+    for (int k = 1; k <= d; ++k)
+      for (int i = 0; i < 6; ++i) {
+        sub(&row[36 * k + 6 * i]);
+        for (int j = 0; j < 6; ++j) Gp[36 * (k - 1) + 6 * i + j] = row[36 * k + 6 * i + j];
+      }
+    for (int k = 0; k < d; ++k) {
+      for (int l = 0; l <= k; ++l)
+        for (int i = 0; i < 6; ++i)
+          for (int j = 0; j < 6; ++j) {
+            double v = S[36 * ((int64_t)k * (k + 1) / 2 + l) + 6 * i + j];
+            for (int q = 0; q < 6; ++q) v -= Gp[36 * k + 6 * i + q] * Gp[36 * l + 6 * j + q];
+            U.at(m.u_off + 36 * ((int64_t)k * (k + 1) / 2 + l) + 6 * i + j) = v;
+          }
+      for (int i = 0; i < 6; ++i) {
+        double v = f[6 * (k + 1) + i];
+        for (int q = 0; q < 6; ++q) v -= Gp[36 * k + 6 * i + q] * f[q];
+        U.at(m.u_off + 36 * ((int64_t)d * (d + 1) / 2) + 6 * k + i) = v;
+      }
+    }
+  }
+  for (int p = s.N - 1; p >= 0; --p) {
+    const FrontMeta& m = P.meta[p];
+    double r[6];
+    for (int j = 0; j < 6; ++j) {
+      r[j] = y[6 * p + j];
+      for (int k = 0; k < m.d; ++k)
+        for (int i = 0; i < 6; ++i) r[j] -= G[36 * (size_t)(m.nb_off + k) + 6 * i + j] * x[6 * P.nb_pose.at(m.nb_off + k) + i];
+    }
+    for (int j = 5; j >= 0; --j) {
+      for (int k = j + 1; k < 6; ++k) r[j] -= L[36 * (size_t)p + k * 6 + j] * r[k];
+      r[j] /= L[36 * (size_t)p + j * 7];
+    }
+    for (int j = 0; j < 6; ++j) x[6 * m.pose + j] = r[j];
+  }
+  return x;
+}
+
+int check(const char* what, int N, const std::vector<std::pair<int, int>>& edges, unsigned seed, int& rpgo_failures_) {
+  const Sys s = random_system(N, edges, seed);
+  DirectPlan P;
+  EXPECT(build_direct_plan(N, (int)s.kind.size(), s.kind.data(), s.fi.data(), s.fj.data(), DirectLimits(), P));
+  // every pose once, levels contiguous, no two poses of a level adjacent
+  std::vector<int> level(N, -1);
+  int seen = 0;
+  for (int l = 0; l < P.levels(); ++l)
+    for (int p = P.lvl[l]; p < P.lvl[l + 1]; ++p) {
+      EXPECT(level.at(P.meta[p].pose) < 0);
+      level[P.meta[p].pose] = l;
+      EXPECT(P.meta[p].d <= P.lvl_max_d[l]);
+      ++seen;
+    }
+  EXPECT(seen == N && P.lvl.back() == N);
+  for (auto& e : edges) EXPECT(level[e.first] != level[e.second]);
+  int bad = 0;
+  const auto x = plan_solve(s, P, bad), ref = dense_solve(s);
+  EXPECT(bad == 0);
+  double err = 0.0, nrm = 0.0;
+  for (size_t k = 0; k < x.size(); ++k) {
+    err = std::max(err, std::fabs(x[k] - ref[k]));
+    nrm = std::max(nrm, std::fabs(ref[k]));
+  }
+  std::printf("  %s N=%d levels=%d max_d=%d err %.1e of %.1e\n", what, N, P.levels(), P.max_d, err, nrm);
+  // condition numbers here stay below about 1e5: 1e5 * 6 N * 2^-53 < 1e-7
+  EXPECT(err <= 1e-7 * (nrm + 1.0));
+  return P.levels();
+}
+
+std::vector<std::pair<int, int>> chain(int N) {
+  std::vector<std::pair<int, int>> e;
+  for (int k = 0; k + 1 < N; ++k) e.push_back({k, k + 1});
+  return e;
+}
+
+}  // namespace
+
+TEST(DirectPlan, Chains) {
+  for (int N : {1, 2, 3, 4, 7, 8, 63, 64, 65, 200}) check("chain", N, chain(N), 10 + N, rpgo_failures_);
+  // odd-even reduction: logarithmic in the length
+  EXPECT(check("chain", 256, chain(256), 3, rpgo_failures_) <= 12);
+}
+
+TEST(DirectPlan, OrdersAndRepeats) {
+  std::mt19937 rng(1);
+  for (int t = 0; t < 12; ++t) {
+    const int N = 2 + (int)(rng() % 70);
+    std::vector<int> name(N);
+    for (int k = 0; k < N; ++k) name[k] = k;
+    std::shuffle(name.begin(), name.end(), rng);
+    std::vector<std::pair<int, int>> e;
+    for (auto& c : chain(N)) {
+      const int a = name[c.first], b = name[c.second];
+      if (rng() % 2) e.push_back({a, b});
+      else e.push_back({b, a});
+      if (rng() % 3 == 0) e.push_back({b, a});  // repeated, other direction
+    }
+    for (int q = 0; q < N / 4; ++q) {
+      const int a = (int)(rng() % N), b = (int)(rng() % N);
+      if (a != b) e.push_back({a, b});
+    }
+    check("shuffled", N, e, 50 + t, rpgo_failures_);
+  }
+}
+
+TEST(DirectPlan, Shapes) {
+  std::vector<std::pair<int, int>> star, clique, two, none;
+  for (int k = 1; k < 60; ++k) star.push_back(k % 2 ? std::make_pair(0, k) : std::make_pair(k, 0));
+  for (int a = 0; a < 20; ++a)
+    for (int b = a + 1; b < 20; ++b) clique.push_back({b, a});
+  for (int k = 0; k < 40; ++k)
+    if (k != 20) two.push_back({k, k + 1});  // two chains, one of them with a loop
+  two.push_back({5, 17});
+  check("star", 60, star, 1, rpgo_failures_);
+  check("clique", 20, clique, 2, rpgo_failures_);
+  check("two chains", 41, two, 3, rpgo_failures_);
+  check("no factors", 5, none, 4, rpgo_failures_);
+  auto ladder = chain(120);  // laps of 12 poses, joined at every third pose
+  for (int k = 0; k + 12 < 120; k += 3) ladder.push_back({k + 12, k});
+  check("laps", 120, ladder, 5, rpgo_failures_);
+}
+
+TEST(DirectPlan, Limits) {
+  std::vector<std::pair<int, int>> clique;
+  for (int a = 0; a < 20; ++a)
+    for (int b = a + 1; b < 20; ++b) clique.push_back({b, a});
+  const Sys s = random_system(20, clique, 2);
+  DirectPlan P;
+  DirectLimits lim;
+  lim.max_d = 18;
+  EXPECT(!build_direct_plan(20, (int)s.kind.size(), s.kind.data(), s.fi.data(), s.fj.data(), lim, P));
+  lim.max_d = 19;
+  EXPECT(build_direct_plan(20, (int)s.kind.size(), s.kind.data(), s.fi.data(), s.fj.data(), lim, P));
+  lim.max_u = P.u_len - 1;
+  EXPECT(!build_direct_plan(20, (int)s.kind.size(), s.kind.data(), s.fi.data(), s.fj.data(), lim, P));
+}
+
+RPGO_TEST_MAIN

@@ -48,3 +48,10 @@ def test_dataset_binary_cpu():
     env = dict(os.environ, RPGO_DATASET_PATH=os.path.join(ROOT, "tests", "golden", "data"))
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60, env=env)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_direct_plan_binary_cpu():
+    """The direct solve's elimination plan against dense solves, on the host."""
+    exe = os.path.join(ROOT, "tests", "cpp", "bin", "test_direct_plan")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout + r.stderr

@@ -5,7 +5,7 @@
 // replay64.hip (the FP64 replay of Pcm.h's fold, odometry check and pairwise
 // check, bit-exact with the oracle) with a graph lookup in front:
 //   measurements   one thread per odometry row / loop closure (all graphs)
-//   fold           one wavefront per graph
+//   fold           one workgroup per graph
 //   odometry check one thread per loop closure
 //   compaction     one workgroup per graph (stable, input order)
 //   pairs          one wavefront per (row, 64-column word) tile; the tiles of
@@ -96,27 +96,25 @@ __device__ __forceinline__ int graph_of(const long long* __restrict__ off, int n
 }
 
 template <int DIM>
-__global__ void __launch_bounds__(64) k_fold_batch(int n_graphs, const long long* __restrict__ pose_off,
-                                                  const double* __restrict__ pose0, const double* __restrict__ delta,
-                                                  const double* __restrict__ hinv, double* __restrict__ traj) {
+__global__ void __launch_bounds__(kFoldThreads) k_fold_batch(int n_graphs, const long long* __restrict__ pose_off,
+                                                             const double* __restrict__ pose0,
+                                                             const double* __restrict__ delta,
+                                                             const double* __restrict__ hinv,
+                                                             double* __restrict__ traj) {
   constexpr int PL = R64<DIM>::PL, D = R64<DIM>::D, PWC = R64<DIM>::PWC, DD = D * D;
-  __shared__ double S[DD], T[DD], P[PL], Hs[DD], Dl[PWC], ob[kFoldAhead * PWC];
-  __shared__ int ri;
+  __shared__ FoldLds<DIM> L;
   const int g = blockIdx.x;
   if (g >= n_graphs) return;
   const long long p0 = pose_off[g];
   const int n_poses = (int)(pose_off[g + 1] - p0);
   const long long o0 = p0 - g;  // odometry rows of graph g
   double* tr = traj + (size_t)p0 * PWC;
-  const int l = threadIdx.x;
-  if (l < DD) S[l] = 0.0;
-  if (l < PL) P[l] = pose0[(size_t)g * PL + l];
-  if (l == 0) ri = 1;
-  __syncthreads();
-  for (int e = l; e < PWC; e += 64) tr[e] = e < PL ? P[e] : (e < PL + DD ? 0.0 : 1.0);
+  const int tid = threadIdx.x;
+  const double* p = pose0 + (size_t)g * PL;
+  fold_start<DIM>(L, p, nullptr, tid);
+  if (tid < PWC) tr[tid] = tid < PL ? p[tid] : (tid < PL + DD ? 0.0 : 1.0);
   if (n_poses > 1)
-    fold_run<DIM>(n_poses - 1, hinv + (size_t)o0 * DD, delta + (size_t)o0 * PWC, tr + PWC, S, T, P, Hs, Dl, &ri,
-                  ob, l);
+    fold_run<DIM>(n_poses - 1, hinv + (size_t)o0 * DD, delta + (size_t)o0 * PWC, tr + PWC, L, tid);
 }
 
 template <int DIM>
@@ -492,12 +490,12 @@ static int launch_stages(rpgo_ctx* ctx, BatchState& s, const rpgo_pcm_params* pr
       k_meas_batch<2><<<(unsigned)((nlc + 255) / 256), 256, 0, st>>>((long long)nlc, s.lc_pose.as<double>(), s.lc_cov.as<double>(),
                                                                      s.lcm.as<double>(), nullptr);
   }
-  // fold: one wavefront per graph
+  // fold: one workgroup per graph
   if (dim == 3)
-    k_fold_batch<3><<<G, 64, 0, st>>>(G, s.d_pose_off.as<long long>(), s.pose0.as<double>(), s.delta.as<double>(),
+    k_fold_batch<3><<<G, kFoldThreads, 0, st>>>(G, s.d_pose_off.as<long long>(), s.pose0.as<double>(), s.delta.as<double>(),
                                       s.hinv.as<double>(), s.traj.as<double>());
   else
-    k_fold_batch<2><<<G, 64, 0, st>>>(G, s.d_pose_off.as<long long>(), s.pose0.as<double>(), s.delta.as<double>(),
+    k_fold_batch<2><<<G, kFoldThreads, 0, st>>>(G, s.d_pose_off.as<long long>(), s.pose0.as<double>(), s.delta.as<double>(),
                                       s.hinv.as<double>(), s.traj.as<double>());
   RPGO_HIP_CHECK(hipGetLastError());
   if (events) RPGO_HIP_CHECK(hipEventRecord(ev[1], st));

@@ -358,26 +358,35 @@ struct R64<2> {
 #undef RPGO_R64_COMMON
 };
 
-// Sequential odometry fold of one chain by one wavefront (Pcm.h:516-557):
-// for step j < n_steps, T_{j+1} = T_j * delta_j and
+// Sequential odometry fold of one chain by one workgroup of four wavefronts
+// (Pcm.h:516-557): for step j < n_steps, T_{j+1} = T_j * delta_j and
 // Sigma_{j+1} = (H_j Sigma_j) H_j^T + Sigma_delta_j, in the oracle's order.
-// Lanes 0..D*D-1 own the covariance entries, the next lanes the pose entries;
-// S, P and ri hold the state on entry (step 0's start) and on exit.  hk, dk:
-// H_j and the delta record of step 0 (rows of D*D and PWC doubles); out:
-// the trajectory record written by step 0 (then one per step); ob: LDS for
-// kFoldAhead records.
-// The steps form one dependent chain, so the time per step is the latency of
-// its LDS round trips; no global memory access may wait inside it.  Steps go
-// in blocks of kFoldAhead: the next block's inputs are loaded into registers
-// while this block runs, the block's records collect in LDS and are stored
-// after it, and the only wait for global memory is at the block boundary.
-// The workgroup is this one wavefront, and LDS operations of a wavefront are
-// performed in issue order, so the steps order their LDS traffic with
-// wavefront-scope fences (no instruction; they keep the compiler from moving
-// memory operations across them).  A __syncthreads() per step is a
-// workgroup-scope fence that waits for every global load and store in
-// flight.  Callers compiled with -ffp-contract=off, launched with 64 threads.
-constexpr int kFoldAhead = 8;
+// L holds the state on entry (fold_start) and on exit; hk, dk: H_j and the
+// delta record of step 0 (rows of D*D and PWC doubles); out: the trajectory
+// record written by step 0 (then one per step).
+//
+// The steps are one dependent chain, so the time is steps times the latency of
+// a covariance step, and everything else is kept off that path:
+//   wavefront 0   the covariance, lane r D + c owning entry (r, c): row r of H
+//                 against column c of Sigma, then row r of that against row c
+//                 of H.  Two LDS exchanges a step; H's rows and Sigma_delta are
+//                 read a step ahead.  Sigma lies transposed in LDS, so each
+//                 operand is D contiguous values.
+//   wavefront 1   the pose (a lane per row: a row of T delta needs only that
+//                 row of T, so no exchange) and the rotation flag.  The pose
+//                 does not depend on the covariance.
+//   wavefronts 2-3  the next kFoldAhead steps' inputs into LDS and the last
+//                 ones' records out, once per block of steps.
+// 175 ns a step on SE(3): 50,000 poses in 8.7 ms, of which about 45 ns are the
+// 13 dependent FP64 operations and the rest the two exchanges.  One wavefront
+// doing all of it took 535 ns a step (26.7 ms): the pose and flag lanes ran
+// after the covariance lanes, and H went through LDS inside the step.
+// LDS operations of a wavefront are performed in issue order, so its steps
+// order their LDS traffic with wavefront-scope fences (no instruction; they
+// keep the compiler from moving memory operations across them).  Callers
+// compiled with -ffp-contract=off, launched with kFoldThreads threads.
+constexpr int kFoldAhead = 24;
+constexpr int kFoldThreads = 256;
 
 __device__ __forceinline__ void fold_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -385,75 +394,210 @@ __device__ __forceinline__ void fold_wave_sync() {
 }
 
 template <int DIM>
+struct FoldLds {
+  static constexpr int PL = R64<DIM>::PL, D = R64<DIM>::D, PWC = R64<DIM>::PWC, DD = D * D, A = kFoldAhead;
+  alignas(16) double H[2][A * DD];   // per step: H_j
+  alignas(16) double P[2][A * PL];   // pose of delta_j
+  alignas(16) double C[2][A * DD];   // Sigma_delta_j
+  double F[2][A];                    // rotation flag of delta_j
+  alignas(16) double o[2][A * PWC];  // the block's records
+  alignas(16) double St[DD], T[DD];  // Sigma transposed, H Sigma
+  double pose[PL];
+  int ri;
+};
+
+// State at the start of a chain (pose given, zero covariance, Pcm.h:534-542)
+// or, with rec, at a stored record; every thread calls it
+template <int DIM>
+__device__ __forceinline__ void fold_start(FoldLds<DIM>& L, const double* __restrict__ pose0,
+                                           const double* __restrict__ rec, int tid) {
+  constexpr int PL = FoldLds<DIM>::PL, D = FoldLds<DIM>::D, DD = FoldLds<DIM>::DD;
+  if (tid < DD) L.St[(tid % D) * D + tid / D] = rec ? rec[PL + tid] : 0.0;
+  if (tid < PL) L.pose[tid] = rec ? rec[tid] : pose0[tid];
+  if (tid == 0) L.ri = rec ? (rec[PL + DD] != 0.0 ? 1 : 0) : 1;
+  __syncthreads();
+}
+
+// covariance steps of one block, lanes l < D*D of wavefront 0
+template <int DIM>
+__device__ __forceinline__ void fold_cov_block(FoldLds<DIM>& L, int b, int nb, int l) {
+  constexpr int PL = FoldLds<DIM>::PL, D = FoldLds<DIM>::D, PWC = FoldLds<DIM>::PWC, DD = D * D;
+  const int r = l / D, c = l - r * D;
+  double hr[D], hc[D], sd;
+#pragma unroll
+  for (int m = 0; m < D; ++m) {
+    hr[m] = L.H[b][r * D + m];
+    hc[m] = L.H[b][c * D + m];
+  }
+  sd = L.C[b][l];
+  for (int u = 0; u < nb; ++u) {
+    double v[D], t[D];
+#pragma unroll
+    for (int m = 0; m < D; ++m) v[m] = L.St[c * D + m];
+    // the next step's operands, in flight behind this step's exchanges
+    const int un = u + 1 < nb ? u + 1 : u;
+    double hrn[D], hcn[D];
+#pragma unroll
+    for (int m = 0; m < D; ++m) {
+      hrn[m] = L.H[b][un * DD + r * D + m];
+      hcn[m] = L.H[b][un * DD + c * D + m];
+    }
+    const double sdn = L.C[b][un * DD + l];
+    double s = hr[0] * v[0];
+#pragma unroll
+    for (int m = 1; m < D; ++m) s += hr[m] * v[m];
+    L.T[l] = s;
+    fold_wave_sync();
+#pragma unroll
+    for (int m = 0; m < D; ++m) t[m] = L.T[r * D + m];
+    s = t[0] * hc[0];
+#pragma unroll
+    for (int m = 1; m < D; ++m) s += t[m] * hc[m];
+    s = s + sd;
+    L.St[c * D + r] = s;
+    fold_wave_sync();
+    L.o[b][u * PWC + PL + l] = s;
+#pragma unroll
+    for (int m = 0; m < D; ++m) {
+      hr[m] = hrn[m];
+      hc[m] = hcn[m];
+    }
+    sd = sdn;
+  }
+}
+
+// pose steps of one block: SE(3) lane r < 3 owns row r, SE(2) lane 0 the pose
+__device__ __forceinline__ void fold_pose_block(FoldLds<3>& L, int b, int nb, int r) {
+  constexpr int PL = 12, PWC = FoldLds<3>::PWC;
+  double a0 = L.pose[r * 3], a1 = L.pose[r * 3 + 1], a2 = L.pose[r * 3 + 2], t = L.pose[9 + r];
+  double q[PL];
+#pragma unroll
+  for (int e = 0; e < PL; ++e) q[e] = L.P[b][e];
+  for (int u = 0; u < nb; ++u) {
+    const int un = u + 1 < nb ? u + 1 : u;
+    double qn[PL];
+#pragma unroll
+    for (int e = 0; e < PL; ++e) qn[e] = L.P[b][un * PL + e];
+    // R64<3>::compose_entry's order
+    double n[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      double s = a0 * q[c];
+      s += a1 * q[3 + c];
+      s += a2 * q[6 + c];
+      n[c] = s;
+    }
+    double s = a0 * q[9];
+    s += a1 * q[10];
+    s += a2 * q[11];
+    t = t + s;
+    a0 = n[0];
+    a1 = n[1];
+    a2 = n[2];
+    double* o = L.o[b] + u * PWC;
+    o[r * 3] = a0;
+    o[r * 3 + 1] = a1;
+    o[r * 3 + 2] = a2;
+    o[9 + r] = t;
+#pragma unroll
+    for (int e = 0; e < PL; ++e) q[e] = qn[e];
+  }
+  L.pose[r * 3] = a0;
+  L.pose[r * 3 + 1] = a1;
+  L.pose[r * 3 + 2] = a2;
+  L.pose[9 + r] = t;
+}
+
+__device__ __forceinline__ void fold_pose_block(FoldLds<2>& L, int b, int nb, int) {
+  constexpr int PL = 4, PWC = FoldLds<2>::PWC;
+  double P[PL];
+#pragma unroll
+  for (int e = 0; e < PL; ++e) P[e] = L.pose[e];
+  for (int u = 0; u < nb; ++u) {
+    double q[PL], n[PL];
+#pragma unroll
+    for (int e = 0; e < PL; ++e) q[e] = L.P[b][u * PL + e];
+    R64<2>::pose_compose(P, q, n);
+#pragma unroll
+    for (int e = 0; e < PL; ++e) {
+      P[e] = n[e];
+      L.o[b][u * PWC + e] = n[e];
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < PL; ++e) L.pose[e] = P[e];
+}
+
+template <int DIM>
 __device__ __forceinline__ void fold_run(int n_steps, const double* __restrict__ hk,
                                          const double* __restrict__ dk, double* __restrict__ out,
-                                         double* S, double* T, double* P, double* Hs, double* Dl, int* ri,
-                                         double* ob, int l) {
-  constexpr int PL = R64<DIM>::PL, D = R64<DIM>::D, PWC = R64<DIM>::PWC, DD = D * D;
-  static_assert(PWC <= 64 && DD <= 64, "one entry per lane");
-  constexpr int A = kFoldAhead;
-  const int lh = l < DD ? l : DD - 1, ld = l < PWC ? l : PWC - 1;  // in-row addresses for every lane
-  double hx[A], dx[A], hy[A], dy[A];
+                                         FoldLds<DIM>& L, int tid) {
+  constexpr int PL = FoldLds<DIM>::PL, D = FoldLds<DIM>::D, PWC = FoldLds<DIM>::PWC, DD = D * D, A = kFoldAhead;
+  constexpr int NT = 128;                              // threads of wavefronts 2-3
+  constexpr int NH = (A * DD + NT - 1) / NT, NR = (A * PWC + NT - 1) / NT;
+  const int wv = tid >> 6, l = tid & 63, ht = tid - 128;
+  const long long nh = (long long)n_steps * DD, nr = (long long)n_steps * PWC;
+  // inputs of the block of steps from j0, through registers: every load of a
+  // block is in flight at once
+  double xh[NH], xr[NR];
+  auto fetch = [&](int j0) {
 #pragma unroll
-  for (int u = 0; u < A; ++u) {
-    const int j = u < n_steps ? u : 0;
-    hx[u] = hk[(size_t)j * DD + lh];
-    dx[u] = dk[(size_t)j * PWC + ld];
+    for (int k = 0; k < NH; ++k) {
+      const long long e = (long long)j0 * DD + ht + NT * k;
+      xh[k] = hk[e < nh ? e : 0];
+    }
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      const long long e = (long long)j0 * PWC + ht + NT * k;
+      xr[k] = dk[e < nr ? e : 0];
+    }
+  };
+  auto place = [&](int b) {
+#pragma unroll
+    for (int k = 0; k < NH; ++k) {
+      const int e = ht + NT * k;
+      if (e < A * DD) L.H[b][e] = xh[k];
+    }
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      const int e = ht + NT * k;
+      if (e >= A * PWC) continue;
+      const int u = e / PWC, q = e - u * PWC;
+      if (q < PL) L.P[b][u * PL + q] = xr[k];
+      else if (q < PL + DD) L.C[b][u * DD + q - PL] = xr[k];
+      else L.F[b][u] = xr[k];
+    }
+  };
+  if (wv >= 2) {
+    fetch(0);
+    place(0);
   }
-  for (int j0 = 0; j0 < n_steps; j0 += A) {
-    // the next block's inputs: independent of the chain, in flight meanwhile
-#pragma unroll
-    for (int u = 0; u < A; ++u) {
-      const int j = j0 + A + u < n_steps ? j0 + A + u : 0;
-      hy[u] = hk[(size_t)j * DD + lh];
-      dy[u] = dk[(size_t)j * PWC + ld];
+  __syncthreads();
+  const int n_blocks = (n_steps + A - 1) / A;
+  for (int k = 0; k < n_blocks; ++k) {
+    const int b = k & 1, j0 = k * A, nb = n_steps - j0 < A ? n_steps - j0 : A;
+    if (wv == 0) {
+      if (l < DD) fold_cov_block<DIM>(L, b, nb, l);
+    } else if (wv == 1) {
+      if (l < (DIM == 3 ? 3 : 1)) fold_pose_block(L, b, nb, l);
+      if (l == 63) {
+        int ri = L.ri;
+        for (int u = 0; u < nb; ++u) {
+          ri = (ri && L.F[b][u] != 0.0) ? 1 : 0;
+          L.o[b][u * PWC + PL + DD] = ri ? 1.0 : 0.0;
+        }
+        L.ri = ri;
+      }
+    } else {
+      if (k + 1 < n_blocks) fetch(j0 + A);
+      if (k > 0)  // the block before this one is whole
+        for (int e = ht; e < A * PWC; e += NT) out[(size_t)(j0 - A) * PWC + e] = L.o[b ^ 1][e];
+      if (k + 1 < n_blocks) place(b ^ 1);
     }
-    const int nb = n_steps - j0 < A ? n_steps - j0 : A;
-#pragma unroll
-    for (int u = 0; u < A; ++u) {
-      if (u >= nb) break;
-      if (l < DD) Hs[l] = hx[u];
-      if (l < PWC) Dl[l] = dx[u];
-      fold_wave_sync();
-      // T = H * Sigma
-      if (l < DD) {
-        const int r = l / D, c = l % D;
-        double s = Hs[r * D] * S[c];
-#pragma unroll
-        for (int m = 1; m < D; ++m) s += Hs[r * D + m] * S[m * D + c];
-        T[l] = s;
-      }
-      double newpose = 0.0;
-      if (l >= DD && l < DD + PL) newpose = R64<DIM>::compose_entry(P, Dl, l - DD);
-      fold_wave_sync();
-      double* o = ob + u * PWC;
-      if (l < DD) {
-        const int r = l / D, c = l % D;
-        double s = T[r * D] * Hs[c * D];
-#pragma unroll
-        for (int m = 1; m < D; ++m) s += T[r * D + m] * Hs[c * D + m];
-        s = s + Dl[PL + l];
-        S[l] = s;
-        o[PL + l] = s;
-      }
-      if (l >= DD && l < DD + PL) {
-        P[l - DD] = newpose;
-        o[l - DD] = newpose;
-      }
-      if (l == 0) {
-        *ri = (*ri && Dl[PL + DD] != 0.0) ? 1 : 0;
-        o[PL + DD] = *ri ? 1.0 : 0.0;
-      }
-      fold_wave_sync();
-    }
-    // the block's records, stored contiguously
-    for (int e = l; e < nb * PWC; e += 64) out[(size_t)j0 * PWC + e] = ob[e];
-#pragma unroll
-    for (int u = 0; u < A; ++u) {
-      hx[u] = hy[u];
-      dx[u] = dy[u];
-    }
+    __syncthreads();
   }
+  const int kl = n_blocks - 1, j0 = kl * A;
+  for (int e = tid; e < (n_steps - j0) * PWC; e += kFoldThreads) out[(size_t)j0 * PWC + e] = L.o[kl & 1][e];
 }
 
 }  // namespace rpgo

@@ -58,66 +58,45 @@ __global__ void k_measurements(int n, const double* __restrict__ pose,
 }
 
 // ---------------------------------------------------------------------------
-// sequential fold, one wavefront:  T_{k+1} = T_k * delta_k,
+// sequential fold, one workgroup:  T_{k+1} = T_k * delta_k,
 // Sigma_{k+1} = (H_k Sigma_k) H_k^T + Sigma_delta_k   (same order as the oracle)
-// lanes 0..D*D-1 own the covariance entries, the next lanes the pose entries.
 // Records start+1 .. n_poses-1 are written; the state at `start` comes from
 // pose0 (chain start, record `start` written too) or from the stored record.
 // ---------------------------------------------------------------------------
 template <int DIM>
-__global__ void __launch_bounds__(64) k_fold(int start, int n_poses,
-                                            const double* __restrict__ pose0,
-                                            const double* __restrict__ delta,
-                                            const double* __restrict__ hinv,
-                                            double* __restrict__ traj) {
+__global__ void __launch_bounds__(kFoldThreads) k_fold(int start, int n_poses, const double* __restrict__ pose0,
+                                                       const double* __restrict__ delta,
+                                                       const double* __restrict__ hinv, double* __restrict__ traj) {
   constexpr int PL = R64<DIM>::PL, D = R64<DIM>::D, PWC = R64<DIM>::PWC, DD = D * D;
-  __shared__ double S[DD], T[DD], P[PL], Hs[DD], Dl[PWC], ob[kFoldAhead * PWC];
-  __shared__ int ri;
-  const int l = threadIdx.x;
-  if (pose0) {
-    // chain start: pose from the values, zero covariance (Pcm.h:534-542)
-    if (l < DD) S[l] = 0.0;
-    if (l < PL) P[l] = pose0[l];
-    if (l == 0) ri = 1;
-    for (int e = l; e < PWC; e += 64)
-      traj[(size_t)start * PWC + e] = e < PL ? pose0[e] : (e < PL + DD ? 0.0 : 1.0);
-  } else {
-    // continue from a stored record: the same values the fold held there
-    const double* rec = traj + (size_t)start * PWC;
-    if (l < DD) S[l] = rec[PL + l];
-    if (l < PL) P[l] = rec[l];
-    if (l == 0) ri = rec[PL + DD] != 0.0 ? 1 : 0;
-  }
-  __syncthreads();
+  __shared__ FoldLds<DIM> L;
+  const int tid = threadIdx.x;
+  double* rec = traj + (size_t)start * PWC;
+  fold_start<DIM>(L, pose0, pose0 ? nullptr : rec, tid);
+  if (pose0 && tid < PWC) rec[tid] = tid < PL ? pose0[tid] : (tid < PL + DD ? 0.0 : 1.0);
   if (start + 1 < n_poses)
-    fold_run<DIM>(n_poses - 1 - start, hinv + (size_t)start * DD, delta + (size_t)start * PWC,
-                  traj + (size_t)(start + 1) * PWC, S, T, P, Hs, Dl, &ri, ob, l);
+    fold_run<DIM>(n_poses - 1 - start, hinv + (size_t)start * DD, delta + (size_t)start * PWC, rec + PWC, L, tid);
 }
 
-// Fold of several chains, one wavefront per chain (Pcm.h:516-557 per robot
+// Fold of several chains, one workgroup per chain (Pcm.h:516-557 per robot
 // prefix): chain c starts at pose0s[c] with zero covariance; its odometry rows
 // are [off[c] - c, off[c+1] - c - 1).  Same arithmetic as k_fold.
 template <int DIM>
-__global__ void __launch_bounds__(64) k_fold_chains(Chains ch, const double* __restrict__ pose0s,
-                                                   const double* __restrict__ delta,
-                                                   const double* __restrict__ hinv,
-                                                   double* __restrict__ traj) {
+__global__ void __launch_bounds__(kFoldThreads) k_fold_chains(Chains ch, const double* __restrict__ pose0s,
+                                                              const double* __restrict__ delta,
+                                                              const double* __restrict__ hinv,
+                                                              double* __restrict__ traj) {
   constexpr int PL = R64<DIM>::PL, D = R64<DIM>::D, PWC = R64<DIM>::PWC, DD = D * D;
-  __shared__ double S[DD], T[DD], P[PL], Hs[DD], Dl[PWC], ob[kFoldAhead * PWC];
-  __shared__ int ri;
+  __shared__ FoldLds<DIM> L;
   const int c = blockIdx.x;
   if (c >= ch.n) return;
   const int p0 = ch.off[c], n_poses = ch.off[c + 1] - p0, o0 = p0 - c;
   double* tr = traj + (size_t)p0 * PWC;
-  const int l = threadIdx.x;
-  if (l < DD) S[l] = 0.0;
-  if (l < PL) P[l] = pose0s[(size_t)c * PL + l];
-  if (l == 0) ri = 1;
-  __syncthreads();
-  for (int e = l; e < PWC; e += 64) tr[e] = e < PL ? P[e] : (e < PL + DD ? 0.0 : 1.0);
+  const int tid = threadIdx.x;
+  const double* p = pose0s + (size_t)c * PL;
+  fold_start<DIM>(L, p, nullptr, tid);
+  if (tid < PWC) tr[tid] = tid < PL ? p[tid] : (tid < PL + DD ? 0.0 : 1.0);
   if (n_poses > 1)
-    fold_run<DIM>(n_poses - 1, hinv + (size_t)o0 * DD, delta + (size_t)o0 * PWC, tr + PWC, S, T, P, Hs, Dl, &ri,
-                  ob, l);
+    fold_run<DIM>(n_poses - 1, hinv + (size_t)o0 * DD, delta + (size_t)o0 * PWC, tr + PWC, L, tid);
 }
 
 // ---------------------------------------------------------------------------
@@ -808,19 +787,19 @@ int pcm_fold(rpgo_ctx* ctx) {
   if ((rc = s.traj.reserve(sizeof(double) * (size_t)s.n_poses * pwc_len(s.dim)))) return rc;
   if (s.n_chains > 1) {
     if (s.dim == 3)
-      k_fold_chains<3><<<s.n_chains, 64, 0, ctx->stream>>>(chains_of(s), s.pose0.as<double>(), s.delta.as<double>(),
+      k_fold_chains<3><<<s.n_chains, kFoldThreads, 0, ctx->stream>>>(chains_of(s), s.pose0.as<double>(), s.delta.as<double>(),
                                                            s.hinv.as<double>(), s.traj.as<double>());
     else
-      k_fold_chains<2><<<s.n_chains, 64, 0, ctx->stream>>>(chains_of(s), s.pose0.as<double>(), s.delta.as<double>(),
+      k_fold_chains<2><<<s.n_chains, kFoldThreads, 0, ctx->stream>>>(chains_of(s), s.pose0.as<double>(), s.delta.as<double>(),
                                                            s.hinv.as<double>(), s.traj.as<double>());
     RPGO_HIP_CHECK(hipGetLastError());
     return RPGO_OK;
   }
   if (s.dim == 3)
-    k_fold<3><<<1, 64, 0, ctx->stream>>>(0, s.n_poses, s.pose0.as<double>(), s.delta.as<double>(),
+    k_fold<3><<<1, kFoldThreads, 0, ctx->stream>>>(0, s.n_poses, s.pose0.as<double>(), s.delta.as<double>(),
                                          s.hinv.as<double>(), s.traj.as<double>());
   else
-    k_fold<2><<<1, 64, 0, ctx->stream>>>(0, s.n_poses, s.pose0.as<double>(), s.delta.as<double>(),
+    k_fold<2><<<1, kFoldThreads, 0, ctx->stream>>>(0, s.n_poses, s.pose0.as<double>(), s.delta.as<double>(),
                                          s.hinv.as<double>(), s.traj.as<double>());
   RPGO_HIP_CHECK(hipGetLastError());
   return RPGO_OK;
@@ -830,10 +809,10 @@ int pcm_fold_from(rpgo_ctx* ctx, int start) {
   PcmState& s = ctx->pcm;
   if (start + 1 >= s.n_poses) return RPGO_OK;
   if (s.dim == 3)
-    k_fold<3><<<1, 64, 0, ctx->stream>>>(start, s.n_poses, nullptr, s.delta.as<double>(),
+    k_fold<3><<<1, kFoldThreads, 0, ctx->stream>>>(start, s.n_poses, nullptr, s.delta.as<double>(),
                                          s.hinv.as<double>(), s.traj.as<double>());
   else
-    k_fold<2><<<1, 64, 0, ctx->stream>>>(start, s.n_poses, nullptr, s.delta.as<double>(),
+    k_fold<2><<<1, kFoldThreads, 0, ctx->stream>>>(start, s.n_poses, nullptr, s.delta.as<double>(),
                                          s.hinv.as<double>(), s.traj.as<double>());
   RPGO_HIP_CHECK(hipGetLastError());
   return RPGO_OK;

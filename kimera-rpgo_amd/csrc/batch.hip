@@ -44,7 +44,7 @@ struct BatchState {
   DevBuf pose0, odom, odom_cov, lc_from, lc_to, lc_pose, lc_cov;
   DevBuf delta, hinv, traj, lcm, odom_dist, flags, accepted, m, c_from, c_to, c_lcm, adj, counters;
   DevBuf deg, cidx, ck;  // clique stage: degrees, members, sizes
-  DevBuf cb_state, cb_icc, cb_dm;  // clique stage: chip-wide rounds
+  DevBuf cb_state, cb_icc, cb_dm, cb_diag, cb_grp;  // clique stage: chip-wide rounds
   // clique rounds' graph placement: graphs grouped by XCD (G entries), then
   // the 9 group offsets; cb_xmax = graphs of the largest group
   DevBuf cb_xorder;
@@ -320,7 +320,7 @@ void batch_destroy(rpgo_ctx* ctx) {
   for (DevBuf* b : {&s.d_pose_off, &s.d_lc_off, &s.d_adj_off, &s.d_tile_off, &s.d_sym_off, &s.d_lc_graph, &s.pose0,
                     &s.odom, &s.odom_cov, &s.lc_from, &s.lc_to, &s.lc_pose, &s.lc_cov, &s.delta, &s.hinv, &s.traj,
                     &s.lcm, &s.odom_dist, &s.flags, &s.accepted, &s.m, &s.c_from, &s.c_to, &s.c_lcm, &s.adj,
-                    &s.counters, &s.deg, &s.cidx, &s.ck, &s.cb_state, &s.cb_icc, &s.cb_dm, &s.cb_xorder, &s.d_blk_off,
+                    &s.counters, &s.deg, &s.cidx, &s.ck, &s.cb_state, &s.cb_icc, &s.cb_dm, &s.cb_diag, &s.cb_grp, &s.cb_xorder, &s.d_blk_off,
                     &s.d_sq_off, &s.d_pblk_off, &s.fp_prec, &s.fp_lcr, &s.fp_pl64, &s.fp_pb64, &s.fp_bend, &s.fp_ta,
                     &s.fp_sanc, &s.fp_terms, &s.fp_queue})
     b->release();
@@ -462,6 +462,8 @@ static CliqueSpread spread_of(BatchState& s) {
   sp.state = s.cb_state.ptr;
   sp.icc = s.cb_icc.as<int>();
   sp.dm = s.cb_dm.as<unsigned long long>();
+  sp.diag = s.cb_diag.as<unsigned long long>();
+  sp.grp = s.cb_grp.as<unsigned long long>();
   sp.xorder = s.cb_xorder.as<int>();
   sp.xmax = s.cb_xmax;
   return sp;
@@ -742,7 +744,8 @@ int rpgo_pcm_batch_run(rpgo_ctx* ctx, const rpgo_pcm_batch* B, const rpgo_pcm_pa
     if ((rc = s.deg.reserve(sizeof(int) * nl1)) || (rc = s.cidx.reserve(sizeof(int) * nl1)) ||
         (rc = s.ck.reserve(sizeof(int) * (size_t)G)) || (rc = s.cb_state.reserve(clique_spread_state_bytes(G))) ||
         (rc = s.cb_icc.reserve(clique_spread_icc_bytes(G))) ||
-        (rc = s.cb_dm.reserve(sizeof(unsigned long long) * nl1)))
+        (rc = s.cb_dm.reserve(sizeof(unsigned long long) * nl1)) ||
+        (rc = s.cb_diag.reserve(sizeof(unsigned long long) * nl1)) || (rc = s.cb_grp.reserve(s.adj.bytes)))
       return rc;
     // The rounds walk each graph's adjacency rows many times over.  Each graph
     // goes to one XCD, so its rows stay in that XCD's L2, and the graphs are
@@ -806,7 +809,7 @@ int rpgo_pcm_batch_run(rpgo_ctx* ctx, const rpgo_pcm_batch* B, const rpgo_pcm_pa
     for (DevBuf* b : {&s.d_pose_off, &s.d_lc_off, &s.d_adj_off, &s.d_tile_off, &s.d_sym_off, &s.d_lc_graph,
                       &s.pose0, &s.odom, &s.odom_cov, &s.lc_from, &s.lc_to, &s.lc_pose, &s.lc_cov, &s.delta,
                       &s.hinv, &s.traj, &s.lcm, &s.odom_dist, &s.flags, &s.accepted, &s.m, &s.c_from, &s.c_to,
-                      &s.c_lcm, &s.adj, &s.counters, &s.deg, &s.cidx, &s.ck, &s.cb_state, &s.cb_icc, &s.cb_dm,
+                      &s.c_lcm, &s.adj, &s.counters, &s.deg, &s.cidx, &s.ck, &s.cb_state, &s.cb_icc, &s.cb_dm, &s.cb_diag, &s.cb_grp,
                       &s.cb_xorder})
       key.push_back((long long)(uintptr_t)b->ptr);
     if (s.exec && key == s.graph_key) {

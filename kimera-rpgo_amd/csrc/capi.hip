@@ -103,8 +103,8 @@ int rpgo_ctx_destroy(rpgo_ctx* ctx) {
                     &s.queue, &s.tmp, &s.chain_off})
     b->release();
   CliqueState& q = ctx->clq;
-  for (DevBuf* b : {&q.adj, &q.deg, &q.dmask, &q.icc, &q.out, &q.scratch, &q.best, &q.ex_adj,
-                    &q.ex_ctl, &q.ex_stack, &q.ex_path})
+  for (DevBuf* b : {&q.adj, &q.deg, &q.dmask, &q.icc, &q.out, &q.scratch, &q.best, &q.cidx, &q.ccol, &q.cdmask,
+                    &q.cadj, &q.cn, &q.caux, &q.picks, &q.replay, &q.ex_adj, &q.ex_ctl, &q.ex_stack, &q.ex_path})
     b->release();
   solver_destroy(ctx);
   mlp_destroy(ctx);

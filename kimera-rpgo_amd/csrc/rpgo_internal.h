@@ -120,6 +120,7 @@ struct CliqueState {
   DevBuf adj;      // caller-provided adjacency (rpgo_max_clique_bits)
   DevBuf deg, dmask, icc, out, scratch, best;
   DevBuf cidx, ccol, cdmask, cadj, cn;  // the heuristic rounds' compacted graph
+  DevBuf caux, picks, replay;           // its derived rows, the walks' picks, the replay
   DevBuf ex_adj, ex_ctl, ex_stack, ex_path;  // exact mode (clique_exact.hip)
 };
 
@@ -140,12 +141,14 @@ struct rpgo_ctx {
   rpgo::SolveLanes* solve_lanes = nullptr;  // created by rpgo_solve_batched
   rpgo::MlpState* mlp = nullptr;      // created by rpgo_mlp_set_params
   rpgo::BatchState* batch = nullptr;  // created by rpgo_pcm_batch_run
-  void* host_pinned = nullptr;        // 256 B pinned host buffer for counter readbacks
+  void* host_pinned = nullptr;        // 256 B pinned host buffer for counter readbacks (PCM
+                                      // counters in the first 128, clique results after them)
   int n_cu = 256;                     // compute units of the device (launch shapes)
   bool stage_timing = true;           // HIP events around the PCM pass stages (ms_* of the stats)
 };
 
 namespace rpgo {
+constexpr int kPinnedClique = 128;  // byte offset in rpgo_ctx::host_pinned
 // PcmSimple thresholds of one check (translation, rotation per node);
 // a negative value disables the check
 struct SimpleThr {
@@ -246,6 +249,8 @@ struct CliqueSpread {
   void* state;
   int* icc;
   unsigned long long* dm;
+  unsigned long long* diag;  // n_slots words: each vertex's word of its own block
+  unsigned long long* grp;   // group rows, laid out like the adjacency
   const int* xorder;  // graphs grouped by XCD (n_graphs entries), then 9 group offsets
   int xmax;           // graphs of the largest group
 };

@@ -56,7 +56,7 @@ struct BatchState {
   int fp32_S = 4;
   std::vector<long long> blk_off, sq_off, pblk_off;
   DevBuf d_blk_off, d_sq_off, d_pblk_off;
-  DevBuf fp_prec, fp_lcr, fp_pl64, fp_pb64, fp_bend, fp_ta, fp_sanc, fp_terms, fp_queue;
+  DevBuf fp_prec, fp_lcr, fp_bend, fp_ta, fp_sanc, fp_terms, fp_queue;
   long long fp_qcap = 0;
   // launch shapes chosen by the autotuner, per tune_slot() (0: not tuned yet)
   int tuned_pair[8] = {}, tuned_clique[8] = {};
@@ -321,7 +321,7 @@ void batch_destroy(rpgo_ctx* ctx) {
                     &s.odom, &s.odom_cov, &s.lc_from, &s.lc_to, &s.lc_pose, &s.lc_cov, &s.delta, &s.hinv, &s.traj,
                     &s.lcm, &s.odom_dist, &s.flags, &s.accepted, &s.m, &s.c_from, &s.c_to, &s.c_lcm, &s.adj,
                     &s.counters, &s.deg, &s.cidx, &s.ck, &s.cb_state, &s.cb_icc, &s.cb_dm, &s.cb_diag, &s.cb_grp, &s.cb_xorder, &s.d_blk_off,
-                    &s.d_sq_off, &s.d_pblk_off, &s.fp_prec, &s.fp_lcr, &s.fp_pl64, &s.fp_pb64, &s.fp_bend, &s.fp_ta,
+                    &s.d_sq_off, &s.d_pblk_off, &s.fp_prec, &s.fp_lcr, &s.fp_bend, &s.fp_ta,
                     &s.fp_sanc, &s.fp_terms, &s.fp_queue})
     b->release();
   if (s.exec) (void)hipGraphExecDestroy(s.exec);
@@ -394,17 +394,14 @@ static BatchFp32Args fp32_args(BatchState& s) {
   a.pblk_off = s.d_pblk_off.as<long long>();
   a.m = s.m.as<int>();
   a.delta = s.delta.as<double>();
-  a.hinv = s.hinv.as<double>();
   a.lcm = s.lcm.as<double>();
-  a.pose0 = s.pose0.as<double>();
+  a.traj = s.traj.as<double>();
   a.c_from = s.c_from.as<int>();
   a.c_to = s.c_to.as<int>();
   a.c_lcm = s.c_lcm.as<double>();
   a.prec = s.fp_prec.ptr;
   a.lcr = s.fp_lcr.ptr;
   a.sanc = s.fp_sanc.ptr;
-  a.pl64 = s.fp_pl64.as<double>();
-  a.pb64 = s.fp_pb64.as<double>();
   a.bend = s.fp_bend.as<double>();
   a.ta = s.fp_ta.as<double>();
   a.terms = s.fp_terms.as<double>();
@@ -725,8 +722,7 @@ int rpgo_pcm_batch_run(rpgo_ctx* ctx, const rpgo_pcm_batch* B, const rpgo_pcm_pa
         (rc = up(s.d_pblk_off, s.pblk_off.data(), sizeof(long long) * (G + 1), st)) ||
         (rc = s.fp_prec.reserve(pcm_fp32_pose_rec_bytes() * (size_t)s.n_poses)) ||
         (rc = s.fp_lcr.reserve(pcm_fp32_lc_rec_bytes() * nl1)) ||
-        (rc = s.fp_pl64.reserve(sizeof(double) * 12 * (size_t)s.n_poses)) ||
-        (rc = s.fp_pb64.reserve(sizeof(double) * 12 * nb)) || (rc = s.fp_ta.reserve(sizeof(double) * 12 * nb)) ||
+        (rc = s.fp_ta.reserve(sizeof(double) * 12 * nb)) ||
         (rc = s.fp_bend.reserve(sizeof(double) * 36 * nb)) ||
         (rc = s.fp_sanc.reserve(pcm_fp32_anchor_entry_bytes() * nsq)) ||
         (rc = s.fp_terms.reserve(sizeof(double) * 36 * nsq)) ||
@@ -802,8 +798,8 @@ int rpgo_pcm_batch_run(rpgo_ctx* ctx, const rpgo_pcm_batch* B, const rpgo_pcm_pa
                                   bm, bc, s.cb_xmax};
     if (s.fp32) {
       key.insert(key.end(), {s.fp32_S, s.blk_off[G], s.sq_off[G], s.pblk_off[G], s.fp_qcap});
-      for (DevBuf* b : {&s.d_blk_off, &s.d_sq_off, &s.d_pblk_off, &s.fp_prec, &s.fp_lcr, &s.fp_pl64, &s.fp_pb64,
-                        &s.fp_bend, &s.fp_ta, &s.fp_sanc, &s.fp_terms, &s.fp_queue})
+      for (DevBuf* b : {&s.d_blk_off, &s.d_sq_off, &s.d_pblk_off, &s.fp_prec, &s.fp_lcr, &s.fp_bend,
+                        &s.fp_ta, &s.fp_sanc, &s.fp_terms, &s.fp_queue})
         key.push_back((long long)(uintptr_t)b->ptr);
     }
     for (DevBuf* b : {&s.d_pose_off, &s.d_lc_off, &s.d_adj_off, &s.d_tile_off, &s.d_sym_off, &s.d_lc_graph,

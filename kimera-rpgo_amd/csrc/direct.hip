@@ -2,11 +2,11 @@
 // multifrontal block Cholesky in FP64 on the elimination plan of
 // direct_plan.h, one launch per level, the pivots of a level independent.
 //
-// A front is one pose and its d remaining neighbours.  Its workgroup gathers
-// the pivot's column (diagonal block, damping, the between factors assembled
-// here, the children's update matrices) into LDS, factors the 6x6 pivot,
-// forms G_k = F_k L^-T for the neighbours, and writes the update matrix
-//   U_kl = sum over children U_kl - G_k G_l^T      (k >= l)
+// A front is a run of s pivots and the rows they share.  Its workgroup gathers
+// the pivots' columns (diagonal blocks, damping, the between factors assembled
+// here, the children's update matrices) into LDS, factors the panel column by
+// column, and writes the update matrix
+//   U_kl = sum over children U_kl - sum over pivots G_kq G_lq^T      (k >= l)
 // for its parent; the right-hand side is one more row of the same elimination,
 // so the forward substitution costs no pass of its own.  The backward
 // substitution runs the levels in reverse.  Every sum has a fixed order: no
@@ -17,9 +17,9 @@
 // four dependent launches.  The whole factorization is about 0.2 GFLOP and
 // 270 MB there; what bounds it is the chain of dependent levels (83 at 50,000
 // poses with 5,000 loop closures), each about as long as one PCG launch.
-// LM at 50,000 poses 429 -> 36 ms, GNC at 3,000 poses 1,404 -> 378 ms, planar
-// GNC at 500 poses 855 -> 110 ms, eight GNC solves of 200-2,000 poses on four
-// lanes 1,689 -> 285 ms (PCG -> this, wall time of the call).
+// LM at 50,000 poses 814 -> 44 ms, GNC at 3,000 poses 1,639 -> 294 ms, planar
+// GNC at 500 poses 776 -> 70 ms, eight GNC solves of 200-2,000 poses on four
+// lanes 1,710 -> 229 ms (PCG -> this, wall time of the call).
 #include <cmath>
 #include <new>
 
@@ -36,10 +36,6 @@ namespace rpgo {
 // of regular ones stay well above (about 1e-10 at the end of a 50,000-pose
 // chain).
 constexpr double kPivotMin = 1e-13;
-
-// rows of a front column in LDS: 6 (d + 1) rows of the blocks, then the
-// right-hand side
-__host__ __device__ constexpr size_t front_lds_doubles(int d) { return 36 * (size_t)(d + 1) + 6; }
 
 __device__ __forceinline__ void load6(const double* __restrict__ s, double (&v)[6]) {
   const double2* q = reinterpret_cast<const double2*>(s);  // every block row is 16-byte aligned
@@ -74,246 +70,515 @@ __device__ __forceinline__ void row_solve(const double (&L)[36], double (&v)[6])
   }
 }
 
-template <int TB>
-__global__ void __launch_bounds__(TB) k_front(int first, const FrontMeta* __restrict__ meta,
-                                              const FrontChild* __restrict__ childs,
-                                              const FrontOrig* __restrict__ origs, const int* __restrict__ maps,
-                                              const double* __restrict__ D, const double* __restrict__ hdiag,
-                                              const double* __restrict__ b, const double* __restrict__ Hij,
-                                              double lambda, int diag_damping, double* U, double* __restrict__ G,
-                                              double* __restrict__ Lo, double* __restrict__ Y,
-                                              int* __restrict__ bad) {
-  extern __shared__ __align__(16) double row[];
-  const int p = first + blockIdx.x, tid = threadIdx.x;
-  const FrontMeta m = meta[p];
-  const int d = m.d, nrow = 6 * (d + 1);
-  for (int t = tid; t <= nrow; t += TB) {
-    double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    if (t < nrow) {
-      const int k = t / 6, i = t - 6 * k;
-      if (k == 0) {
-        load6(D + (size_t)m.pose * 36 + 6 * i, v);
-        const double dd = diag_damping ? fmin(fmax(hdiag[(size_t)m.pose * 6 + i], 1e-6), 1e32) : 1.0;
-#pragma unroll
-        for (int j = 0; j < 6; ++j) v[j] += j == i ? lambda * dd : 0.0;
-      } else {
-        for (int o = 0; o < m.n_orig; ++o) {
-          const FrontOrig a = origs[m.orig_off + o];
-          if ((a.slot_t >> 1) != k) continue;
-          const double* B = Hij + (size_t)a.f * 36;
-          if (a.slot_t & 1) {
-#pragma unroll
-            for (int j = 0; j < 6; ++j) v[j] += B[j * 6 + i];
-          } else {
-            add6(B + 6 * i, v);
-          }
-        }
-      }
-      for (int c = 0; c < m.n_child; ++c) {
-        const FrontChild ch = childs[m.child_off + c];
-        const int pk = maps[ch.map_off + k];
-        if (pk >= 0) add6(U + ch.u_off + 36 * (pk * (pk + 1) / 2) + 6 * i, v);
-      }
-    } else {
-      load6(b + (size_t)m.pose * 6, v);
-      for (int c = 0; c < m.n_child; ++c) {
-        const FrontChild ch = childs[m.child_off + c];
-        add6(U + ch.u_off + 36 * ((size_t)ch.d * (ch.d + 1) / 2), v);
-      }
-    }
-    store6(row + 6 * t, v);
-  }
-  __syncthreads();
-  // 6x6 Cholesky of the pivot, in every thread (broadcast reads of rows 0-5,
-  // which nothing writes until the next barrier)
-  double L[36], hd[6];
-  load6(hdiag + (size_t)m.pose * 6, hd);
+// 6x6 Cholesky of the block at s, in every thread (broadcast reads); L lower
+// with its diagonal inverted.  False when a pivot is noise of its pose's own
+// diagonal hd, or NaN.
+__device__ __forceinline__ bool block_factor(const double* s, const double (&hd)[6], double (&L)[36]) {
   bool ok = true;
 #pragma unroll
   for (int c = 0; c < 6; ++c) {
 #pragma unroll
     for (int r = c; r < 6; ++r) {
-      double v = row[r * 6 + c];
+      double v = s[r * 6 + c];
 #pragma unroll
       for (int k = 0; k < c; ++k) v -= L[r * 6 + k] * L[c * 6 + k];
       if (r == c) {
-        ok = ok && v > kPivotMin * hd[c] && v > 0.0;  // false for NaN too
-        L[c * 7] = 1.0 / sqrt(fmax(v, 1e-300));
+        ok = ok && v > kPivotMin * hd[c] && v > 0.0;
+        L[c * 7] = rsqrt(fmax(v, 1e-300));
       } else {
         L[r * 6 + c] = v * L[c * 7];
       }
     }
   }
-  for (int t = 6 + tid; t <= nrow; t += TB) {
-    double v[6];
-    load6(row + 6 * t, v);
-    row_solve(L, v);
-    store6(row + 6 * t, v);
-    if (blockIdx.y == 0) {
-      if (t < nrow) store6(G + 36 * (size_t)m.nb_off + 6 * (t - 6), v);
-      else store6(Y + 6 * (size_t)p, v);
+  return ok;
+}
+
+__device__ __forceinline__ void load_lower(const double* s, double (&L)[36]) {
+#pragma unroll
+  for (int r = 0; r < 6; ++r)
+#pragma unroll
+    for (int c = 0; c <= r; ++c) L[r * 6 + c] = s[r * 6 + c];
+}
+
+// v += the children's update rows at block (R, C), row i; R = -1: their
+// vectors at C.  Two children at a time, so their loads overlap.
+__device__ __forceinline__ void gather_children(const FrontMeta& m, const FrontChild* __restrict__ childs,
+                                                const int* __restrict__ maps, const double* U, int R, int C, int i,
+                                                double (&v)[6]) {
+  for (int c = 0; c < m.n_child; c += 2) {
+    double a[2][6];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int e = 0; e < 6; ++e) a[u][e] = 0.0;
+      if (c + u < m.n_child) {
+        const FrontChild ch = childs[m.child_off + c + u];
+        const int* map = maps + m.map_off + (size_t)(c + u) * m.n;
+        const int pl = map[C], pk = R < 0 ? pl : map[R];
+        if (pl >= 0 && pk >= 0)
+          load6(U + ch.u_off + (R < 0 ? 36 * ((size_t)ch.d * (ch.d + 1) / 2) + 6 * pl
+                                      : 36 * ((size_t)pk * (pk + 1) / 2 + pl) + 6 * i),
+                a[u]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 6; ++e) v[e] = (v[e] + a[0][e]) + a[1][e];
+  }
+}
+
+// the sum of a run of between factors of one block, row i
+__device__ __forceinline__ void gather_factors(const FrontOrig* __restrict__ o, int i, const double* __restrict__ Hij,
+                                               double (&v)[6]) {
+  const int run = o->run;
+  for (int k = 0; k < run; ++k) {
+    const double* B = Hij + (size_t)o[k].f * 36;
+    if (o[k].slot & 1) {
+#pragma unroll
+      for (int j = 0; j < 6; ++j) v[j] += B[j * 6 + i];
+    } else {
+      add6(B + 6 * i, v);
     }
   }
-  if (tid == 0 && blockIdx.y == 0) {
+}
+
+// block index of the lower triangle -> row and column
+__device__ __forceinline__ void tri_index(int blk, int* k, int* l) {
+  int r = (int)((sqrtf(8.0f * (float)blk + 1.0f) - 1.0f) * 0.5f);
+  while ((r + 1) * (r + 2) / 2 <= blk) ++r;
+  while (r * (r + 1) / 2 > blk) --r;
+  *k = r;
+  *l = blk - r * (r + 1) / 2;
+}
+
+// Element (ri, ci) of a front's update matrix (scalar rows and columns of the
+// front from 6 s on; row 6 n: the update vector): its place from u_off, or -1
+// above the block diagonal
+__device__ __forceinline__ long long update_at(int n, int s, int ri, int ci) {
+  const int k = ri / 6 - s, i = ri % 6, l = ci / 6 - s, j = ci % 6;
+  if (ci >= 6 * n || ri > 6 * n || k < l) return -1;
+  const long long blk = (long long)k * (k + 1) / 2;
+  if (ri == 6 * n) return 36 * ((long long)(n - s) * (n - s + 1) / 2) + 6 * l + j;
+  return 36 * (blk + l) + 6 * i + j;
+}
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+// Where element (row ri, scalar column ci) of the panel stands, less 6 ri
+__device__ __forceinline__ int panel_col(int n, int ci) {
+  const int q = (ci * 43691) >> 18;  // ci / 6, exact below 1 << 16
+  return 6 * (__mul24(6 * q, n) - 3 * __mul24(q, q - 1) - 5 * q) + ci - 6 * q;
+}
+
+// c - P(r0 .., k0 .. k1) P(c0 .., k0 .. k1)^T of the panel in LDS, a 16x16
+// tile: lane holds column lane % 16, rows 4 r + lane / 16.  Rows past the
+// panel repeat its last one (their results are not stored).
+__device__ __forceinline__ d4 tile_product(const double* row, int n, int r0, int c0, int k0, int k1, int lane, d4 c) {
+  const int ra = 6 * min(r0 + (lane & 15), 6 * n), rb = 6 * min(c0 + (lane & 15), 6 * n);
+  for (int k = k0; k < k1; k += 4) {
+    const int g = k + (lane >> 4);
+    const double* col = row + panel_col(n, min(g, k1 - 1));
+    const double a = col[ra], b = col[rb];
+    c = __builtin_amdgcn_mfma_f64_16x16x4f64(g < k1 ? -a : 0.0, g < k1 ? b : 0.0, c, 0, 0, 0);
+  }
+  return c;
+}
+
+// A front's panel from the Hessian, the between factors and the children's
+// updates; `mid` runs while those loads are in flight.
+template <int TB, class F>
+__device__ __forceinline__ void front_gather(const FrontMeta& m, const FrontChild* __restrict__ childs,
+                                             const FrontOrig* __restrict__ origs, const int* __restrict__ maps,
+                                             const int* __restrict__ rows, const double* __restrict__ D,
+                                             const double* __restrict__ hdiag, const double* __restrict__ b,
+                                             const double* __restrict__ Hij, double lambda, int diag_damping,
+                                             const double* U, double* row, F&& mid) {
+  const int tid = threadIdx.x, n = m.n, s = m.s, w = 6 * n + 1;
+  // the pivots' own diagonals behind the panel (a load per pivot in the
+  // factorization would be two memory latencies each)
+  for (int q = tid; q < s; q += TB) {
+    double v[6];
+    load6(hdiag + (size_t)rows[m.row_off + q] * 6, v);
+    store6(row + 6 * (panel_row(n, s) + q), v);
+  }
+  // panel rows: column q, row i of block R (R = n: the right-hand side)
+  for (int t = tid; t < s * w; t += TB) {
+    const int q = t / w, rr = t - q * w, R = rr / 6, i = rr - 6 * R;
+    if (R < q) continue;
+    double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    if (R == n) {
+      load6(b + (size_t)rows[m.row_off + q] * 6, v);
+      gather_children(m, childs, maps, U, -1, q, 0, v);
+    } else {
+      if (R == q) {
+        const size_t pose = (size_t)rows[m.row_off + q];
+        load6(D + pose * 36 + 6 * i, v);
+        const double dd = diag_damping ? fmin(fmax(hdiag[pose * 6 + i], 1e-6), 1e32) : 1.0;
+#pragma unroll
+        for (int j = 0; j < 6; ++j) v[j] += j == i ? lambda * dd : 0.0;
+      }
+      gather_children(m, childs, maps, U, R, q, i, v);
+    }
+    store6(row + 6 * (panel_row(n, q) + rr - 6 * q), v);
+  }
+  // the between factors' blocks, each by the first of its run; by other
+  // wavefronts than the panel's first rows and `mid`, so that the three chains
+  // of dependent loads run side by side
+  const FrontOrig* og = origs + m.orig_off;
+  const int to = (tid + TB / 2) % TB;
+  double ov[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  if (to < 6 * m.n_orig) gather_factors(og + to / 6, to % 6, Hij, ov);
+  mid();
+  __syncthreads();
+  if (m.n_orig == 0) return;
+  for (int t = to; t < 6 * m.n_orig; t += TB) {
+    const FrontOrig* o = og + t / 6;
+    if (o->run == 0) continue;
+    const int q = o->slot >> 16, R = (o->slot >> 1) & 0x7fff;
+    if (t != to) {
+#pragma unroll
+      for (int e = 0; e < 6; ++e) ov[e] = 0.0;
+      gather_factors(o, t % 6, Hij, ov);
+    }
+    double* r = row + 6 * (panel_row(n, q) + 6 * (R - q) + t % 6);
+    add6(r, ov);
+    store6(r, ov);
+  }
+  __syncthreads();
+}
+
+// The 6x6 pivot of column q and the rows below it; afterwards the factor's
+// block stands in place of the pivot.  Only wavefronts with rows to solve
+// factor the pivot: all sixteen of a workgroup doing so cost 1.5 us a pivot in
+// LDS reads and FP64 issue.
+template <int TB>
+__device__ __forceinline__ void front_pivot(const FrontMeta& m, int q, double* row, int* bad) {
+  const int tid = threadIdx.x, nr = 6 * (m.n - q), w0 = __builtin_amdgcn_readfirstlane(tid & ~63);
+  double* col = row + 6 * panel_row(m.n, q);
+  double L[36];
+  bool ok = true;
+  if (w0 == 0 || 6 + w0 <= nr) {
+    double hd[6];
+    load6(row + 6 * (panel_row(m.n, m.s) + q), hd);
+    ok = block_factor(col, hd, L);
+    for (int t = 6 + tid; t <= nr; t += TB) {
+      double v[6];
+      load6(col + 6 * t, v);
+      row_solve(L, v);
+      store6(col + 6 * t, v);
+    }
+  }
+  __syncthreads();
+  if (tid == 0) {
 #pragma unroll
     for (int r = 0; r < 6; ++r)
 #pragma unroll
-      for (int c = 0; c <= r; ++c) Lo[(size_t)p * 36 + r * 6 + c] = L[r * 6 + c];
-    if (!ok) *bad = 1;
+      for (int c = 0; c <= r; ++c) col[r * 6 + c] = L[r * 6 + c];
+    if (!ok && blockIdx.y == 0) *bad = 1;
   }
-  __syncthreads();
-  // update rows: row i of block (k, l), then the update vector's blocks
-  const int nblk = d * (d + 1) / 2, ntask = 6 * nblk + d;
-  for (int t = blockIdx.y * TB + tid; t < ntask; t += TB * gridDim.y) {
-    double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+}
+
+#define RPGO_FRONT_PARAMS                                                                                      \
+  int first, const FrontMeta *__restrict__ meta, const FrontChild *__restrict__ childs,                        \
+      const FrontOrig *__restrict__ origs, const int *__restrict__ maps, const int *__restrict__ rows,         \
+      const double *__restrict__ D, const double *__restrict__ hdiag, const double *__restrict__ b,            \
+      const double *__restrict__ Hij, double lambda, int diag_damping, double *U, double *__restrict__ G,      \
+      int *__restrict__ bad
+
+// Small fronts (the thousands of the first levels), every update row of six
+// by one lane
+template <int TB>
+__global__ void __launch_bounds__(TB) k_front_small(RPGO_FRONT_PARAMS) {
+  extern __shared__ __align__(16) double row[];
+  const int tid = threadIdx.x, t0 = TB - 1 - tid;
+  const FrontMeta m = meta[first + blockIdx.x];
+  const int n = m.n, s = m.s, d = n - s, nblk = d * (d + 1) / 2, ntask = 6 * nblk + d;
+  // the first update row's children are loaded before the panel is factored
+  const auto children = [&](int t, double (&v)[6]) {
     if (t < 6 * nblk) {
-      const int blk = t / 6, i = t - 6 * blk;
-      int k = (int)((sqrtf(8.0f * (float)blk + 1.0f) - 1.0f) * 0.5f);
-      while ((k + 1) * (k + 2) / 2 <= blk) ++k;
-      while (k * (k + 1) / 2 > blk) --k;
-      const int l = blk - k * (k + 1) / 2;
-      for (int c = 0; c < m.n_child; ++c) {
-        const FrontChild ch = childs[m.child_off + c];
-        const int pk = maps[ch.map_off + k + 1], pl = maps[ch.map_off + l + 1];
-        if (pk >= 0 && pl >= 0) add6(U + ch.u_off + 36 * (pk * (pk + 1) / 2 + pl) + 6 * i, v);
-      }
-      double g[6];
-      load6(row + 36 * (k + 1) + 6 * i, g);
+      int k, l;
+      tri_index(t / 6, &k, &l);
+      gather_children(m, childs, maps, U, s + k, s + l, t % 6, v);
+    } else {
+      gather_children(m, childs, maps, U, -1, s + t - 6 * nblk, 0, v);
+    }
+  };
+  double pre[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  front_gather<TB>(m, childs, origs, maps, rows, D, hdiag, b, Hij, lambda, diag_damping, U, row, [&] {
+    if (t0 < ntask) children(t0, pre);
+  });
+  for (int q = 0; q < s; ++q) {
+    const double* col = row + 6 * panel_row(n, q);
+    front_pivot<TB>(m, q, row, bad);
+    // the panel's other columns
+    const int wq = 6 * (n - q) - 5, nc = s - 1 - q;
+    for (int t = tid; t < nc * wq; t += TB) {
+      const int C = t / wq, rr = t - C * wq;  // both from q + 1
+      if (rr < 6 * C) continue;
+      double* r = row + 6 * (panel_row(n, q + 1 + C) + rr - 6 * C);
+      const double* hc = col + 36 * (C + 1);
+      double v[6], g[6];
+      load6(r, v);
+      load6(col + 6 * (6 + rr), g);
 #pragma unroll
       for (int j = 0; j < 6; ++j) {
         double h[6];
-        load6(row + 36 * (l + 1) + 6 * j, h);
+        load6(hc + 6 * j, h);
 #pragma unroll
-        for (int q = 0; q < 6; ++q) v[j] -= g[q] * h[q];
+        for (int k = 0; k < 6; ++k) v[j] -= g[k] * h[k];
       }
-      store6(U + m.u_off + 36 * (size_t)blk + 6 * i, v);
+      store6(r, v);
+    }
+    __syncthreads();
+  }
+  {
+    const double2* src = reinterpret_cast<const double2*>(row);
+    double2* dst = reinterpret_cast<double2*>(G + m.g_off);
+    for (int t = tid; t < 3 * panel_row(n, s); t += TB) dst[t] = src[t];
+  }
+  for (int t = t0; t < ntask; t += TB) {
+    double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    if (t == t0) {
+#pragma unroll
+      for (int e = 0; e < 6; ++e) v[e] = pre[e];
     } else {
-      const int k = t - 6 * nblk;
-      for (int c = 0; c < m.n_child; ++c) {
-        const FrontChild ch = childs[m.child_off + c];
-        const int pk = maps[ch.map_off + k + 1];
-        if (pk >= 0) add6(U + ch.u_off + 36 * ((size_t)ch.d * (ch.d + 1) / 2) + 6 * pk, v);
-      }
-      double y[6];
-      load6(row + 6 * nrow, y);
+      children(t, v);
+    }
+    int k = d, l = t - 6 * nblk, i = 0;  // the right-hand side's row is row 0 of block n
+    if (t < 6 * nblk) {
+      tri_index(t / 6, &k, &l);
+      i = t % 6;
+    }
+    for (int q = 0; q < s; ++q) {
+      const double* col = row + 6 * panel_row(n, q);
+      double g[6];
+      load6(col + 36 * (s + k - q) + 6 * i, g);
 #pragma unroll
-      for (int i = 0; i < 6; ++i) {
+      for (int j = 0; j < 6; ++j) {
         double h[6];
-        load6(row + 36 * (k + 1) + 6 * i, h);
+        load6(col + 36 * (s + l - q) + 6 * j, h);
 #pragma unroll
-        for (int q = 0; q < 6; ++q) v[i] -= h[q] * y[q];
+        for (int e = 0; e < 6; ++e) v[j] -= g[e] * h[e];
       }
-      store6(U + m.u_off + 36 * (size_t)nblk + 6 * k, v);
+    }
+    store6(U + m.u_off + 6 * (size_t)t, v);
+  }
+}
+
+// Wider fronts, a workgroup each (gridDim.y of them share a front's update
+// tiles, each repeating the panel).  What bounds it is latency: meta, maps and
+// update matrix are dependent loads, then each pivot is a 6x6 Cholesky and two
+// barriers (1.6 us; the 3,000-pose graph's levels of five to ten pivots take
+// 23 to 37 us, where a launch per pivot took 6.7 us and a gap each).  Updates
+// go 16x16 tiles at a time through the matrix cores; by rows of six in vector
+// FMA they were bound by the LDS (21 16-byte reads for 36 FMAs) and a level of
+// 50,000 poses took 45 us against 34.
+template <int TB>
+__global__ void __launch_bounds__(TB) k_front(RPGO_FRONT_PARAMS) {
+  extern __shared__ __align__(16) double row[];
+  constexpr int NW = TB / 64;
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const FrontMeta m = meta[first + blockIdx.x];
+  const int n = m.n, s = m.s, T = (6 * (n - s) + 16) / 16, ntile = T * (T + 1) / 2;
+  // children's sum of update tile (ti, tj)
+  const auto children = [&](int t) {
+    d4 c = {0.0, 0.0, 0.0, 0.0};
+    int ti, tj;
+    tri_index(t, &ti, &tj);
+    const int ci = 6 * s + 16 * tj + (lane & 15), r0 = 6 * s + 16 * ti + (lane >> 4);
+    if (ci >= 6 * n) return c;
+    const int l = ci / 6, j = ci - 6 * l;
+    for (int k = 0; k < m.n_child; k += 2) {  // two children's loads overlap
+      double v[2][4];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const bool has = k + u < m.n_child;
+        const FrontChild ch = childs[m.child_off + (has ? k + u : k)];
+        const int* map = maps + m.map_off + (size_t)(has ? k + u : k) * n;
+        const int pl = map[l];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int ri = r0 + 4 * r, R = ri / 6;
+          const int pk = ri >= 6 * n ? ch.d : map[R];
+          const size_t o = 36 * ((size_t)pk * (pk + 1) / 2 + (ri == 6 * n ? 0 : pl)) +
+                           (ri == 6 * n ? 6 * pl : 6 * (ri - 6 * R)) + j;
+          v[u][r] = has && pl >= 0 && pk >= pl && R >= l && ri <= 6 * n ? U[ch.u_off + o] : 0.0;
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) c[r] = (c[r] + v[0][r]) + v[1][r];
+    }
+    return c;
+  };
+  const int t0 = blockIdx.y * NW + NW - 1 - wv;
+  d4 pre = {0.0, 0.0, 0.0, 0.0};
+  // the first tile's children are loaded before the panel is factored
+  front_gather<TB>(m, childs, origs, maps, rows, D, hdiag, b, Hij, lambda, diag_damping, U, row, [&] {
+    if (n > s && t0 < ntile) pre = children(t0);
+  });
+  for (int q = 0; q < s; ++q) {
+    front_pivot<TB>(m, q, row, bad);
+    // the panel's other columns: a strip of 16 rows to two wavefronts, each
+    // every other tile, its own fragments held over them
+    const int c0 = 6 * (q + 1), nct = (6 * s - c0 + 15) / 16, nrt = (6 * n + 16 - c0) / 16;
+    const int g0 = 6 * q + (lane >> 4), g1 = min(g0 + 4, 6 * q + 5);
+    const double *f0 = row + panel_col(n, g0), *f1 = row + panel_col(n, g1);
+    for (int ti = nct > 0 ? wv >> 1 : nrt; ti < nrt; ti += NW / 2) {
+      const int ra = 6 * min(c0 + 16 * ti + (lane & 15), 6 * n), r0 = c0 + 16 * ti + (lane >> 4);
+      const double a0 = -f0[ra], a1 = lane < 32 ? -f1[ra] : 0.0;
+      for (int tj = wv & 1; tj < nct && tj <= ti; tj += 2) {
+        const int ci = min(c0 + 16 * tj + (lane & 15), 6 * s - 1), rb = 6 * (c0 + 16 * tj + (lane & 15));
+        const int rc = min(rb, 36 * n);
+        double* p = row + panel_col(n, ci);
+        const double b0 = f0[rc], b1 = f1[rc];
+        d4 c;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) c[r] = p[6 * min(r0 + 4 * r, 6 * n)];
+        c = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, c, 0, 0, 0);
+        c = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, lane < 32 ? b1 : 0.0, c, 0, 0, 0);
+        const bool in = rb < 36 * s;
+        const int top = ci - ci % 6;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (in && r0 + 4 * r <= 6 * n && r0 + 4 * r >= top) p[6 * (r0 + 4 * r)] = c[r];
+      }
+    }
+    __syncthreads();
+  }
+  // the factored panel, then the update tiles
+  {
+    const double2* src = reinterpret_cast<const double2*>(row);
+    double2* dst = reinterpret_cast<double2*>(G + m.g_off);
+    const int np = 3 * panel_row(n, s);
+    for (int t = blockIdx.y * TB + tid; t < np; t += TB * gridDim.y) dst[t] = src[t];
+  }
+  if (n == s) return;
+  for (int t = t0; t < ntile; t += NW * gridDim.y) {
+    int ti, tj;
+    tri_index(t, &ti, &tj);
+    const int c0 = 6 * s + 16 * tj, r0 = 6 * s + 16 * ti;
+    if (c0 >= 6 * n) continue;
+    const d4 c = tile_product(row, n, r0, c0, 0, 6 * s, lane, t == t0 ? pre : children(t));
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const long long o = update_at(n, s, r0 + 4 * r + (lane >> 4), c0 + (lane & 15));
+      if (o >= 0) U[m.u_off + o] = c[r];
     }
   }
 }
 
 // Forward substitution of another right-hand side with the stored factor
-// (iterative refinement): one wavefront per front, the update vectors in the
-// fronts' own vector slots.
-__global__ void __launch_bounds__(64) k_front_forward(int first, const FrontMeta* __restrict__ meta,
+// (iterative refinement): the panel copied to LDS, a front's vector behind it,
+// the update vectors in the fronts' own vector slots.
+template <int TB>
+__global__ void __launch_bounds__(TB) k_front_forward(int first, const FrontMeta* __restrict__ meta,
                                                       const FrontChild* __restrict__ childs,
-                                                      const int* __restrict__ maps, const double* __restrict__ b,
-                                                      const double* __restrict__ G, const double* __restrict__ Lo,
-                                                      double* U, double* __restrict__ Y) {
-  const int p = first + blockIdx.x, lane = threadIdx.x;
-  const FrontMeta m = meta[p];
-  const int d = m.d;
-  double y[6], L[36];
-  load6(b + (size_t)m.pose * 6, y);
-  for (int c = 0; c < m.n_child; ++c) {
-    const FrontChild ch = childs[m.child_off + c];
-    add6(U + ch.u_off + 36 * ((size_t)ch.d * (ch.d + 1) / 2), y);
+                                                      const int* __restrict__ maps, const int* __restrict__ rows,
+                                                      const double* __restrict__ b, double* G, double* U) {
+  extern __shared__ __align__(16) double row[];
+  const int tid = threadIdx.x;
+  const FrontMeta m = meta[first + blockIdx.x];
+  const int n = m.n, s = m.s, np = panel_row(n, s), d = n - s, w0 = __builtin_amdgcn_readfirstlane(tid & ~63);
+  double* vec = row + 6 * np;
+  {
+    const double2* src = reinterpret_cast<const double2*>(G + m.g_off);
+    double2* dst = reinterpret_cast<double2*>(row);
+    for (int t = tid; t < 3 * np; t += TB) dst[t] = src[t];
   }
-#pragma unroll
-  for (int r = 0; r < 6; ++r)
-#pragma unroll
-    for (int c = 0; c <= r; ++c) L[r * 6 + c] = Lo[(size_t)p * 36 + r * 6 + c];
-  row_solve(L, y);
-  if (lane == 0) store6(Y + 6 * (size_t)p, y);
-  double* u = U + m.u_off + 36 * ((size_t)d * (d + 1) / 2);
-  for (int k = lane; k < d; k += 64) {
+  for (int R = tid; R < n; R += TB) {
     double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int c = 0; c < m.n_child; ++c) {
-      const FrontChild ch = childs[m.child_off + c];
-      const int pk = maps[ch.map_off + k + 1];
-      if (pk >= 0) add6(U + ch.u_off + 36 * ((size_t)ch.d * (ch.d + 1) / 2) + 6 * pk, v);
-    }
-#pragma unroll
-    for (int i = 0; i < 6; ++i) {
-      double h[6];
-      load6(G + 36 * (size_t)(m.nb_off + k) + 6 * i, h);
-#pragma unroll
-      for (int q = 0; q < 6; ++q) v[i] -= h[q] * y[q];
-    }
-    store6(u + 6 * k, v);
+    if (R < s) load6(b + (size_t)rows[m.row_off + R] * 6, v);
+    gather_children(m, childs, maps, U, -1, R, 0, v);
+    store6(vec + 6 * R, v);
   }
+  __syncthreads();
+  for (int q = 0; q < s; ++q) {
+    const double* col = row + 6 * panel_row(n, q);
+    if (w0 > 0 && 6 + w0 >= 6 * (n - q)) {  // no rows for this wavefront
+      __syncthreads();
+      continue;
+    }
+    double L[36], y[6];
+    load_lower(col, L);
+    load6(vec + 6 * q, y);
+    row_solve(L, y);
+    if (tid == 0) store6(G + m.g_off + 6 * (panel_row(n, q) + 6 * (n - q)), y);
+    for (int t = 6 + tid; t < 6 * (n - q); t += TB) {
+      double h[6], v = vec[6 * q + t];
+      load6(col + 6 * t, h);
+#pragma unroll
+      for (int k = 0; k < 6; ++k) v -= h[k] * y[k];
+      vec[6 * q + t] = v;
+    }
+    __syncthreads();
+  }
+  double* u = U + m.u_off + 36 * ((size_t)d * (d + 1) / 2);
+  for (int t = tid; t < 6 * d; t += TB) u[t] = vec[6 * s + t];
 }
 
-// Backward substitution of one front by one wavefront: x = L^-T (y - sum_k
-// G_k^T x_k), ten neighbours at a time (lane 6 g + j: neighbours g, g + 10,
-// ..., component j), partials added in a fixed order.  s: 64 doubles of LDS.
-__device__ __forceinline__ void front_backward(int p, int lane, const FrontMeta* __restrict__ meta,
-                                               const int* __restrict__ nb, const double* __restrict__ G,
-                                               const double* __restrict__ Lo, const double* __restrict__ Y,
-                                               double* x, double* s) {
-  const FrontMeta m = meta[p];
-  const int g = lane / 6, j = lane - 6 * g;
+// Backward substitution of one level, a workgroup a front: the neighbours'
+// part of every pivot at once (thread e = (pivot, component), the rows split
+// among TB / (6 s) parts, partials added in a fixed order), then the pivots
+// from the last to the first on the triangle in LDS.
+template <int TB>
+__global__ void __launch_bounds__(TB) k_back(int first, const FrontMeta* __restrict__ meta,
+                                             const int* __restrict__ rows, const double* __restrict__ G, double* x) {
+  extern __shared__ __align__(16) double tri[];
+  __shared__ double red[TB];
+  const int tid = threadIdx.x;
+  const FrontMeta m = meta[first + blockIdx.x];
+  const int n = m.n, s = m.s, ns = 6 * s, w0 = __builtin_amdgcn_readfirstlane(tid & ~63);
+  const double* P = G + m.g_off;
+  double* xs = tri + 18 * s * (s + 1);  // the neighbours' x, later the pivots'
+  for (int R = s + tid; R < n; R += TB) {
+    double v[6];
+    load6(x + 6 * (size_t)rows[m.row_off + R], v);
+    store6(xs + 6 * (R - s), v);
+  }
+  for (int q = 0; q < s; ++q) {  // rows of the pivots, blocks (q, q .. s-1)
+    const double2* src = reinterpret_cast<const double2*>(P + 6 * panel_row(n, q));
+    double2* dst = reinterpret_cast<double2*>(tri + 36 * (q * s - q * (q - 1) / 2));
+    for (int t = tid; t < 18 * (s - q); t += TB) dst[t] = src[t];
+  }
+  const int parts = TB / ns, part = tid / ns, e = tid - part * ns, eq = e / 6, j = e - 6 * eq;
+  double y = tid < ns ? P[6 * (panel_row(n, eq) + 6 * (n - eq)) + j] : 0.0;
+  __syncthreads();
   double acc = 0.0;
-  if (g < 10)
-    for (int k = g; k < m.d; k += 10) {
-      const double* B = G + 36 * (size_t)(m.nb_off + k) + j;
-      double xk[6];
-      load6(x + 6 * (size_t)nb[m.nb_off + k], xk);
+  if (part < parts) {
+    const double* B = P + 6 * panel_row(n, eq) + 36 * (s - eq) + j;
+    for (int r = part; r < n - s; r += parts)
 #pragma unroll
-      for (int i = 0; i < 6; ++i) acc += B[6 * i] * xk[i];
-    }
-  s[lane] = acc;
-  fold_wave_sync();
-  double L[36], r[6];
-#pragma unroll
-  for (int i = 0; i < 6; ++i)
-#pragma unroll
-    for (int c = 0; c <= i; ++c) L[i * 6 + c] = Lo[(size_t)p * 36 + i * 6 + c];
-  load6(Y + 6 * (size_t)p, r);
-#pragma unroll
-  for (int i = 0; i < 6; ++i) {
+      for (int i = 0; i < 6; ++i) acc += B[36 * r + 6 * i] * xs[6 * r + i];
+  }
+  red[tid] = acc;
+  __syncthreads();
+  if (tid < ns) {
     double t = 0.0;
-#pragma unroll
-    for (int q = 0; q < 10; ++q) t += s[6 * q + i];
-    r[i] -= t;
+    for (int k = 0; k < parts; ++k) t += red[k * ns + tid];
+    y -= t;
+    xs[tid] = y;
   }
+  __syncthreads();
+  for (int q = s - 1; q >= 0; --q) {
+    if (w0 > 0 && w0 >= 6 * q) {  // no components for this wavefront
+      __syncthreads();
+      continue;
+    }
+    double L[36], r[6];
+    load_lower(tri + 36 * (q * s - q * (q - 1) / 2), L);
+    load6(xs + 6 * q, r);
 #pragma unroll
-  for (int i = 5; i >= 0; --i) {
+    for (int i = 5; i >= 0; --i) {
 #pragma unroll
-    for (int k = i + 1; k < 6; ++k) r[i] -= L[k * 6 + i] * r[k];
-    r[i] *= L[i * 7];
-  }
-  if (lane == 0) store6(x + 6 * (size_t)m.pose, r);
-  fold_wave_sync();
-}
-
-// One level, four fronts per workgroup
-__global__ void __launch_bounds__(256) k_back_level(int first, int count, const FrontMeta* __restrict__ meta,
-                                                    const int* __restrict__ nb, const double* __restrict__ G,
-                                                    const double* __restrict__ Lo, const double* __restrict__ Y,
-                                                    double* x) {
-  __shared__ double s[4][64];
-  const int wv = threadIdx.x >> 6, q = blockIdx.x * 4 + wv;
-  if (q < count) front_backward(first + q, threadIdx.x & 63, meta, nb, G, Lo, Y, x, s[wv]);
-}
-
-// Levels n_lvl-1 down to l0 (few fronts each) in one workgroup, a barrier
-// between levels instead of a launch
-__global__ void __launch_bounds__(1024) k_back_top(int l0, int n_lvl, const int* __restrict__ lvl,
-                                                   const FrontMeta* __restrict__ meta, const int* __restrict__ nb,
-                                                   const double* __restrict__ G, const double* __restrict__ Lo,
-                                                   const double* __restrict__ Y, double* x) {
-  __shared__ double s[16][64];
-  const int wv = threadIdx.x >> 6;
-  for (int l = n_lvl - 1; l >= l0; --l) {
-    for (int p = lvl[l] + wv; p < lvl[l + 1]; p += 16)
-      front_backward(p, threadIdx.x & 63, meta, nb, G, Lo, Y, x, s[wv]);
+      for (int k = i + 1; k < 6; ++k) r[i] -= L[k * 6 + i] * r[k];
+      r[i] *= L[i * 7];
+    }
+    if (tid == 0) store6(x + 6 * (size_t)rows[m.row_off + q], r);
+    if (tid < 6 * q) {
+      const double* B = tri + 36 * (eq * s - eq * (eq - 1) / 2 + q - eq) + j;
+#pragma unroll
+      for (int i = 0; i < 6; ++i) y -= B[6 * i] * r[i];
+      xs[tid] = y;
+    }
     __syncthreads();
   }
 }
@@ -420,7 +685,7 @@ __global__ void k_direct_axpy(long long n, const double* __restrict__ a, double*
 }
 
 // ------------------------------------------------------------------ host
-static_assert(front_lds_doubles(DirectLimits().max_d) * sizeof(double) <= 64 * 1024, "front column in LDS");
+static_assert(panel_bytes(DirectLimits().max_d + 1, 1) <= kPanelBytes, "one pivot's panel in LDS");
 
 int SolverRun::direct_setup(hipStream_t st, const int32_t* h_kind, const int32_t* h_fi, const int32_t* h_fj) {
   direct_ready = false;
@@ -432,44 +697,55 @@ int SolverRun::direct_setup(hipStream_t st, const int32_t* h_kind, const int32_t
   } catch (const std::bad_alloc&) {
     return RPGO_OK;
   }
-  const size_t bytes[6] = {P.meta.size() * sizeof(FrontMeta), P.childs.size() * sizeof(FrontChild),
-                           P.origs.size() * sizeof(FrontOrig), P.nb_pose.size() * sizeof(int32_t),
-                           P.maps.size() * sizeof(int32_t), P.lvl.size() * sizeof(int)};
-  const void* src[6] = {P.meta.data(), P.childs.data(), P.origs.data(), P.nb_pose.data(), P.maps.data(), P.lvl.data()};
-  DevBuf* dst[6] = {&d_meta, &d_childs, &d_origs, &d_nb, &d_maps, &d_lvl};
-  for (int k = 0; k < 6; ++k)
+  const size_t bytes[5] = {P.meta.size() * sizeof(FrontMeta), P.childs.size() * sizeof(FrontChild),
+                           P.origs.size() * sizeof(FrontOrig), P.row_pose.size() * sizeof(int32_t),
+                           P.maps.size() * sizeof(int32_t)};
+  const void* src[5] = {P.meta.data(), P.childs.data(), P.origs.data(), P.row_pose.data(), P.maps.data()};
+  DevBuf* dst[5] = {&d_meta, &d_childs, &d_origs, &d_rows, &d_maps};
+  for (int k = 0; k < 5; ++k)
     if (dst[k]->reserve(bytes[k])) return RPGO_OK;  // no room: keep the iterative solve
   const size_t nblk = (size_t)(N + 63) / 64, ncost = (size_t)(F + 255) / 256;
-  if (d_U.reserve(sizeof(double) * (size_t)P.u_len) || d_G.reserve(sizeof(double) * 36 * P.nb_pose.size()) ||
-      d_L.reserve(sizeof(double) * 36 * (size_t)N) || d_Y.reserve(sizeof(double) * 6 * (size_t)N) ||
+  if (d_U.reserve(sizeof(double) * (size_t)P.u_len) || d_G.reserve(sizeof(double) * (size_t)P.g_len) ||
       d_part.reserve(sizeof(double) * (4 * nblk + ncost)) || d_bad.reserve(sizeof(int)))
     return RPGO_OK;
   if (!pinned_scalars()) return RPGO_OK;
-  for (int k = 0; k < 6; ++k)
+  for (int k = 0; k < 5; ++k)
     if (bytes[k]) RPGO_HIP_CHECK(hipMemcpyAsync(dst[k]->ptr, src[k], bytes[k], hipMemcpyHostToDevice, st));
   RPGO_HIP_CHECK(hipMemsetAsync(d_bad.ptr, 0, sizeof(int), st));
   direct_ready = true;
   return RPGO_OK;
 }
 
+// Where every front of the level is small its update rows go to single lanes:
+// a tile of 16x16 is larger than the whole update below three neighbours, and
+// at n = 8 both take 8 us
+static bool small_level(const DirectPlan& P, int l) { return P.lvl_n[l] <= 8; }
+
 // Factor H + lambda damp and substitute forward with b: one launch per level.
 int SolverRun::direct_factor(hipStream_t st, double lambda) {
   const DirectPlan& P = plan;
   for (int l = 0; l < P.levels(); ++l) {
-    const int first = P.lvl[l], n = P.lvl[l + 1] - first, d = P.lvl_max_d[l];
-    const size_t lds = front_lds_doubles(d) * sizeof(double);
-#define RPGO_FRONT_ARGS                                                                                       \
-  first, d_meta.as<FrontMeta>(), d_childs.as<FrontChild>(), d_origs.as<FrontOrig>(), d_maps.as<int>(),        \
-      D.as<double>(), hdiag.as<double>(), b64.as<double>(), Hij.as<double>(), lambda, prm.lm_diagonal_damping, \
-      d_U.as<double>(), d_G.as<double>(), d_L.as<double>(), d_Y.as<double>(), d_bad.as<int>()
-    if (d <= 4) {
-      k_front<64><<<n, 64, lds, st>>>(RPGO_FRONT_ARGS);
+    const int first = P.lvl[l], n = P.lvl[l + 1] - first;
+    const size_t lds = (size_t)P.lvl_bytes[l];
+#define RPGO_FRONT_ARGS                                                                                          \
+  first, d_meta.as<FrontMeta>(), d_childs.as<FrontChild>(), d_origs.as<FrontOrig>(), d_maps.as<int>(),           \
+      d_rows.as<int>(), D.as<double>(), hdiag.as<double>(), b64.as<double>(), Hij.as<double>(), lambda,          \
+      prm.lm_diagonal_damping, d_U.as<double>(), d_G.as<double>(), d_bad.as<int>()
+    if (small_level(P, l)) {
+      // a wavefront a front where the level fills the chip by itself: 22,520
+      // fronts 50 us; four wavefronts run a front's three chains of loads side
+      // by side: levels of 100 to 600 fronts 11 -> 7.8 us
+      if (n > 4096) k_front_small<64><<<n, 64, lds, st>>>(RPGO_FRONT_ARGS);
+      else k_front_small<256><<<n, 256, lds, st>>>(RPGO_FRONT_ARGS);
     } else {
-      // wide fronts of a narrow level share their update rows among
-      // workgroups, each repeating the pivot column
-      const int rounds = (3 * d * (d + 1) + d + 255) / 256;
-      const int split = std::max(1, std::min(rounds, 1024 / n));
-      k_front<256><<<dim3(n, split), 256, lds, st>>>(RPGO_FRONT_ARGS);
+      // wide fronts of a narrow level share their update tiles among
+      // workgroups, each repeating the panel
+      const int T = (6 * P.lvl_d[l] + 16) / 16, tiles = T * (T + 1) / 2;
+      const auto split = [&](int waves) { return std::max(1, std::min((tiles + waves - 1) / waves, 1024 / n)); };
+      // sixteen wavefronts for the pivots' latency, four where fronts
+      // outnumber half the CUs: levels of 207 to 1,166 fronts 28-45 -> 20-26 us
+      if (n > 128) k_front<256><<<dim3(n, split(4)), 256, lds, st>>>(RPGO_FRONT_ARGS);
+      else k_front<1024><<<dim3(n, split(16)), 1024, lds, st>>>(RPGO_FRONT_ARGS);
     }
 #undef RPGO_FRONT_ARGS
   }
@@ -479,17 +755,13 @@ int SolverRun::direct_factor(hipStream_t st, double lambda) {
 
 int SolverRun::direct_backward(hipStream_t st, double* out) {
   const DirectPlan& P = plan;
-  // levels of at most kTop fronts from the top down in one workgroup
-  constexpr int kTop = 48;
-  int l0 = P.levels();
-  while (l0 > 0 && P.lvl[l0] - P.lvl[l0 - 1] <= kTop) --l0;
-  if (l0 < P.levels())
-    k_back_top<<<1, 1024, 0, st>>>(l0, P.levels(), d_lvl.as<int>(), d_meta.as<FrontMeta>(), d_nb.as<int>(),
-                                   d_G.as<double>(), d_L.as<double>(), d_Y.as<double>(), out);
-  for (int l = l0 - 1; l >= 0; --l) {
+  for (int l = P.levels() - 1; l >= 0; --l) {
     const int first = P.lvl[l], n = P.lvl[l + 1] - first;
-    k_back_level<<<(n + 3) / 4, 256, 0, st>>>(first, n, d_meta.as<FrontMeta>(), d_nb.as<int>(), d_G.as<double>(),
-                                              d_L.as<double>(), d_Y.as<double>(), out);
+    const size_t lds = (size_t)P.lvl_back[l];
+    if (small_level(P, l))
+      k_back<64><<<n, 64, lds, st>>>(first, d_meta.as<FrontMeta>(), d_rows.as<int>(), d_G.as<double>(), out);
+    else
+      k_back<256><<<n, 256, lds, st>>>(first, d_meta.as<FrontMeta>(), d_rows.as<int>(), d_G.as<double>(), out);
   }
   RPGO_HIP_CHECK(hipGetLastError());
   return RPGO_OK;
@@ -510,9 +782,13 @@ int SolverRun::direct_refine(hipStream_t st) {
   const DirectPlan& P = plan;
   for (int l = 0; l < P.levels(); ++l) {
     const int first = P.lvl[l], n = P.lvl[l + 1] - first;
-    k_front_forward<<<n, 64, 0, st>>>(first, d_meta.as<FrontMeta>(), d_childs.as<FrontChild>(), d_maps.as<int>(),
-                                      r.as<double>(), d_G.as<double>(), d_L.as<double>(), d_U.as<double>(),
-                                      d_Y.as<double>());
+    const size_t lds = (size_t)P.lvl_bytes[l];
+#define RPGO_FORWARD_ARGS                                                                                     \
+  first, d_meta.as<FrontMeta>(), d_childs.as<FrontChild>(), d_maps.as<int>(), d_rows.as<int>(), r.as<double>(), \
+      d_G.as<double>(), d_U.as<double>()
+    if (small_level(P, l)) k_front_forward<64><<<n, 64, lds, st>>>(RPGO_FORWARD_ARGS);
+    else k_front_forward<256><<<n, 256, lds, st>>>(RPGO_FORWARD_ARGS);
+#undef RPGO_FORWARD_ARGS
   }
   int rc;
   if ((rc = direct_backward(st, zv.as<double>()))) return rc;

@@ -16,6 +16,13 @@
 // blocks, against 83 levels and 445,827 blocks with the relaxed threshold.
 // The numeric work is small either way (0.4 M 6x6 products); the number of
 // dependent levels is what a GPU pays for.
+//
+// A run of poses, each the parent of the one before and with one neighbour
+// less (the end of the elimination: a clique loses a pose at a time), is one
+// front with several pivots: its columns are the same rows, so one workgroup
+// eliminates them from one copy in LDS.  The levels of the fronts are the
+// heights of the merged tree: 69 -> 20 at 3,000 poses with 601 loop closures,
+// 97 -> 23 at 50,000 with 5,000, 22 -> 14 for 500 planar poses.
 #pragma once
 
 #include <algorithm>
@@ -24,47 +31,66 @@
 
 namespace rpgo {
 
-// One eliminated pose.  Its front is the pose itself (position 0) and its d
-// remaining neighbours (positions 1 .. d, in elimination order).
+// One front: s pivots and their n - s remaining neighbours, n rows of 6x6
+// blocks in elimination order.  Column q of its panel holds rows q .. n-1 and
+// the right-hand side as one more row of six.
 struct FrontMeta {
-  int32_t pose;
-  int32_t d;
-  int32_t nb_off;      // neighbours in nb_pose; its G blocks start at 36 * nb_off
-  int32_t child_off;   // children: fronts whose first neighbour is this pose
+  int32_t s, n;
+  int32_t row_off;     // rows as poses in row_pose, pivots first
+  int32_t child_off;   // children: fronts whose first neighbour is a pivot here
   int32_t n_child;
+  int32_t map_off;     // child c's map at map_off + c * n
   int32_t orig_off;    // between factors assembled here
   int32_t n_orig;
-  int32_t pad;
+  int64_t g_off;       // factored panel, in doubles
   int64_t u_off;       // update matrix and vector, in doubles
 };
 
-// A child's update matrix and the map from this front's positions to the
-// child's neighbour indices (-1: not a neighbour of the child)
+// A child's update matrix; its map gives, per row here, the child's neighbour
+// index (-1: not a neighbour of the child)
 struct FrontChild {
   int64_t u_off;
-  int32_t map_off;
   int32_t d;
+  int32_t pad;
 };
 
-// factor f, its block's position in the front and whether its Hij is the
-// transpose of the block (neighbour rows, pivot columns)
+// factor f, its block (column q, row r) and whether its Hij is the transpose
+// of the block (row pose first, pivot second).  run: the number of factors of
+// the block at its first one, 0 at the others.
 struct FrontOrig {
   int32_t f;
-  int32_t slot_t;  // 2 * position + transposed
+  int32_t slot;  // q << 16 | r << 1 | transposed
+  int32_t run;
+  int32_t pad;
 };
 
 inline int64_t front_update_len(int64_t d) { return d * (d + 1) / 2 * 36 + 6 * d; }
+// first panel row (of six doubles) of column q of a front of n rows; at q = s
+// the rows of the whole panel
+#ifdef __HIPCC__
+__host__ __device__
+#endif
+constexpr int panel_row(int n, int q) { return 6 * (q * n - q * (q - 1) / 2) + q; }
+// LDS of a front's panel and one more vector of its rows; a front takes
+// pivots up to kPanelBytes
+constexpr int panel_bytes(int n, int s) { return 48 * (panel_row(n, s) + n); }
+constexpr int kPanelBytes = 64 * 1024;
+// LDS of the backward substitution: the pivots' triangle and one vector of
+// the rows
+constexpr int back_bytes(int n, int s) { return 8 * (18 * s * (s + 1) + 6 * n); }
 
 struct DirectPlan {
   int N = 0;
-  int max_d = 0;
-  int64_t u_len = 0;                // doubles of all update matrices
+  int max_d = 0;                    // neighbours of the widest pivot
+  int64_t u_len = 0, g_len = 0;     // doubles of all update matrices and panels
   std::vector<int> lvl;             // level offsets into meta
-  std::vector<int> lvl_max_d;       // largest front of each level
-  std::vector<FrontMeta> meta;      // in elimination order
+  std::vector<int> lvl_bytes;       // largest panel_bytes of each level
+  std::vector<int> lvl_back;        // largest back_bytes
+  std::vector<int> lvl_s, lvl_n, lvl_d;  // most pivots, rows, neighbours of a front
+  std::vector<FrontMeta> meta;      // by level
   std::vector<FrontChild> childs;
   std::vector<FrontOrig> origs;
-  std::vector<int32_t> nb_pose;     // neighbours as poses
+  std::vector<int32_t> row_pose;
   std::vector<int32_t> maps;
   int levels() const { return (int)lvl.size() - 1; }
 };
@@ -149,7 +175,6 @@ inline bool build_direct_plan(int N, int F, const int32_t* kind, const int32_t* 
   std::vector<int32_t> bucket_off, cand;
   int64_t steps = 0, u_len = 0;
   const int64_t max_u = std::min(lim.max_u, std::max(lim.u_free, lim.max_u_pose * N));
-  P.lvl.push_back(0);
   for (int level = 0; !alive.empty(); ++level) {
     int dmin = A.len[alive[0]];
     for (int v : alive) dmin = std::min(dmin, (int)A.len[v]);
@@ -204,103 +229,163 @@ inline bool build_direct_plan(int N, int F, const int32_t* kind, const int32_t* 
       }
     }
     P.max_d = std::max(P.max_d, level_max);
-    P.lvl_max_d.push_back(level_max);
-    P.lvl.push_back((int)order.size());
     size_t keep = 0;
     for (int v : alive)
       if (elim[v] < 0) alive[keep++] = v;
     alive.resize(keep);
   }
-  P.u_len = u_len;
-  // elimination positions; fronts
+  // neighbours as elimination positions, ascending; parents
   std::vector<int32_t>& pos = mark;
   for (int p = 0; p < N; ++p) pos[order[p]] = p;
-  P.meta.resize(N);
-  int64_t nb_total = 0, uo = 0;
-  for (int v = 0; v < N; ++v) nb_total += A.len[v];
-  if (nb_total > INT32_MAX / 36) return false;
-  P.nb_pose.resize(nb_total);
-  std::vector<int32_t> nb(nb_total);  // neighbours as positions, ascending
-  int32_t no = 0;
+  std::vector<int64_t> nb_off(N + 1, 0);
+  for (int p = 0; p < N; ++p) nb_off[p + 1] = nb_off[p] + A.len[order[p]];
+  if (nb_off[N] + N > INT32_MAX / 36) return false;
+  std::vector<int32_t> nb(nb_off[N]), par(N, -1);
   for (int p = 0; p < N; ++p) {
-    const int v = order[p], d = A.len[v];
-    FrontMeta& m = P.meta[p];
-    m = FrontMeta{};
-    m.pose = v;
-    m.d = d;
-    m.nb_off = no;
-    m.u_off = uo;
-    for (int k = 0; k < d; ++k) nb[no + k] = pos[A.at(v)[k]];
-    std::sort(nb.begin() + no, nb.begin() + no + d);
-    for (int k = 0; k < d; ++k) P.nb_pose[no + k] = order[nb[no + k]];
-    no += d;
-    uo += front_update_len(d);
+    const int32_t* a = A.at(order[p]);
+    int32_t* o = nb.data() + nb_off[p];
+    const int d = A.len[order[p]];
+    for (int k = 0; k < d; ++k) o[k] = pos[a[k]];
+    if (d > 2) std::sort(o, o + d);
+    else if (d == 2 && o[0] > o[1]) std::swap(o[0], o[1]);
+    if (d > 0) par[p] = o[0];
   }
-  // children (a front's parent is its first neighbour) and position maps
-  for (int p = 0; p < N; ++p)
-    if (P.meta[p].d > 0) ++P.meta[nb[P.meta[p].nb_off]].n_child;
-  int32_t co = 0;
-  int64_t mo = 0;
+  const auto deg = [&](int p) { return (int)(nb_off[p + 1] - nb_off[p]); };
+  // fronts: a pose joins its child with one neighbour more (the rows are then
+  // the same), the one that ends the longest run
+  std::vector<int32_t> best(N, -1), run(N, 1), next(N, -1), sn(N, -1), idx(N, 0), first_of;
   for (int p = 0; p < N; ++p) {
-    P.meta[p].child_off = co;
-    co += P.meta[p].n_child;
-    mo += (int64_t)P.meta[p].n_child * (P.meta[p].d + 1);
-    P.meta[p].n_child = 0;
+    if (best[p] >= 0) {
+      run[p] += run[best[p]];
+      next[best[p]] = p;
+    }
+    const int q = par[p];
+    if (q >= 0 && deg(p) == deg(q) + 1 && (best[q] < 0 || run[p] > run[best[q]])) best[q] = p;
   }
-  if (mo > lim.max_maps) return false;
-  P.childs.resize(co);
-  P.maps.resize(mo);
-  int32_t map_off = 0;
-  std::vector<int32_t> map_base(N);
+  for (int p = 0; p < N; ++p) {
+    if (best[p] >= 0) continue;  // not the start of a run
+    for (int q = p; q >= 0;) {
+      const int n = deg(q) + 1, id = (int)first_of.size();
+      first_of.push_back(q);
+      int s = 0;
+      do {
+        sn[q] = id;
+        idx[q] = s++;
+        q = next[q];
+      } while (q >= 0 && panel_bytes(n, s + 1) <= kPanelBytes);
+    }
+  }
+  const int M = (int)first_of.size();
+  std::vector<int32_t> size(M, 0), last(M, 0), height(M, 0), at(M), n_orig(M, 0), n_child(M, 0);
+  for (int p = 0; p < N; ++p) {
+    ++size[sn[p]];
+    last[sn[p]] = p;
+  }
+  int levels = 0;
+  for (int p = 0; p < N; ++p) {  // a front's children end before its own last pivot
+    const int g = sn[p];
+    if (p != last[g]) continue;
+    levels = std::max(levels, height[g] + 1);
+    if (par[p] >= 0) {
+      const int q = sn[par[p]];
+      height[q] = std::max(height[q], height[g] + 1);
+      ++n_child[q];
+    }
+  }
+  for (int f = 0; f < F; ++f)
+    if (kind[f] == 0) ++n_orig[sn[std::min(pos[fi[f]], pos[fj[f]])]];
+  P.lvl.assign(levels + 1, 0);
+  P.lvl_bytes.assign(levels, 0);
+  P.lvl_back.assign(levels, 0);
+  P.lvl_s.assign(levels, 0);
+  P.lvl_n.assign(levels, 0);
+  P.lvl_d.assign(levels, 0);
+  for (int g = 0; g < M; ++g) ++P.lvl[height[g] + 1];
+  for (int l = 0; l < levels; ++l) P.lvl[l + 1] += P.lvl[l];
   {
-    int64_t m = 0;
-    std::vector<int32_t> cnt(N, 0);
-    for (int p = 0; p < N; ++p)
-      if (P.meta[p].d > 0) ++cnt[nb[P.meta[p].nb_off]];
-    for (int p = 0; p < N; ++p) {
-      map_base[p] = (int32_t)m;
-      m += (int64_t)cnt[p] * (P.meta[p].d + 1);
-    }
+    std::vector<int> o(P.lvl.begin(), P.lvl.end() - 1);
+    for (int g = 0; g < M; ++g) at[g] = o[height[g]]++;
   }
-  (void)map_off;
-  for (int c = 0; c < N; ++c) {  // ascending: a front's children in elimination order
-    const FrontMeta& cm = P.meta[c];
-    if (cm.d == 0) continue;
-    const int p = nb[cm.nb_off];
-    FrontMeta& m = P.meta[p];
-    FrontChild& ch = P.childs[m.child_off + m.n_child];
-    ch.u_off = cm.u_off;
-    ch.d = cm.d;
-    ch.map_off = map_base[p] + m.n_child * (m.d + 1);
-    ++m.n_child;
-    int32_t* map = P.maps.data() + ch.map_off;
-    map[0] = 0;
-    int j = 1;  // child neighbours past the parent itself, a subset of the parent's
-    for (int k = 1; k <= m.d; ++k) {
-      const bool hit = j < cm.d && nb[cm.nb_off + j] == nb[m.nb_off + k - 1];
-      map[k] = hit ? j++ : -1;
+  P.meta.resize(M);
+  for (int g = 0; g < M; ++g) {
+    FrontMeta& m = P.meta[at[g]];
+    m = FrontMeta{};
+    m.s = size[g];
+    m.n = deg(first_of[g]) + 1;
+    m.n_child = n_child[g];
+    m.n_orig = n_orig[g];
+    m.row_off = first_of[g];  // replaced below
+  }
+  int64_t rows = 0, maps = 0, childs = 0, origs = 0;
+  for (int g = 0, l = 0; g < M; ++g) {
+    FrontMeta& m = P.meta[g];
+    while (g >= P.lvl[l + 1]) ++l;
+    const int p = m.row_off, d = m.n - m.s;
+    m.row_off = (int32_t)rows;
+    m.child_off = (int32_t)childs;
+    m.map_off = (int32_t)maps;
+    m.orig_off = (int32_t)origs;
+    m.g_off = P.g_len;
+    m.u_off = P.u_len;
+    rows += m.n;
+    maps += (int64_t)m.n_child * m.n;
+    childs += m.n_child;
+    origs += m.n_orig;
+    P.g_len += 6ll * panel_row(m.n, m.s);
+    P.u_len += front_update_len(d);
+    if (maps > lim.max_maps) return false;
+    P.lvl_bytes[l] = std::max(P.lvl_bytes[l], panel_bytes(m.n, m.s));
+    P.lvl_back[l] = std::max(P.lvl_back[l], back_bytes(m.n, m.s));
+    P.lvl_d[l] = std::max(P.lvl_d[l], d);
+    P.lvl_s[l] = std::max(P.lvl_s[l], m.s);
+    P.lvl_n[l] = std::max(P.lvl_n[l], m.n);
+    P.row_pose.push_back(order[p]);
+    for (int64_t k = nb_off[p]; k < nb_off[p + 1]; ++k) P.row_pose.push_back(order[nb[k]]);
+  }
+  // children and row maps (in the order of the children's first pivots)
+  P.childs.resize(childs);
+  P.maps.resize(maps);
+  std::vector<int32_t>& fill = n_child;
+  std::fill(fill.begin(), fill.end(), 0);
+  for (int g = 0; g < M; ++g) {
+    const int c = last[g], dc = deg(c);
+    if (dc == 0) continue;
+    const int q = sn[par[c]];
+    const FrontMeta& m = P.meta[at[q]];
+    const int k = fill[q]++;
+    P.childs[m.child_off + k] = FrontChild{P.meta[at[g]].u_off, dc, 0};
+    int32_t* map = P.maps.data() + m.map_off + (int64_t)k * m.n;
+    const int32_t *x = nb.data() + nb_off[c], *y = nb.data() + nb_off[first_of[q]];
+    int j = 0;  // the child's neighbours are a subset of the rows
+    for (int r = 0; r < m.n; ++r) {
+      const int row = r == 0 ? first_of[q] : y[r - 1];
+      map[r] = j < dc && x[j] == row ? j++ : -1;
     }
-    if (j != cm.d) return false;  // not reached: fill makes the child's rest a subset
+    if (j != dc) return false;  // not reached: fill makes them one
   }
   // between factors, assembled at the endpoint eliminated first
-  for (int f = 0; f < F; ++f)
-    if (kind[f] == 0) ++P.meta[std::min(pos[fi[f]], pos[fj[f]])].n_orig;
-  int32_t oo = 0;
-  for (int p = 0; p < N; ++p) {
-    P.meta[p].orig_off = oo;
-    oo += P.meta[p].n_orig;
-    P.meta[p].n_orig = 0;
-  }
-  P.origs.resize(oo);
+  P.origs.resize(origs);
+  std::fill(n_orig.begin(), n_orig.end(), 0);
   for (int f = 0; f < F; ++f) {
     if (kind[f] != 0) continue;
-    const int a = pos[fi[f]], b = pos[fj[f]];
-    FrontMeta& m = P.meta[std::min(a, b)];
-    const int32_t* s = nb.data() + m.nb_off;
-    const int slot = (int)(std::lower_bound(s, s + m.d, std::max(a, b)) - s) + 1;
-    // the block has neighbour rows and pivot columns: Hij (rows i, columns j)
+    const int a = pos[fi[f]], b = pos[fj[f]], lo = std::min(a, b), hi = std::max(a, b), g = sn[lo];
+    const int32_t *y = nb.data() + nb_off[first_of[g]], *e = nb.data() + nb_off[first_of[g] + 1];
+    const int r = sn[hi] == g ? idx[hi] : (int)(std::lower_bound(y, e, hi) - y) + 1;
+    // the block has row-pose rows and pivot columns: Hij (rows i, columns j)
     // is its transpose when the pivot is key i
-    P.origs[m.orig_off + m.n_orig++] = FrontOrig{f, 2 * slot + (a < b ? 1 : 0)};
+    P.origs[P.meta[at[g]].orig_off + n_orig[g]++] = FrontOrig{f, idx[lo] << 16 | r << 1 | (a < b ? 1 : 0), 1, 0};
+  }
+  for (int g = 0; g < M; ++g) {
+    const FrontMeta& m = P.meta[g];
+    if (m.n_orig < 2) continue;
+    FrontOrig* o = P.origs.data() + m.orig_off;
+    std::sort(o, o + m.n_orig, [](const FrontOrig& a, const FrontOrig& b) {
+      return (a.slot >> 1) != (b.slot >> 1) ? (a.slot >> 1) < (b.slot >> 1) : a.f < b.f;
+    });
+    for (int i = 0, j; i < m.n_orig; i = j) {
+      for (j = i + 1; j < m.n_orig && (o[j].slot >> 1) == (o[i].slot >> 1); ++j) o[j].run = 0;
+      o[i].run = j - i;
+    }
   }
   return true;
 }

@@ -77,8 +77,8 @@ struct SolverRun {
   bool direct_ready = false;
   DirectPlan plan;
   double last_residual = 0.0;      // relative residual of the last direct solve
-  DevBuf d_meta, d_childs, d_origs, d_nb, d_maps, d_lvl;
-  DevBuf d_U, d_G, d_L, d_Y, d_part, d_bad;
+  DevBuf d_meta, d_childs, d_origs, d_rows, d_maps;
+  DevBuf d_U, d_G, d_part, d_bad;
   // pinned host buffers of this run's readbacks (scalars; one PCG chunk's
   // residual history), allocated on first use
   double* h_scalars = nullptr;
@@ -122,8 +122,8 @@ struct SolverRun {
                       &Hjj, &Hij, &gi, &gj, &inc_off, &inc_cnt, &inc, &inc_q, &D, &Minv, &hdiag, &b64,
                       &chain, &Useg, &Ds, &Cs, &ext_off, &ext, &ext_q, &Pb, &Ac, &Lci, &LcT, &Ainv, &cres,
                       &ccor,
-                      &dx, &r, &zv, &p, &q, &hx, &sc, &d_meta, &d_childs, &d_origs, &d_nb, &d_maps, &d_lvl,
-                      &d_U, &d_G, &d_L, &d_Y, &d_part, &d_bad})
+                      &dx, &r, &zv, &p, &q, &hx, &sc, &d_meta, &d_childs, &d_origs, &d_rows, &d_maps,
+                      &d_U, &d_G, &d_part, &d_bad})
       v->release();
   }
 };

@@ -90,90 +90,75 @@ std::vector<double> dense_solve(const Sys& s) {
 
 // The plan's factorization and both substitutions, front by front
 std::vector<double> plan_solve(const Sys& s, const DirectPlan& P, int& bad) {
-  std::vector<double> U(P.u_len, 0.0), G(36 * P.nb_pose.size(), 0.0), L(36 * (size_t)s.N, 0.0), y(6 * (size_t)s.N),
-      x(6 * (size_t)s.N, 0.0);
-  for (int p = 0; p < s.N; ++p) {
-    const FrontMeta& m = P.meta.at(p);
-    const int d = m.d;
-    std::vector<double> row(36 * (size_t)(d + 1), 0.0), f(6 * (size_t)(d + 1), 0.0), S((size_t)front_update_len(d), 0.0);
-    for (int q = 0; q < 36; ++q) row[q] = s.D.at(m.pose)[q];
-    for (int i = 0; i < 6; ++i) f[i] = s.b[6 * m.pose + i];
+  std::vector<double> U(P.u_len, 0.0), G(P.g_len, 0.0), x(6 * (size_t)s.N, 0.0);
+  for (size_t g = 0; g < P.meta.size(); ++g) {
+    const FrontMeta& m = P.meta[g];
+    const int n = m.n, np = m.s, d = n - np;
+    // dense front: n + 1 block rows (the last, one row, the right-hand side)
+    const int w = 6 * n;
+    std::vector<double> A((size_t)(w + 1) * w, 0.0);
+    for (int q = 0; q < np; ++q) {
+      const int pose = P.row_pose.at(m.row_off + q);
+      for (int e = 0; e < 36; ++e) A[(size_t)(6 * q + e / 6) * w + 6 * q + e % 6] += s.D.at(pose)[e];
+      for (int i = 0; i < 6; ++i) A[(size_t)w * w + 6 * q + i] += s.b[6 * pose + i];
+    }
     for (int o = 0; o < m.n_orig; ++o) {
-      const FrontOrig& a = P.origs.at(m.orig_off + o);
-      const int slot = a.slot_t >> 1;
-      if (slot < 1 || slot > d) { ++bad; continue; }
-      for (int i = 0; i < 6; ++i)
-        for (int j = 0; j < 6; ++j) row[36 * slot + i * 6 + j] += s.H.at(a.f)[(a.slot_t & 1) ? j * 6 + i : i * 6 + j];
+      const FrontOrig& lead = P.origs.at(m.orig_off + o);
+      for (int k = 0; k < lead.run; ++k) {
+        const FrontOrig& a = P.origs.at(m.orig_off + o + k);
+        const int q = a.slot >> 16, R = (a.slot >> 1) & 0x7fff;
+        if ((a.slot >> 1) != (lead.slot >> 1) || q >= np || R <= q || R >= n || (k > 0 && a.run != 0)) { ++bad; continue; }
+        const int row = P.row_pose.at(m.row_off + R), piv = P.row_pose.at(m.row_off + q);
+        if ((a.slot & 1) ? (s.fi.at(a.f) != piv || s.fj.at(a.f) != row) : (s.fi.at(a.f) != row || s.fj.at(a.f) != piv)) ++bad;
+        for (int e = 0; e < 36; ++e)
+          A[(size_t)(6 * R + e / 6) * w + 6 * q + e % 6] += s.H.at(a.f)[(a.slot & 1) ? (e % 6) * 6 + e / 6 : e];
+      }
+      if (lead.run > 0 && o + lead.run < m.n_orig && P.origs.at(m.orig_off + o + lead.run).run == 0) ++bad;
     }
     for (int c = 0; c < m.n_child; ++c) {
       const FrontChild& ch = P.childs.at(m.child_off + c);
-      for (int k = 0; k <= d; ++k) {
-        const int pk = P.maps.at(ch.map_off + k);
+      const int64_t vec = ch.u_off + (int64_t)ch.d * (ch.d + 1) / 2 * 36;
+      for (int k = 0; k < n; ++k) {
+        const int pk = P.maps.at(m.map_off + c * n + k);
         if (pk < 0) continue;
-        if (pk >= ch.d || (k == 0) != (pk == 0)) { ++bad; continue; }
-        const int64_t uc = ch.u_off + (int64_t)ch.d * (ch.d + 1) / 2 * 36 + 6 * pk;
-        for (int i = 0; i < 6; ++i) f[6 * k + i] += U.at(uc + i);
+        if (pk >= ch.d) { ++bad; continue; }
+        for (int i = 0; i < 6; ++i) A[(size_t)w * w + 6 * k + i] += U.at(vec + 6 * pk + i);
         for (int l = 0; l <= k; ++l) {
-          const int pl = P.maps.at(ch.map_off + l);
+          const int pl = P.maps.at(m.map_off + c * n + l);
           if (pl < 0) continue;
           if (pl > pk) { ++bad; continue; }
-          for (int q = 0; q < 36; ++q) {
-            const double v = U.at(ch.u_off + 36 * ((int64_t)pk * (pk + 1) / 2 + pl) + q);
-            if (l == 0) row[36 * k + q] += v;
-            else S[36 * ((int64_t)(k - 1) * k / 2 + l - 1) + q] += v;
-          }
+          for (int e = 0; e < 36; ++e)
+            A[(size_t)(6 * k + e / 6) * w + 6 * l + e % 6] += U.at(ch.u_off + 36 * ((int64_t)pk * (pk + 1) / 2 + pl) + e);
         }
       }
     }
-    double* Lp = &L[36 * (size_t)p];
-    for (int c = 0; c < 6; ++c)
-      for (int r = c; r < 6; ++r) {
-        double v = row[r * 6 + c];
-        for (int k = 0; k < c; ++k) v -= Lp[r * 6 + k] * Lp[c * 6 + k];
-        Lp[r * 6 + c] = r == c ? std::sqrt(v) : v / Lp[c * 7];
-      }
-    auto sub = [&](double* g) {  // g L^-T, a row of six
-      for (int j = 0; j < 6; ++j) {
-        for (int k = 0; k < j; ++k) g[j] -= g[k] * Lp[j * 6 + k];
-        g[j] /= Lp[j * 7];
-      }
-    };
-    sub(f.data());
-    for (int i = 0; i < 6; ++i) y[6 * p + i] = f[i];
-    double* Gp = d ? &G.at(36 * (size_t)m.nb_off) : nullptr;
-    for (int k = 1; k <= d; ++k)
-      for (int i = 0; i < 6; ++i) {
-        sub(&row[36 * k + 6 * i]);
-        for (int j = 0; j < 6; ++j) Gp[36 * (k - 1) + 6 * i + j] = row[36 * k + 6 * i + j];
-      }
+    // eliminate the pivots' columns from the lower triangle and the last row
+    for (int c = 0; c < 6 * np; ++c) {
+      const double p = std::sqrt(A[(size_t)c * w + c]);
+      for (int r = c; r <= w; ++r) A[(size_t)r * w + c] /= p;
+      for (int c2 = c + 1; c2 < w; ++c2)
+        for (int r = c2; r <= w; ++r) A[(size_t)r * w + c2] -= A[(size_t)r * w + c] * A[(size_t)c2 * w + c];
+    }
+    for (int q = 0; q < np; ++q)
+      for (int r = 6 * q; r <= w; ++r)
+        for (int j = 0; j < 6; ++j) G.at(m.g_off + 6 * (panel_row(n, q) + r - 6 * q) + j) = A[(size_t)r * w + 6 * q + j];
     for (int k = 0; k < d; ++k) {
       for (int l = 0; l <= k; ++l)
-        for (int i = 0; i < 6; ++i)
-          for (int j = 0; j < 6; ++j) {
-            double v = S[36 * ((int64_t)k * (k + 1) / 2 + l) + 6 * i + j];
-            for (int q = 0; q < 6; ++q) v -= Gp[36 * k + 6 * i + q] * Gp[36 * l + 6 * j + q];
-            U.at(m.u_off + 36 * ((int64_t)k * (k + 1) / 2 + l) + 6 * i + j) = v;
-          }
-      for (int i = 0; i < 6; ++i) {
-        double v = f[6 * (k + 1) + i];
-        for (int q = 0; q < 6; ++q) v -= Gp[36 * k + 6 * i + q] * f[q];
-        U.at(m.u_off + 36 * ((int64_t)d * (d + 1) / 2) + 6 * k + i) = v;
-      }
+        for (int e = 0; e < 36; ++e)
+          U.at(m.u_off + 36 * ((int64_t)k * (k + 1) / 2 + l) + e) = A[(size_t)(6 * (np + k) + e / 6) * w + 6 * (np + l) + e % 6];
+      for (int i = 0; i < 6; ++i) U.at(m.u_off + 36 * ((int64_t)d * (d + 1) / 2) + 6 * k + i) = A[(size_t)w * w + 6 * (np + k) + i];
     }
   }
-  for (int p = s.N - 1; p >= 0; --p) {
-    const FrontMeta& m = P.meta[p];
-    double r[6];
-    for (int j = 0; j < 6; ++j) {
-      r[j] = y[6 * p + j];
-      for (int k = 0; k < m.d; ++k)
-        for (int i = 0; i < 6; ++i) r[j] -= G[36 * (size_t)(m.nb_off + k) + 6 * i + j] * x[6 * P.nb_pose.at(m.nb_off + k) + i];
+  for (size_t g = P.meta.size(); g-- > 0;) {
+    const FrontMeta& m = P.meta[g];
+    const int n = m.n;
+    for (int c = 6 * m.s - 1; c >= 0; --c) {
+      const int q = c / 6, j = c % 6;
+      const auto at = [&](int r) { return G.at(m.g_off + 6 * (panel_row(n, q) + r - 6 * q) + j); };
+      double v = at(6 * n);
+      for (int r = c + 1; r < 6 * n; ++r) v -= at(r) * x.at(6 * P.row_pose.at(m.row_off + r / 6) + r % 6);
+      x[6 * P.row_pose[m.row_off + q] + j] = v / at(c);
     }
-    for (int j = 5; j >= 0; --j) {
-      for (int k = j + 1; k < 6; ++k) r[j] -= L[36 * (size_t)p + k * 6 + j] * r[k];
-      r[j] /= L[36 * (size_t)p + j * 7];
-    }
-    for (int j = 0; j < 6; ++j) x[6 * m.pose + j] = r[j];
   }
   return x;
 }
@@ -182,18 +167,28 @@ int check(const char* what, int N, const std::vector<std::pair<int, int>>& edges
   const Sys s = random_system(N, edges, seed);
   DirectPlan P;
   EXPECT(build_direct_plan(N, (int)s.kind.size(), s.kind.data(), s.fi.data(), s.fj.data(), DirectLimits(), P));
-  // every pose once, levels contiguous, no two poses of a level adjacent
-  std::vector<int> level(N, -1);
+  // every pose a pivot once, levels contiguous, no factor between two fronts
+  // of a level, every front within the level's bounds and the LDS
+  std::vector<int> level(N, -1), front(N, -1);
   int seen = 0;
   for (int l = 0; l < P.levels(); ++l)
     for (int p = P.lvl[l]; p < P.lvl[l + 1]; ++p) {
-      EXPECT(level.at(P.meta[p].pose) < 0);
-      level[P.meta[p].pose] = l;
-      EXPECT(P.meta[p].d <= P.lvl_max_d[l]);
-      ++seen;
+      const FrontMeta& m = P.meta.at(p);
+      EXPECT(m.s >= 1 && m.s <= m.n && m.s <= P.lvl_s[l] && m.n <= P.lvl_n[l] && m.n - m.s <= P.lvl_d[l]);
+      EXPECT(panel_bytes(m.n, m.s) <= P.lvl_bytes[l] && P.lvl_bytes[l] <= kPanelBytes);
+      // with 2 KB of its own the backward kernel keeps within the LDS too; a
+      // thread per pivot component
+      EXPECT(back_bytes(m.n, m.s) <= P.lvl_back[l] && P.lvl_back[l] + 2048 <= kPanelBytes && 6 * m.s <= 256);
+      for (int q = 0; q < m.s; ++q) {
+        const int pose = P.row_pose.at(m.row_off + q);
+        EXPECT(level.at(pose) < 0);
+        level[pose] = l;
+        front[pose] = p;
+        ++seen;
+      }
     }
-  EXPECT(seen == N && P.lvl.back() == N);
-  for (auto& e : edges) EXPECT(level[e.first] != level[e.second]);
+  EXPECT(seen == N && P.lvl.back() == (int)P.meta.size());
+  for (auto& e : edges) EXPECT(level[e.first] != level[e.second] || front[e.first] == front[e.second]);
   int bad = 0;
   const auto x = plan_solve(s, P, bad), ref = dense_solve(s);
   EXPECT(bad == 0);
@@ -254,6 +249,9 @@ TEST(DirectPlan, Shapes) {
   two.push_back({5, 17});
   check("star", 60, star, 1, rpgo_failures_);
   check("clique", 20, clique, 2, rpgo_failures_);
+  for (int a = 20; a < 45; ++a)  // too wide for one panel
+    for (int b = 0; b < a; ++b) clique.push_back({b, a});
+  EXPECT(check("clique", 45, clique, 6, rpgo_failures_) > 1);
   check("two chains", 41, two, 3, rpgo_failures_);
   check("no factors", 5, none, 4, rpgo_failures_);
   auto ladder = chain(120);  // laps of 12 poses, joined at every third pose
@@ -272,7 +270,8 @@ TEST(DirectPlan, Limits) {
   EXPECT(!build_direct_plan(20, (int)s.kind.size(), s.kind.data(), s.fi.data(), s.fj.data(), lim, P));
   lim.max_d = 19;
   EXPECT(build_direct_plan(20, (int)s.kind.size(), s.kind.data(), s.fi.data(), s.fj.data(), lim, P));
-  lim.max_u = P.u_len - 1;
+  lim.max_u = -1;  // the limit counts every pivot's update by itself
+  for (int d = 0; d < 20; ++d) lim.max_u += front_update_len(d);
   EXPECT(!build_direct_plan(20, (int)s.kind.size(), s.kind.data(), s.fi.data(), s.fj.data(), lim, P));
 }
 

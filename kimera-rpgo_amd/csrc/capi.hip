@@ -110,6 +110,7 @@ int rpgo_ctx_destroy(rpgo_ctx* ctx) {
   mlp_destroy(ctx);
   batch_destroy(ctx);
   if (ctx->host_pinned) (void)hipHostFree(ctx->host_pinned);
+  if (ctx->append_stage) (void)hipHostFree(ctx->append_stage);
   for (auto& ev : ctx->ev)
     if (ev) (void)hipEventDestroy(ev);
   (void)hipStreamDestroy(ctx->stream);
@@ -512,30 +513,34 @@ int pcm_append_impl(rpgo_ctx* ctx, const rpgo_pcm_increment* inc, double odom_th
   if ((rc = s.lc_pose.grow_keep(8 * PL * L1, 8 * PL * L0, st))) return rc;
   if ((rc = s.lc_cov.grow_keep(8 * DD * L1, 8 * DD * L0, st))) return rc;
   if ((rc = s.lcm.grow_keep(8 * PWC * L1, 8 * PWC * L0, st))) return rc;
-  if (inc->n_odom > 0) {
-    RPGO_HIP_CHECK(hipMemcpyAsync(s.odom.as<double>() + PL * d0, inc->odom, 8 * PL * inc->n_odom,
-                                  hipMemcpyHostToDevice, st));
-    RPGO_HIP_CHECK(hipMemcpyAsync(s.odom_cov.as<double>() + DD * d0, inc->odom_cov, 8 * DD * inc->n_odom,
-                                  hipMemcpyHostToDevice, st));
-  }
-  if (inc->n_lc > 0) {
-    RPGO_HIP_CHECK(hipMemcpyAsync(s.lc_from.as<int>() + L0, inc->lc_from, 4 * (size_t)inc->n_lc,
-                                  hipMemcpyHostToDevice, st));
-    RPGO_HIP_CHECK(hipMemcpyAsync(s.lc_to.as<int>() + L0, inc->lc_to, 4 * (size_t)inc->n_lc,
-                                  hipMemcpyHostToDevice, st));
-    RPGO_HIP_CHECK(hipMemcpyAsync(s.lc_pose.as<double>() + PL * L0, inc->lc_pose, 8 * PL * inc->n_lc,
-                                  hipMemcpyHostToDevice, st));
-    RPGO_HIP_CHECK(hipMemcpyAsync(s.lc_cov.as<double>() + DD * L0, inc->lc_cov, 8 * DD * inc->n_lc,
-                                  hipMemcpyHostToDevice, st));
-  }
   s.n_poses = n1;
   s.n_lc = l1;
   s.fp32_ready = false;
   s.fp32_fallback = false;
   s.have_dist = false;
-  RPGO_HIP_CHECK(hipMemsetAsync(s.counters.ptr, 0, 256, st));
   RPGO_HIP_CHECK(hipEventRecord(ev[0], st));
-  if ((rc = pcm_measure_range(ctx, n0 - 1, n1 - 1, l0, l1))) return rc;
+  bool staged = false;
+  if ((rc = pcm_append_in(ctx, inc, n0 - 1, l0, &staged))) return rc;
+  if (!staged) {
+    if (inc->n_odom > 0) {
+      RPGO_HIP_CHECK(hipMemcpyAsync(s.odom.as<double>() + PL * d0, inc->odom, 8 * PL * inc->n_odom,
+                                    hipMemcpyHostToDevice, st));
+      RPGO_HIP_CHECK(hipMemcpyAsync(s.odom_cov.as<double>() + DD * d0, inc->odom_cov, 8 * DD * inc->n_odom,
+                                    hipMemcpyHostToDevice, st));
+    }
+    if (inc->n_lc > 0) {
+      RPGO_HIP_CHECK(hipMemcpyAsync(s.lc_from.as<int>() + L0, inc->lc_from, 4 * (size_t)inc->n_lc,
+                                    hipMemcpyHostToDevice, st));
+      RPGO_HIP_CHECK(hipMemcpyAsync(s.lc_to.as<int>() + L0, inc->lc_to, 4 * (size_t)inc->n_lc,
+                                    hipMemcpyHostToDevice, st));
+      RPGO_HIP_CHECK(hipMemcpyAsync(s.lc_pose.as<double>() + PL * L0, inc->lc_pose, 8 * PL * inc->n_lc,
+                                    hipMemcpyHostToDevice, st));
+      RPGO_HIP_CHECK(hipMemcpyAsync(s.lc_cov.as<double>() + DD * L0, inc->lc_cov, 8 * DD * inc->n_lc,
+                                    hipMemcpyHostToDevice, st));
+    }
+    RPGO_HIP_CHECK(hipMemsetAsync(s.counters.ptr, 0, 256, st));
+    if ((rc = pcm_measure_range(ctx, n0 - 1, n1 - 1, l0, l1))) return rc;
+  }
   if ((rc = pcm_fold_from(ctx, n0 - 1))) return rc;
   RPGO_HIP_CHECK(hipEventRecord(ev[1], st));
   int mn = 0;
@@ -545,16 +550,18 @@ int pcm_append_impl(rpgo_ctx* ctx, const rpgo_pcm_increment* inc, double odom_th
   s.m = m_old + mn;
   if ((rc = pcm_adj_append(ctx, m_old, lc_thr, s_loop))) return rc;
   RPGO_HIP_CHECK(hipEventRecord(ev[3], st));
-  RPGO_HIP_CHECK(hipEventSynchronize(ev[3]));
+  unsigned long long* cnt = static_cast<unsigned long long*>(ctx->host_pinned);
+  *cnt = 0;  // no new row: the counters stayed zero
+  if (stats && mn > 0) RPGO_HIP_CHECK(hipMemcpyAsync(cnt, s.counters.ptr, sizeof(*cnt), hipMemcpyDeviceToHost, st));
+  RPGO_HIP_CHECK(hipStreamSynchronize(st));
+  ctx->append_pending = false;
   if (stats) {
     const bool check = s_loop ? (s_loop->trans >= 0.0 && s_loop->rot >= 0.0) : lc_thr >= 0.0;
-    unsigned long long cnt = 0;
-    RPGO_HIP_CHECK(hipMemcpy(&cnt, s.counters.ptr, sizeof(cnt), hipMemcpyDeviceToHost));
     const int m = s.m;
     *stats = rpgo_pcm_stats{};
     stats->n_accepted = m;
     stats->n_pairs = check ? ((int64_t)m * (m - 1) - (int64_t)m_old * (m_old - 1)) / 2 : 0;
-    stats->n_consistent = (int64_t)cnt;
+    stats->n_consistent = (int64_t)*cnt;
     stats->ms_fold = elapsed(ev[0], ev[1]);
     stats->ms_odom = elapsed(ev[1], ev[2]);
     stats->ms_pairs = elapsed(ev[2], ev[3]);

@@ -10,6 +10,8 @@
 //   - adjacency bit packing    (Pcm.h:725-768, row-packed and symmetrized)
 //   - the PcmSimple checks     (Pcm.h:581-596, 654-662, PoseWithNode norms)
 // and the device functions reused by the FP32 path's near-threshold recheck.
+#include <cstring>
+
 #include "replay64.h"
 #include "rpgo_internal.h"
 
@@ -40,21 +42,28 @@ struct Chains {
 // the fold Jacobians H_k = Ad(delta_k^-1)          (GeometryUtils.h:91-129)
 // ---------------------------------------------------------------------------
 template <int DIM>
+__device__ __forceinline__ void measure_one(const double* pose, const double* cov, double* pwc, double* hinv) {
+  constexpr int PL = R64<DIM>::PL, D = R64<DIM>::D, PWC = R64<DIM>::PWC;
+  double rec[PWC];
+  R64<DIM>::from_measurement(pose, cov, rec);
+  for (int i = 0; i < PWC; ++i) pwc[i] = rec[i];
+  if (hinv) {
+    double inv[PL], H[D * D];
+    R64<DIM>::pose_inverse(rec, inv);
+    R64<DIM>::adjoint(inv, H);
+    for (int i = 0; i < D * D; ++i) hinv[i] = H[i];
+  }
+}
+
+template <int DIM>
 __global__ void k_measurements(int n, const double* __restrict__ pose,
                                const double* __restrict__ cov, double* __restrict__ pwc,
                                double* __restrict__ hinv) {
   constexpr int PL = R64<DIM>::PL, D = R64<DIM>::D, PWC = R64<DIM>::PWC;
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
-  double rec[PWC];
-  R64<DIM>::from_measurement(pose + (size_t)k * PL, cov + (size_t)k * D * D, rec);
-  for (int i = 0; i < PWC; ++i) pwc[(size_t)k * PWC + i] = rec[i];
-  if (hinv) {
-    double inv[PL], H[D * D];
-    R64<DIM>::pose_inverse(rec, inv);
-    R64<DIM>::adjoint(inv, H);
-    for (int i = 0; i < D * D; ++i) hinv[(size_t)k * D * D + i] = H[i];
-  }
+  measure_one<DIM>(pose + (size_t)k * PL, cov + (size_t)k * D * D, pwc + (size_t)k * PWC,
+                   hinv ? hinv + (size_t)k * D * D : nullptr);
 }
 
 // ---------------------------------------------------------------------------
@@ -621,6 +630,95 @@ __global__ void __launch_bounds__(64) k_recheck64_wave(const unsigned int* __res
 // ---------------------------------------------------------------------------
 // streaming append (one update() of the reference after another)
 // ---------------------------------------------------------------------------
+// A small increment from pinned host memory: the arrays of nd odometry steps
+// and nl loop closures to their places, their records as k_measurements, the
+// counters zeroed.  One workgroup, the increment through LDS.  A keyframe's
+// append is launches and copies, not work: this stands for up to six copies,
+// two launches and a memset.  One pose: 61 -> 44 us, with a loop closure 138
+// -> 85 us (with k_check_append).  It ends where the staging buffer does; at 80
+// poses it takes 76 us, at 90 the copies take 92.
+struct AppendIn {
+  const double* src;  // odom | odom_cov | lc_pose | lc_cov | lc_from, lc_to (int)
+  int nd, nl;
+  double *odom, *odom_cov, *lc_pose, *lc_cov, *delta, *hinv, *lcm;
+  int *lc_from, *lc_to;
+  unsigned int* counters;  // 64 words
+};
+
+template <int DIM>
+__global__ void __launch_bounds__(256) k_append_in(AppendIn a) {
+  constexpr int PL = R64<DIM>::PL, D = R64<DIM>::D, DD = D * D, PWC = R64<DIM>::PWC;
+  extern __shared__ double in[];
+  const int tid = threadIdx.x;
+  const int o1 = PL * a.nd, o2 = o1 + DD * a.nd, o3 = o2 + PL * a.nl, o4 = o3 + DD * a.nl;
+  for (int e = tid; e < o4; e += 256) {
+    const double v = a.src[e];
+    in[e] = v;
+    double* dst = e < o1 ? a.odom + e : e < o2 ? a.odom_cov + (e - o1) : e < o3 ? a.lc_pose + (e - o2) : a.lc_cov + (e - o3);
+    *dst = v;
+  }
+  const int* keys = reinterpret_cast<const int*>(a.src + o4);
+  for (int k = tid; k < a.nl; k += 256) {
+    a.lc_from[k] = keys[k];
+    a.lc_to[k] = keys[a.nl + k];
+  }
+  if (tid < 64) a.counters[tid] = 0u;
+  __syncthreads();
+  for (int k = tid; k < a.nd + a.nl; k += 256) {
+    const int q = k - a.nd;
+    if (q < 0)
+      measure_one<DIM>(in + PL * k, in + o1 + DD * k, a.delta + (size_t)k * PWC, a.hinv + (size_t)k * DD);
+    else
+      measure_one<DIM>(in + o2 + PL * q, in + o3 + DD * q, a.lcm + (size_t)q * PWC, nullptr);
+  }
+}
+
+// k_odom_check / k_odom_simple, the compaction and k_gather_append of up to
+// 256 new loop closures in one workgroup; the number accepted goes to *count
+// (pinned host memory)
+template <int DIM, bool SIMPLE>
+__global__ void __launch_bounds__(256) k_check_append(int nn, int l0, int m_old, const double* __restrict__ traj,
+                                                      const int* __restrict__ from, const int* __restrict__ to,
+                                                      const double* __restrict__ lcm, bool check, double thr,
+                                                      double thr_r, double* __restrict__ dist, int* __restrict__ flag,
+                                                      int* __restrict__ accepted, int* __restrict__ cf,
+                                                      int* __restrict__ ct, double* __restrict__ clcm,
+                                                      int* __restrict__ count) {
+  constexpr int PWC = R64<DIM>::PWC;
+  __shared__ int sums[4];
+  const int k = threadIdx.x, lane = k & 63, wid = k >> 6;
+  bool take = false;
+  int a = 0, b = 0;
+  if (k < nn) {
+    a = from[k];
+    b = to[k];
+    const double *ta = traj + (size_t)a * PWC, *tb = traj + (size_t)b * PWC, *z = lcm + (size_t)k * PWC;
+    double d;
+    if (SIMPLE) {
+      double rn;
+      R64<DIM>::simple_odom(ta, tb, z, abs(b - a) + 1, &d, &rn);
+      take = !check || (d < thr && rn < thr_r);
+    } else {
+      d = R64<DIM>::odom_dist(ta, tb, z);
+      take = !check || d < thr;
+    }
+    dist[k] = d;
+    flag[k] = take ? 1 : 0;
+  }
+  const unsigned long long bits = __ballot(take);
+  if (lane == 0) sums[wid] = __popcll(bits);
+  __syncthreads();
+  int o = m_old + __popcll(bits & ((1ull << lane) - 1ull));
+  for (int w = 0; w < wid; ++w) o += sums[w];
+  if (take) {
+    accepted[o] = l0 + k;
+    cf[o] = a;
+    ct[o] = b;
+    for (int e = 0; e < PWC; ++e) clcm[(size_t)o * PWC + e] = lcm[(size_t)k * PWC + e];
+  }
+  if (k == 0) *count = sums[0] + sums[1] + sums[2] + sums[3];
+}
+
 // accepted[m_old + t] = l0 + tmp[t] and the compacted records, t < m_new
 template <int DIM>
 __global__ void k_gather_append(int m_old, int m_new, int l0, const int* __restrict__ tmp,
@@ -928,6 +1026,58 @@ int pcm_symmetrize(rpgo_ctx* ctx) {
   return RPGO_OK;
 }
 
+// The increment (odometry from o0, loop closures from l0) through the pinned
+// staging buffer; *done = false when it is too large for it
+int pcm_append_in(rpgo_ctx* ctx, const rpgo_pcm_increment* inc, int o0, int l0, bool* done) {
+  PcmState& s = ctx->pcm;
+  const size_t PL = pose_len(s.dim), D = tan_dim(s.dim), DD = D * D, pwc = pwc_len(s.dim);
+  const size_t nd = (size_t)inc->n_odom, nl = (size_t)inc->n_lc;
+  *done = false;
+  if (nd + nl > kAppendStage / 64) return RPGO_OK;
+  const size_t words = (PL + DD) * (nd + nl), bytes = 8 * words + 8 * nl;
+  if (bytes > (size_t)kAppendStage) return RPGO_OK;
+  if (!ctx->append_stage && hipHostMalloc(&ctx->append_stage, kAppendStage, hipHostMallocDefault) != hipSuccess) {
+    ctx->append_stage = nullptr;
+    (void)hipGetLastError();
+    return RPGO_OK;
+  }
+  // an append that failed half way may have left its kernel reading
+  if (ctx->append_pending) RPGO_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+  double* h = static_cast<double*>(ctx->append_stage);
+  const auto put = [&h](const double* src, size_t n) {
+    if (n) std::memcpy(h, src, 8 * n);
+    h += n;
+  };
+  put(inc->odom, PL * nd);
+  put(inc->odom_cov, DD * nd);
+  put(inc->lc_pose, PL * nl);
+  put(inc->lc_cov, DD * nl);
+  if (nl) {
+    std::memcpy(h, inc->lc_from, 4 * nl);
+    std::memcpy(reinterpret_cast<int*>(h) + nl, inc->lc_to, 4 * nl);
+  }
+  AppendIn a;
+  a.src = static_cast<const double*>(ctx->append_stage);
+  a.nd = (int)nd;
+  a.nl = (int)nl;
+  a.odom = s.odom.as<double>() + PL * o0;
+  a.odom_cov = s.odom_cov.as<double>() + DD * o0;
+  a.lc_pose = s.lc_pose.as<double>() + PL * l0;
+  a.lc_cov = s.lc_cov.as<double>() + DD * l0;
+  a.delta = s.delta.as<double>() + pwc * o0;
+  a.hinv = s.hinv.as<double>() + DD * o0;
+  a.lcm = s.lcm.as<double>() + pwc * l0;
+  a.lc_from = s.lc_from.as<int>() + l0;
+  a.lc_to = s.lc_to.as<int>() + l0;
+  a.counters = s.counters.as<unsigned int>();
+  ctx->append_pending = true;
+  if (s.dim == 3) k_append_in<3><<<1, 256, 8 * words, ctx->stream>>>(a);
+  else k_append_in<2><<<1, 256, 8 * words, ctx->stream>>>(a);
+  RPGO_HIP_CHECK(hipGetLastError());
+  *done = true;
+  return RPGO_OK;
+}
+
 int pcm_odom_append(rpgo_ctx* ctx, int l0, double odom_thr, const SimpleThr* simple, int* m_new) {
   PcmState& s = ctx->pcm;
   const int n = s.n_lc, nn = n - l0, m_old = s.m, pwc = pwc_len(s.dim);
@@ -951,6 +1101,29 @@ int pcm_odom_append(rpgo_ctx* ctx, int l0, double odom_thr, const SimpleThr* sim
   double* od = s.odom_dist.as<double>() + l0;
   int* fl = s.flags.as<int>() + l0;
   const unsigned g = (unsigned)((nn + 255) / 256);
+  if (nn <= 256) {
+    // one launch and the count in pinned memory, where the general path takes
+    // three launches and a copy
+    int* count = reinterpret_cast<int*>(static_cast<char*>(ctx->host_pinned) + kPinnedAppend);
+    const bool check = simple ? simple->trans >= 0.0 && simple->rot >= 0.0 : !(odom_thr < 0.0);
+    const double t1 = simple ? simple->trans : odom_thr, t2 = simple ? simple->rot : 0.0;
+#define RPGO_CHECK_APPEND(DIM, SIMPLE)                                                                             \
+  k_check_append<DIM, SIMPLE><<<1, 256, 0, st>>>(nn, l0, m_old, s.traj.as<double>(), from, to, lcm, check, t1, t2, \
+                                                 od, fl, s.accepted.as<int>(), s.c_from.as<int>(),                \
+                                                 s.c_to.as<int>(), s.c_lcm.as<double>(), count)
+    if (s.dim == 3) {
+      if (simple) RPGO_CHECK_APPEND(3, true);
+      else RPGO_CHECK_APPEND(3, false);
+    } else {
+      if (simple) RPGO_CHECK_APPEND(2, true);
+      else RPGO_CHECK_APPEND(2, false);
+    }
+#undef RPGO_CHECK_APPEND
+    RPGO_HIP_CHECK(hipGetLastError());
+    RPGO_HIP_CHECK(hipStreamSynchronize(st));
+    *m_new = *static_cast<volatile int*>(count);
+    return RPGO_OK;
+  }
   if (simple) {
     const bool check = simple->trans >= 0.0 && simple->rot >= 0.0;
     if (s.dim == 3)

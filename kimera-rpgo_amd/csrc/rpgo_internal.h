@@ -141,6 +141,8 @@ struct rpgo_ctx {
   rpgo::SolveLanes* solve_lanes = nullptr;  // created by rpgo_solve_batched
   rpgo::MlpState* mlp = nullptr;      // created by rpgo_mlp_set_params
   rpgo::BatchState* batch = nullptr;  // created by rpgo_pcm_batch_run
+  void* append_stage = nullptr;       // pinned staging of a small append, on first use
+  bool append_pending = false;        // a kernel may still read append_stage
   void* host_pinned = nullptr;        // 256 B pinned host buffer for counter readbacks (PCM
                                       // counters in the first 128, clique results after them)
   int n_cu = 256;                     // compute units of the device (launch shapes)
@@ -149,6 +151,8 @@ struct rpgo_ctx {
 
 namespace rpgo {
 constexpr int kPinnedClique = 128;  // byte offset in rpgo_ctx::host_pinned
+constexpr int kPinnedAppend = 96;   // likewise: loop closures an append accepted
+constexpr int kAppendStage = 32 * 1024;  // bytes of rpgo_ctx::append_stage
 // PcmSimple thresholds of one check (translation, rotation per node);
 // a negative value disables the check
 struct SimpleThr {
@@ -164,6 +168,7 @@ int pcm_odom_and_compact(rpgo_ctx* ctx, double odom_thr, int* m_out,
 int pcm_pairs_fp64(rpgo_ctx* ctx, double lc_thr, bool want_dist);
 int pcm_pairs_simple(rpgo_ctx* ctx, const SimpleThr& thr, bool want_dist);
 // measurement records of odometry [o0, o1) and loop closures [l0, l1)
+int pcm_append_in(rpgo_ctx* ctx, const rpgo_pcm_increment* inc, int o0, int l0, bool* done);
 int pcm_measure_range(rpgo_ctx* ctx, int o0, int o1, int l0, int l1);
 // continue the fold from chain record `start` up to record n_poses-1
 int pcm_fold_from(rpgo_ctx* ctx, int start);

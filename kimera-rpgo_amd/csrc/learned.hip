@@ -162,7 +162,14 @@ __global__ void k_pack(const float* __restrict__ P, bf16* __restrict__ W1t, bf16
 // Forward pass, 64 rows per workgroup (one wavefront per 16 rows).  Rows are
 // gathered through idx when given.  Saves the BF16 layer inputs (Xb, H1, H2)
 // for the backward pass when the pointers are non-null.
-constexpr int kLdA = kH + 8;  // LDS row pitch of the activations (BF16)
+constexpr int kLdA = kH + 8;  // LDS row pitch of the activations and of W2 (BF16): 16 bytes past a
+                              // multiple of the banks, so sixteen rows read at once do not collide
+
+// W2 (128 x 128, row-major) to LDS rows of kLdA
+__device__ __forceinline__ void stage_w2(const bf16* __restrict__ W, bf16 (*sW)[kLdA]) {
+  for (int e = threadIdx.x; e < kH * kH / 8; e += blockDim.x)
+    *reinterpret_cast<uint4*>(&sW[e / (kH / 8)][8 * (e % (kH / 8))]) = reinterpret_cast<const uint4*>(W)[e];
+}
 
 __global__ void __launch_bounds__(256) k_mlp_forward(int n, const float* __restrict__ X, const int* __restrict__ idx,
                                                      const float* __restrict__ norm, const bf16* __restrict__ W1t,
@@ -170,11 +177,10 @@ __global__ void __launch_bounds__(256) k_mlp_forward(int n, const float* __restr
                                                      const float* __restrict__ P, float* __restrict__ Y,
                                                      bf16* __restrict__ Xb, bf16* __restrict__ H1,
                                                      bf16* __restrict__ H2) {
-  __shared__ bf16 sW2[kH * kH];
-  __shared__ bf16 act1[4][16][kLdA];
-  __shared__ bf16 act2[4][16][kLdA];
-  for (int e = threadIdx.x; e < kH * kH / 4; e += blockDim.x)
-    reinterpret_cast<uint2*>(sW2)[e] = reinterpret_cast<const uint2*>(W2t)[e];
+  __shared__ __align__(16) bf16 sW2[kH][kLdA];
+  __shared__ __align__(16) bf16 act1[4][16][kLdA];
+  __shared__ __align__(16) bf16 act2[4][16][kLdA];
+  stage_w2(W2t, sW2);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, q = l >> 4, r = l & 15;
   const int row0 = blockIdx.x * 64 + w * 16;
   const float* b1 = P + oB1;
@@ -222,7 +228,7 @@ __global__ void __launch_bounds__(256) k_mlp_forward(int n, const float* __restr
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         aa[j] = (short)act1[w][r][kt * 32 + 8 * q + j];
-        bb[j] = (short)sW2[(nt * 16 + r) * kH + kt * 32 + 8 * q + j];
+        bb[j] = (short)sW2[nt * 16 + r][kt * 32 + 8 * q + j];
       }
       acc = mfma32(aa, bb, acc);
     }
@@ -296,29 +302,30 @@ __global__ void k_mlp_back_h2(int n, const float* __restrict__ dY, const bf16* _
   dH2[t] = bf2f(H2[t]) > 0.f ? f2bf(g) : (bf16)0;
 }
 
-// dH1 = relu'(H1) * (dH2 W2^T) on the matrix cores, 64 rows per workgroup
+// dH1 = relu'(H1) * (dH2 W2^T) on the matrix cores, 64 rows per workgroup.
+// Each lane holds its row's fragments of dH2 (four 16-byte loads) for all
+// eight column tiles.  With two-byte loads repeated for every tile and W2's rows
+// on the same banks 5,000 rows took 41 us, so 12.5 us (k_mlp_forward, by the
+// banks alone, 17.4 -> 14.9 us).
 __global__ void __launch_bounds__(256) k_mlp_back_h1(int n, const bf16* __restrict__ dH2,
                                                      const bf16* __restrict__ W2b, const bf16* __restrict__ H1,
                                                      bf16* __restrict__ dH1) {
-  __shared__ bf16 sW2[kH * kH];
-  for (int e = threadIdx.x; e < kH * kH / 4; e += blockDim.x)
-    reinterpret_cast<uint2*>(sW2)[e] = reinterpret_cast<const uint2*>(W2b)[e];
-  __syncthreads();
+  __shared__ __align__(16) bf16 sW2[kH][kLdA];
+  stage_w2(W2b, sW2);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, q = l >> 4, r = l & 15;
   const int row0 = blockIdx.x * 64 + w * 16;
   const int arow = row0 + r;
+  bf16x8 a[kH / 32];
+#pragma unroll
+  for (int kt = 0; kt < kH / 32; ++kt)
+    a[kt] = arow < n ? *reinterpret_cast<const bf16x8*>(dH2 + (size_t)arow * kH + kt * 32 + 8 * q) : bf16x8{};
+  __syncthreads();
 #pragma unroll
   for (int nt = 0; nt < kH / 16; ++nt) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kt = 0; kt < kH / 32; ++kt) {
-      bf16x8 aa, bb;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        aa[j] = arow < n ? (short)dH2[(size_t)arow * kH + kt * 32 + 8 * q + j] : (short)0;
-        bb[j] = (short)sW2[(nt * 16 + r) * kH + kt * 32 + 8 * q + j];
-      }
-      acc = mfma32(aa, bb, acc);
+      acc = mfma32(a[kt], *reinterpret_cast<const bf16x8*>(&sW2[nt * 16 + r][kt * 32 + 8 * q]), acc);
     }
     const int col = nt * 16 + r;
 #pragma unroll
@@ -448,7 +455,10 @@ static void mlp_grad_pass(MlpState& s, hipStream_t st, int n, const float* X, co
   k_mlp_back_h2<<<(unsigned)(((long long)n * kH + 255) / 256), 256, 0, st>>>(n, s.dY.as<float>(), s.W3t.as<bf16>(),
                                                                           s.H2.as<bf16>(), s.dH2.as<bf16>());
   k_mlp_back_h1<<<blocks, 256, 0, st>>>(n, s.dH2.as<bf16>(), s.W2b.as<bf16>(), s.H1.as<bf16>(), s.dH1.as<bf16>());
-  const int zs = std::max(1, std::min(64, n / 1024));
+  // row splits: every wavefront's loads are a memory latency per 32 rows, so a
+  // split is one such step up to the 64 atomic adds an entry takes.  5,000
+  // rows: 4 splits 26 us, 39 splits 7.8 us.
+  const int zs = std::max(1, std::min(64, n / 128));
   float* G = s.G.as<float>();
   k_mlp_wgrad<<<dim3(kF / 16, kH / 16, zs), 256, 0, st>>>(n, s.Xb.as<bf16>(), kF, s.dH1.as<bf16>(), kH, G + oW1,
                                                          kH, kH);

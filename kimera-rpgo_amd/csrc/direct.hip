@@ -23,7 +23,6 @@
 #include <cmath>
 #include <new>
 
-#include "replay64.h"
 #include "rpgo_internal.h"
 #include "rpgo_solver.h"
 #include "solver_device.h"

@@ -100,8 +100,9 @@ struct DirectPlan {
 // between random poses (outliers left in the graph) end in one wide clique,
 // eliminated a pose a level.  LM on helices with loop closures 1/5 of the
 // poses, outliers kept, direct / PCG: 2,000 poses, 50 % (widest front 122, 118
-// MB of updates) 233 / 419 ms; 5,000, 10 % (162, 370 MB) 465 / 626 ms; 5,000,
-// 20 % (223, 754 MB) 622 / 474 ms; 10,000, 10 % (256, 1.7 GB) 803 / 611 ms.
+// MB of updates) 197 / 417 ms; 5,000, 10 % (162, 370 MB) 387 / 629 ms; with one
+// pivot a front (wide fronts have one either way) 5,000, 20 % (223, 754 MB) 622
+// / 474 ms; 10,000, 10 % (256, 1.7 GB) 803 / 611 ms.
 // Graphs after PCM stay far below in width (50,000 poses: 26, 135 MB; with
 // 10,000 loop closures 58, 514 MB).
 struct DirectLimits {

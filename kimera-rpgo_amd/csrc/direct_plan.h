@@ -8,8 +8,14 @@
 // and a level is one launch.  While poses of degree <= 2 exist (the odometry
 // chain between loop closures) a level takes an independent set of them, which
 // is odd-even reduction of the chain: log2 of the longest run of levels.
-// After that a level takes an independent set of the poses of degree at most
-// max(3 dmin, dmin + 4), smallest degree first.  The exact minimum degree
+// After that, and once kThinLevels of those levels had such poses in less than
+// an eighth of the graph, a level takes an independent set of the poses of
+// degree at most max(3 dmin, dmin + 4), smallest degree first.  (A chain seen
+// from one landmark is a fan: only its two ends have degree 2, every pose
+// between them 3.  Two poses a level made 1,003 levels of 10,000 poses seen
+// 2,000 times and 10,001 of 20,000 poses all seen; 30 and 28 so.  Chains with
+// loop closures end their degree <= 2 phase with at most 12 such levels, so
+// their plans do not change.)  The exact minimum degree
 // (threshold dmin) gives the least fill but, once the graph is a strip of
 // cliques, eats it from its ends in long dependent chains: on a helix of
 // 50,000 poses with 5,000 loop closures 1,148 levels and 320,187 update
@@ -112,6 +118,9 @@ struct DirectLimits {
   int64_t u_free = 64ll << 20;
   int64_t max_steps = 400ll << 20;   // list entries touched while eliminating
   int64_t max_maps = 64ll << 20;
+  // elimination levels: about 8 us each, forward and backward, so that these
+  // cost what 300 PCG iterations of 57 us do at 50,000 poses
+  int max_levels = 2048;
 };
 
 namespace plan_detail {
@@ -133,10 +142,13 @@ struct Lists {
   }
 };
 
+constexpr int kThinLevels = 12;
+
 }  // namespace plan_detail
 
 inline bool build_direct_plan(int N, int F, const int32_t* kind, const int32_t* fi, const int32_t* fj,
                               const DirectLimits& lim, DirectPlan& P) {
+  using plan_detail::kThinLevels;
   using plan_detail::Lists;
   P = DirectPlan();
   P.N = N;
@@ -175,14 +187,22 @@ inline bool build_direct_plan(int N, int F, const int32_t* kind, const int32_t* 
   std::vector<int32_t> mark(N, -1), elim(N, -1), tmp;
   std::vector<int32_t> bucket_off, cand;
   int64_t steps = 0, u_len = 0;
+  int thin_levels = 0;
   const int64_t max_u = std::min(lim.max_u, std::max(lim.u_free, lim.max_u_pose * N));
   for (int level = 0; !alive.empty(); ++level) {
+    if (level >= lim.max_levels) return false;
     int dmin = A.len[alive[0]];
-    for (int v : alive) dmin = std::min(dmin, (int)A.len[v]);
+    size_t chain_poses = 0;
+    for (int v : alive) {
+      dmin = std::min(dmin, (int)A.len[v]);
+      chain_poses += A.len[v] <= 2;
+    }
+    const bool thin = dmin <= 2 && 8 * chain_poses < alive.size();
+    thin_levels += thin;
     // the fill still to come is more than a quarter of what the remaining
     // poses' present degree would make: give up early when that is too much
     if (u_len + (int64_t)(alive.size() / 4) * front_update_len(dmin) > max_u) return false;
-    const int thr = dmin <= 2 ? 2 : std::max(3 * dmin, dmin + 4);
+    const int thr = dmin <= 2 && !(thin && thin_levels > kThinLevels) ? 2 : std::max(3 * dmin, dmin + 4);
     // candidates by degree, then index (counting sort)
     bucket_off.assign(thr + 2, 0);
     for (int v : alive)

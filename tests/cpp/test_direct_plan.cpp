@@ -209,6 +209,22 @@ std::vector<std::pair<int, int>> chain(int N) {
   return e;
 }
 
+// a chain of N poses and pose N, seen from `seen` of them, evenly spread
+std::vector<std::pair<int, int>> chain_hub(int N, int seen) {
+  auto e = chain(N);
+  for (int k = 0; k < seen; ++k) e.push_back({(int)((int64_t)k * N / seen), N});
+  return e;
+}
+
+bool plan(int N, const std::vector<std::pair<int, int>>& edges, const DirectLimits& lim, DirectPlan& P) {
+  std::vector<int32_t> kind(edges.size(), 0), fi, fj;
+  for (auto& e : edges) {
+    fi.push_back(e.first);
+    fj.push_back(e.second);
+  }
+  return build_direct_plan(N, (int)edges.size(), kind.data(), fi.data(), fj.data(), lim, P);
+}
+
 }  // namespace
 
 TEST(DirectPlan, Chains) {
@@ -259,6 +275,22 @@ TEST(DirectPlan, Shapes) {
   check("laps", 120, ladder, 5, rpgo_failures_);
 }
 
+// Poses around one shared pose: the levels stay logarithmic in the chain (a fan
+// halves per level once the first thin levels are past), and the plan solves
+TEST(DirectPlan, ChainAndHub) {
+  EXPECT(check("hub", 101, chain_hub(100, 100), 7, rpgo_failures_) <= 12 + 10);
+  EXPECT(check("hub", 201, chain_hub(200, 60), 8, rpgo_failures_) <= 12 + 12);
+  const int sizes[4][2] = {{3000, 300}, {10000, 2000}, {20000, 20000}, {50000, 5000}};
+  for (auto& z : sizes) {
+    DirectPlan P;
+    EXPECT(plan(z[0] + 1, chain_hub(z[0], z[1]), DirectLimits(), P));
+    std::printf("  hub %d/%d: %d levels\n", z[1], z[0], P.levels());
+    // odd-even reduction to the poses that see the hub, the thin levels, and
+    // halving of the fan: at most log2(N) + 12 + log2(N) with a few to spare
+    EXPECT(P.levels() <= 12 + 2 * 16 + 4);
+  }
+}
+
 TEST(DirectPlan, Limits) {
   std::vector<std::pair<int, int>> clique;
   for (int a = 0; a < 20; ++a)
@@ -269,6 +301,10 @@ TEST(DirectPlan, Limits) {
   lim.max_d = 18;
   EXPECT(!build_direct_plan(20, (int)s.kind.size(), s.kind.data(), s.fi.data(), s.fj.data(), lim, P));
   lim.max_d = 19;
+  EXPECT(build_direct_plan(20, (int)s.kind.size(), s.kind.data(), s.fi.data(), s.fj.data(), lim, P));
+  lim.max_levels = 19;  // a pose a level
+  EXPECT(!build_direct_plan(20, (int)s.kind.size(), s.kind.data(), s.fi.data(), s.fj.data(), lim, P));
+  lim.max_levels = 20;
   EXPECT(build_direct_plan(20, (int)s.kind.size(), s.kind.data(), s.fi.data(), s.fj.data(), lim, P));
   lim.max_u = -1;  // the limit counts every pivot's update by itself
   for (int d = 0; d < 20; ++d) lim.max_u += front_update_len(d);

@@ -74,6 +74,11 @@ def _clique(n):
     return [(a, b) for a in range(n) for b in range(a + 1, n)]
 
 
+def _chain_hub(n, seen):
+    """A chain of n poses and pose n, seen from `seen` of them."""
+    return n + 1, _chain(n) + [(k * n // seen, n) for k in range(seen)]
+
+
 CASES = {
     "one_pose": (1, [], (0,)),
     "two_poses": (2, [(1, 0)], (1,)),
@@ -82,6 +87,8 @@ CASES = {
     "chain_65_repeated": (65, _chain(65) + _flip(_chain(65)[::2], 2), (30,)),
     "shuffled_130": (130, _shuffled(130, 40, 3), (0,)),
     "star_70": (70, _flip([(0, k) for k in range(1, 70)], 4), (0,)),
+    "hub_60_of_200": (*_chain_hub(200, 60), (0,)),
+    "hub_300_of_300": (*_chain_hub(300, 300), (0,)),
     "two_components": (41, _chain(20) + [(k, k + 1) for k in range(20, 40)] + [(3, 15)], (0, 20)),
     "clique_6": (6, _clique(6), (0,)),
     "clique_11": (11, _flip(_clique(11), 5), (0,)),
@@ -136,3 +143,18 @@ def test_gnc_large_refinement(ctx):
     d = np.abs(a - b).max()
     print(f"[direct] 9001 poses lm {ra.lm_iterations}/{rb.lm_iterations} d {d:.1e}", flush=True)
     assert ra.lm_iterations == rb.lm_iterations and d < TOL
+
+
+def test_hub_not_slower_than_pcg(ctx):
+    """A landmark seen from a tenth of a chain: the plan's levels stay few, so
+    a direct solve takes less device time than the PCG (about a tenth)."""
+    n, edges = _chain_hub(3000, 300)
+    g = _graph(n, edges, 5)
+    ctx.solve(*g)
+    a, _, ra = ctx.solve(*g)
+    ctx.solve(*g, pcg_segment=16, pcg_rel_tol=1e-9)
+    b, _, rb = ctx.solve(*g, pcg_segment=16, pcg_rel_tol=1e-9)
+    d = np.abs(a - b).max()
+    print(f"[direct] hub 300/3000 {ra.ms_total:.2f} ms, pcg {rb.ms_total:.2f} ms, d {d:.1e}", flush=True)
+    assert ra.lm_iterations == rb.lm_iterations and d < TOL
+    assert ra.ms_total < rb.ms_total

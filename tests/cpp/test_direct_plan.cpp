@@ -163,10 +163,11 @@ std::vector<double> plan_solve(const Sys& s, const DirectPlan& P, int& bad) {
   return x;
 }
 
-int check(const char* what, int N, const std::vector<std::pair<int, int>>& edges, unsigned seed, int& rpgo_failures_) {
+int check(const char* what, int N, const std::vector<std::pair<int, int>>& edges, unsigned seed, int& rpgo_failures_,
+          const DirectLimits& lim = DirectLimits()) {
   const Sys s = random_system(N, edges, seed);
   DirectPlan P;
-  EXPECT(build_direct_plan(N, (int)s.kind.size(), s.kind.data(), s.fi.data(), s.fj.data(), DirectLimits(), P));
+  EXPECT(build_direct_plan(N, (int)s.kind.size(), s.kind.data(), s.fi.data(), s.fj.data(), lim, P));
   // every pose a pivot once, levels contiguous, no factor between two fronts
   // of a level, every front within the level's bounds and the LDS
   std::vector<int> level(N, -1), front(N, -1);
@@ -288,6 +289,38 @@ TEST(DirectPlan, ChainAndHub) {
     // odd-even reduction to the poses that see the hub, the thin levels, and
     // halving of the fan: at most log2(N) + 12 + log2(N) with a few to spare
     EXPECT(P.levels() <= 12 + 2 * 16 + 4);
+  }
+}
+
+// The work of planning is linear in the poses around a shared pose (a few
+// list entries a factor and level), not quadratic; lists above the length from
+// which a level's merges are joined plan the same solve
+TEST(DirectPlan, LongLists) {
+  std::vector<std::pair<int, int>> star, two;
+  for (int k = 0; k < 20000; ++k) star.push_back({k % 2 ? k : 20000, k % 2 ? 20000 : k});
+  DirectLimits lim;
+  lim.max_steps = 100 * 20000;  // one merge a pose took 2e8
+  DirectPlan P;
+  EXPECT(plan(20001, star, lim, P) && P.levels() == 2);
+  EXPECT(plan(20001, chain_hub(20000, 20000), lim, P));
+  // every pose with more than `long_list` neighbours takes the joined merge
+  std::vector<std::pair<int, int>> clique;
+  two = chain(90);  // two hubs, each seen from all
+  for (int k = 0; k < 90; ++k)
+    for (int h : {90, 91}) two.push_back({h, k});
+  for (int a = 0; a < 30; ++a)
+    for (int b = a + 1; b < 30; ++b) clique.push_back({b, a});
+  for (int l : {0, 1, 3, 8, 40}) {
+    lim = DirectLimits();
+    lim.long_list = l;
+    const auto hub = chain_hub(120, 90);
+    const int direct = check("two hubs", 92, two, 13, rpgo_failures_);
+    EXPECT(check("two hubs", 92, two, 13, rpgo_failures_, lim) == direct);
+    EXPECT(check("hub", 121, hub, 14, rpgo_failures_, lim) == check("hub", 121, hub, 14, rpgo_failures_));
+    check("clique", 30, clique, 15, rpgo_failures_, lim);
+    DirectPlan A, B;  // the same plan
+    EXPECT(plan(121, hub, lim, A) && plan(121, hub, DirectLimits(), B));
+    EXPECT(A.row_pose == B.row_pose && A.maps == B.maps && A.lvl == B.lvl && A.u_len == B.u_len);
   }
 }
 

@@ -701,13 +701,18 @@ int SolverRun::direct_setup(hipStream_t st, const int32_t* h_kind, const int32_t
                            P.maps.size() * sizeof(int32_t)};
   const void* src[5] = {P.meta.data(), P.childs.data(), P.origs.data(), P.row_pose.data(), P.maps.data()};
   DevBuf* dst[5] = {&d_meta, &d_childs, &d_origs, &d_rows, &d_maps};
-  for (int k = 0; k < 5; ++k)
-    if (dst[k]->reserve(bytes[k])) return RPGO_OK;  // no room: keep the iterative solve
   const size_t nblk = (size_t)(N + 63) / 64, ncost = (size_t)(F + 255) / 256;
-  if (d_U.reserve(sizeof(double) * (size_t)P.u_len) || d_G.reserve(sizeof(double) * (size_t)P.g_len) ||
-      d_part.reserve(sizeof(double) * (4 * nblk + ncost)) || d_bad.reserve(sizeof(int)))
+  int failed = 0;
+  for (int k = 0; k < 5 && !failed; ++k) failed = dst[k]->reserve(bytes[k]);
+  if (failed || d_U.reserve(sizeof(double) * (size_t)P.u_len) || d_G.reserve(sizeof(double) * (size_t)P.g_len) ||
+      d_part.reserve(sizeof(double) * (4 * nblk + ncost)) || d_bad.reserve(sizeof(int)) || !pinned_scalars()) {
+    // no room: keep the iterative solve, with the memory these buffers hold
+    // and without the failed allocation's error, which the next launch's check
+    // would report
+    (void)hipGetLastError();
+    direct_release();
     return RPGO_OK;
-  if (!pinned_scalars()) return RPGO_OK;
+  }
   for (int k = 0; k < 5; ++k)
     if (bytes[k]) RPGO_HIP_CHECK(hipMemcpyAsync(dst[k]->ptr, src[k], bytes[k], hipMemcpyHostToDevice, st));
   RPGO_HIP_CHECK(hipMemsetAsync(d_bad.ptr, 0, sizeof(int), st));

@@ -112,7 +112,12 @@ struct SolverRun {
   int direct_cost(hipStream_t st, const double* xp, double* out);
   int run(hipStream_t st, const rpgo_solve_problem* pr, rpgo_solve_report* rep);
   double* cost_buf() { return cost.as<double>(); }
+  void direct_release() {
+    direct_ready = false;
+    for (DevBuf* v : {&d_meta, &d_childs, &d_origs, &d_rows, &d_maps, &d_U, &d_G, &d_part, &d_bad}) v->release();
+  }
   void release() {
+    direct_release();
     if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
     graph_exec = nullptr;
     if (h_scalars) (void)hipHostFree(h_scalars);
@@ -122,8 +127,7 @@ struct SolverRun {
                       &Hjj, &Hij, &gi, &gj, &inc_off, &inc_cnt, &inc, &inc_q, &D, &Minv, &hdiag, &b64,
                       &chain, &Useg, &Ds, &Cs, &ext_off, &ext, &ext_q, &Pb, &Ac, &Lci, &LcT, &Ainv, &cres,
                       &ccor,
-                      &dx, &r, &zv, &p, &q, &hx, &sc, &d_meta, &d_childs, &d_origs, &d_rows, &d_maps,
-                      &d_U, &d_G, &d_part, &d_bad})
+                      &dx, &r, &zv, &p, &q, &hx, &sc})
       v->release();
   }
 };

@@ -10,6 +10,9 @@ to at most 1e-9 (PCG) and 1e-10 (direct) of its right-hand side; the graphs'
 condition numbers stay below about 1e3 per unit of pose, so steps agree to
 1e-6 with room.
 """
+import os
+import subprocess
+
 import numpy as np
 import pytest
 
@@ -158,3 +161,12 @@ def test_hub_not_slower_than_pcg(ctx):
     print(f"[direct] hub 300/3000 {ra.ms_total:.2f} ms, pcg {rb.ms_total:.2f} ms, d {d:.1e}", flush=True)
     assert ra.lm_iterations == rb.lm_iterations and d < TOL
     assert ra.ms_total < rb.ms_total
+
+
+def test_allocation_failure_binary():
+    """A device allocation of the direct path that fails (tests/cpp): the solve
+    goes on with the PCG, and a later one takes the direct path again."""
+    exe = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "bin", "test_alloc_failure")
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=100)
+    print(r.stdout, r.stderr, flush=True)
+    assert r.returncode == 0

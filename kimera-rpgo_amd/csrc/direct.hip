@@ -678,9 +678,14 @@ __global__ void __launch_bounds__(256) k_direct_reduce(int n, const double* __re
   if (threadIdx.x == 0) out[5] = bad ? (double)*bad : 0.0;
 }
 
-__global__ void k_direct_axpy(long long n, const double* __restrict__ a, double* __restrict__ y) {
+// y += a, the former y kept in old
+__global__ void k_direct_axpy(long long n, const double* __restrict__ a, double* __restrict__ y,
+                              double* __restrict__ old) {
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) y[t] += a[t];
+  if (t >= n) return;
+  const double v = y[t];
+  old[t] = v;
+  y[t] = v + a[t];
 }
 
 // ------------------------------------------------------------------ host
@@ -781,7 +786,8 @@ int SolverRun::direct_check(hipStream_t st, double lambda) {
   return RPGO_OK;
 }
 
-// One refinement step: dx += (H + lambda damp)^-1 r with the stored factor
+// One refinement step: dx += (H + lambda damp)^-1 r with the stored factor; the
+// step before it stays in q
 int SolverRun::direct_refine(hipStream_t st) {
   const DirectPlan& P = plan;
   for (int l = 0; l < P.levels(); ++l) {
@@ -797,7 +803,7 @@ int SolverRun::direct_refine(hipStream_t st) {
   int rc;
   if ((rc = direct_backward(st, zv.as<double>()))) return rc;
   const long long n6 = 6ll * N;
-  k_direct_axpy<<<(unsigned)((n6 + 255) / 256), 256, 0, st>>>(n6, zv.as<double>(), dx.as<double>());
+  k_direct_axpy<<<(unsigned)((n6 + 255) / 256), 256, 0, st>>>(n6, zv.as<double>(), dx.as<double>(), q.as<double>());
   RPGO_HIP_CHECK(hipGetLastError());
   return RPGO_OK;
 }
@@ -805,14 +811,16 @@ int SolverRun::direct_refine(hipStream_t st) {
 // One linear step by the factorization, the step's candidate poses xn and
 // their weighted cost: *lin the model decrease b.dx - dx.H dx / 2 (undamped
 // H), *cost_new the cost.  *ok = false when a pivot was not positive or the
-// residual stayed large: the caller then takes the iterative solve.
+// residual stayed above what the caller asked for: the caller then takes the
+// iterative solve.
 int SolverRun::direct_step(hipStream_t st, double lambda, double* lin, double* cost_new, bool* ok) {
   int rc;
   double* h = pinned_scalars();
   const int nblk = (N + 63) / 64, ncost = (F + 255) / 256;
   double* cpart = d_part.as<double>() + 4 * (size_t)nblk;
+  const double tol = std::min(prm.pcg_rel_tol, kDirectTol);
   *ok = false;
-  double prev = INFINITY;
+  double best = INFINITY;
   if ((rc = direct_factor(st, lambda))) return rc;
   if ((rc = direct_backward(st, dx.as<double>()))) return rc;
   stats.pcg_iterations += 1;
@@ -828,33 +836,49 @@ int SolverRun::direct_step(hipStream_t st, double lambda, double* lin, double* c
       RPGO_HIP_CHECK(hipMemsetAsync(d_bad.ptr, 0, sizeof(int), st));
       return RPGO_OK;
     }
-    *lin = bdx - 0.5 * xhx;
-    *cost_new = h[36];
-    last_residual = bb > 0.0 ? std::sqrt(rr / bb) : 0.0;
-    if (!(rr == rr) || !(last_residual < 1e-2)) return RPGO_OK;
+    const double residual = std::sqrt(bb > 0.0 ? rr / bb : rr);  // b = 0: dx and r are 0, or NaN
+    const double before = best;
+    if (refine == 0 && !(residual < 1e-2)) return RPGO_OK;
+    if (residual < best) {
+      best = residual;
+      *lin = bdx - 0.5 * xhx;
+      *cost_new = h[36];
+    } else if (refine > 0) {  // the refinement lost: the step before it
+      RPGO_HIP_CHECK(hipMemcpyAsync(dx.ptr, q.ptr, sizeof(double) * 6 * N, hipMemcpyDeviceToDevice, st));
+      retract(st);
+    }
     // done at the tolerance, after the last refinement, or when a refinement
     // no longer gains (the residual's own rounding)
-    const double tol = std::min(prm.pcg_rel_tol, kDirectTol);
-    if (last_residual <= tol || refine == kDirectRefine || last_residual > 0.25 * prev) {
-      *ok = true;
+    if (best <= tol || refine == kDirectRefine || !(residual <= 0.25 * before)) {
+      *ok = best <= std::max(prm.pcg_rel_tol, kDirectAccept);
       return RPGO_OK;
     }
-    prev = last_residual;
     if ((rc = direct_refine(st))) return rc;
     stats.pcg_iterations += 1;
   }
 }
 
 // One refinement of the accepted step that ends a nonlinear solve of a large
-// graph, its poses in xn and their cost
+// graph, its poses in xn and their cost; kept unless the cost is not finite or
+// rises by 1e-6 of itself.  (It moves the step by about 1e-4 of its length, and
+// the last step by default gains less than 1e-5 of the cost.)
 int SolverRun::direct_finish(hipStream_t st, double lambda, double* cost_new) {
   if (N < kDirectFinishMin) return RPGO_OK;
   int rc;
+  double cost = 0.0;
   if ((rc = direct_check(st, lambda))) return rc;  // the residual of the step in dx
   if ((rc = direct_refine(st))) return rc;
   stats.pcg_iterations += 1;
   retract(st);
-  return direct_cost(st, xn.as<double>(), cost_new);
+  if ((rc = direct_cost(st, xn.as<double>(), &cost))) return rc;
+  if (cost <= *cost_new * (1.0 + 1e-6)) {
+    *cost_new = cost;
+    return RPGO_OK;
+  }
+  RPGO_HIP_CHECK(hipMemcpyAsync(dx.ptr, q.ptr, sizeof(double) * 6 * N, hipMemcpyDeviceToDevice, st));
+  retract(st);
+  RPGO_HIP_CHECK(hipGetLastError());
+  return RPGO_OK;
 }
 
 // weighted cost at poses xp in one read-back (the reduction's other sums unused)

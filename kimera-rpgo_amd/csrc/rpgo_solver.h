@@ -20,6 +20,10 @@ constexpr int kCoarseMax = 6 * kCoarseSegMax;
 // stopped 1.4e-7 (relative) from the converged steps at 1e-6, 5e-9 at 1e-10.
 constexpr double kDirectTol = 1e-10;
 constexpr int kDirectRefine = 3;
+// and accepted at pcg_rel_tol or this, whichever is larger: the residual's own
+// rounding, which a refinement cannot lower, ends at 7e-10 on 18 drawn graphs
+// and at 4e-9 on chains held by a weak prior.  Above, the step is the PCG's.
+constexpr double kDirectAccept = 1e-8;
 // From this many poses the last step of a nonlinear solve gets one more
 // refinement.  The factor takes damping and diagonal rounded to one FP64
 // number, an error of about 1e-16 of the diagonal with the same sign at every
@@ -76,7 +80,6 @@ struct SolverRun {
   // copy, and the factor's storage
   bool direct_ready = false;
   DirectPlan plan;
-  double last_residual = 0.0;      // relative residual of the last direct solve
   DevBuf d_meta, d_childs, d_origs, d_rows, d_maps;
   DevBuf d_U, d_G, d_part, d_bad;
   // pinned host buffers of this run's readbacks (scalars; one PCG chunk's

@@ -29,11 +29,11 @@
 
 namespace rpgo {
 
-// A pivot this far below the pose's own Hessian diagonal is rounding noise of
-// a singular system (a graph without a prior under Gauss-Newton): the solve
-// is left to the PCG, which takes semidefinite systems.  The smallest pivots
-// of regular ones stay well above (about 1e-10 at the end of a 50,000-pose
-// chain).
+// A pivot this far below the pose's own Hessian diagonal is rounding: the
+// matrix is singular or indefinite to FP64 and the solve is left to the PCG.
+// The smallest pivots of regular systems are about 1e-10 (the end of a
+// 50,000-pose chain).  It does not tell a free graph: there the noise itself
+// reaches 1e-9, so an undamped step needs poses_held.
 constexpr double kPivotMin = 1e-13;
 
 __device__ __forceinline__ void load6(const double* __restrict__ s, double (&v)[6]) {
@@ -691,13 +691,37 @@ __global__ void k_direct_axpy(long long n, const double* __restrict__ a, double*
 // ------------------------------------------------------------------ host
 static_assert(panel_bytes(DirectLimits().max_d + 1, 1) <= kPanelBytes, "one pivot's panel in LDS");
 
-int SolverRun::direct_setup(hipStream_t st, const int32_t* h_kind, const int32_t* h_fi, const int32_t* h_fj) {
+// Whether the weights of this nonlinear solve hold every pose (*held: -1 until
+// it is known).  Factors whose weights do not change in a run are looked at once.
+int SolverRun::poses_held_now(hipStream_t st, const rpgo_solve_problem* pr, int* held) {
+  if (*held >= 0) return RPGO_OK;
+  if (held_always == 1) {
+    *held = 1;
+    return RPGO_OK;
+  }
+  std::vector<double> wt(F);
+  RPGO_HIP_CHECK(hipMemcpyAsync(wt.data(), w.ptr, sizeof(double) * F, hipMemcpyDeviceToHost, st));
+  RPGO_HIP_CHECK(hipStreamSynchronize(st));
+  const auto holds = [&](int f) {
+    if (!(wt[f] > kHoldWeight)) return false;
+    for (int e = 0; e < 36; e += 7)  // a factor of some directions only holds none
+      if (!(pr->information[36 * (size_t)f + e] > 0.0)) return false;
+    return true;
+  };
+  if (held_always < 0)
+    held_always = poses_held(N, F, pr->kind, pr->key_i, pr->key_j,
+                             [&](int f) { return (!prm.use_gnc || f < n_known) && holds(f); });
+  *held = held_always == 1 || poses_held(N, F, pr->kind, pr->key_i, pr->key_j, holds);
+  return RPGO_OK;
+}
+
+int SolverRun::direct_setup(hipStream_t st, const rpgo_solve_problem* pr) {
   direct_ready = false;
   // an explicit preconditioner choice asks for the PCG
-  if (prm.pcg_segment > 0 || prm.pcg_coarse != 0 || !h_kind || F <= 0) return RPGO_OK;
+  if (prm.pcg_segment > 0 || prm.pcg_coarse != 0 || F <= 0) return RPGO_OK;
   DirectPlan& P = plan;
   try {
-    if (!build_direct_plan(N, F, h_kind, h_fi, h_fj, DirectLimits(), P)) return RPGO_OK;
+    if (!build_direct_plan(N, F, pr->kind, pr->key_i, pr->key_j, DirectLimits(), P)) return RPGO_OK;
   } catch (const std::bad_alloc&) {
     return RPGO_OK;
   }
@@ -721,6 +745,7 @@ int SolverRun::direct_setup(hipStream_t st, const int32_t* h_kind, const int32_t
   for (int k = 0; k < 5; ++k)
     if (bytes[k]) RPGO_HIP_CHECK(hipMemcpyAsync(dst[k]->ptr, src[k], bytes[k], hipMemcpyHostToDevice, st));
   RPGO_HIP_CHECK(hipMemsetAsync(d_bad.ptr, 0, sizeof(int), st));
+  held_always = -1;
   direct_ready = true;
   return RPGO_OK;
 }

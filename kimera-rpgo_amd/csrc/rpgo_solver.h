@@ -31,6 +31,13 @@ constexpr double kDirectAccept = 1e-8;
 // 3e-8 of the poses when it is the last (earlier steps' errors are corrected
 // by the later ones).  Below, the bias is far under the solve's 1e-10.
 constexpr int kDirectFinishMin = 8192;
+// A factor below this weight does not hold a pose (poses_held): the noise of
+// singular systems reaches 1e-9 of the diagonal, a factor of 1e3 below.
+constexpr double kHoldWeight = 1e-6;
+// A step is undamped up to this lambda: lambda damp is lost in the FP64
+// diagonal (LM reaches 1e-20 to 1e-66 in GNC's later solves).  Down to 1e-15 a
+// free graph's direct and PCG steps move it alike, above 1e-16 within a third.
+constexpr double kUndamped = 1e-16;
 
 struct GraphKey {
   int N = 0, S = 0, Sc = 0, nseg_c = 0;
@@ -79,6 +86,7 @@ struct SolverRun {
   // direct solve (direct.hip): the plan of the current problem, its device
   // copy, and the factor's storage
   bool direct_ready = false;
+  int held_always = -1;            // every pose held whatever GNC's weights become (-1: not known)
   DirectPlan plan;
   DevBuf d_meta, d_childs, d_origs, d_rows, d_maps;
   DevBuf d_U, d_G, d_part, d_bad;
@@ -98,13 +106,14 @@ struct SolverRun {
   int model_decrease(hipStream_t st, double* out);
   int total_cost(hipStream_t st, const double* xp, double* out);
   int compute_errors(hipStream_t st, const double* xp);
-  int nonlinear_solve(hipStream_t st, bool from_x0, double* cost, int* iters);
+  int nonlinear_solve(hipStream_t st, const rpgo_solve_problem* pr, bool from_x0, double* cost, int* iters);
   int read_scalars(hipStream_t st, int count, double* out);
   double* pinned_scalars();
   double* pinned_history();
   void retract(hipStream_t st);
   void cost_partials(hipStream_t st, const double* xp, double* part);
-  int direct_setup(hipStream_t st, const int32_t* h_kind, const int32_t* h_fi, const int32_t* h_fj);
+  int direct_setup(hipStream_t st, const rpgo_solve_problem* pr);
+  int poses_held_now(hipStream_t st, const rpgo_solve_problem* pr, int* held);
   int direct_factor(hipStream_t st, double lambda);
   int direct_backward(hipStream_t st, double* out);
   int direct_check(hipStream_t st, double lambda);

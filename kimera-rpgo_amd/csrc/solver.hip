@@ -2239,7 +2239,8 @@ bool SolverRun::last_step(double cur, double nw, int it) const {
 
 // One LevenbergMarquardtOptimizer / GaussNewtonOptimizer run from x0 with the
 // current weights; leaves the result in x and its weighted cost in *cost_out.
-int SolverRun::nonlinear_solve(hipStream_t st, bool from_x0, double* cost_out, int* iters_out) {
+int SolverRun::nonlinear_solve(hipStream_t st, const rpgo_solve_problem* pr, bool from_x0, double* cost_out,
+                               int* iters_out) {
   int rc;
   if (from_x0) RPGO_HIP_CHECK(hipMemcpyAsync(x.ptr, x0.ptr, sizeof(double) * 12 * N, hipMemcpyDeviceToDevice, st));
   double err;
@@ -2247,13 +2248,26 @@ int SolverRun::nonlinear_solve(hipStream_t st, bool from_x0, double* cost_out, i
   double lambda = prm.lambda_initial;
   int it = 0;
   const bool gn = prm.solver == RPGO_SOLVER_GN;
+  // an undamped step is direct only where the weights hold every pose (so is one
+  // damped by lambda itself, which a large diagonal loses much earlier)
+  int held = -1;
+  const auto direct = [&](double lam, double* lin, double* nerr, bool* solved) -> int {
+    *solved = false;
+    if (!direct_ready) return RPGO_OK;
+    if (!(lam > kUndamped) || !prm.lm_diagonal_damping) {
+      int rh;
+      if ((rh = poses_held_now(st, pr, &held))) return rh;
+      if (!held) return RPGO_OK;
+    }
+    return direct_step(st, lam, lin, nerr, solved);
+  };
   while (it < prm.lm_max_iterations) {
     if ((rc = linearize(st))) return rc;
     if (gn) {
       int pit;
       double nerr, lin;
-      bool solved = false;
-      if (direct_ready && (rc = direct_step(st, 0.0, &lin, &nerr, &solved))) return rc;
+      bool solved;
+      if ((rc = direct(0.0, &lin, &nerr, &solved))) return rc;
       if (!solved) {
         if ((rc = pcg(st, 0.0, &pit))) return rc;
         retract(st);
@@ -2273,9 +2287,8 @@ int SolverRun::nonlinear_solve(hipStream_t st, bool from_x0, double* cost_out, i
     while (true) {
       int pit;
       double lin;
-      solved = false;
       lambda_step = lambda;
-      if (direct_ready && (rc = direct_step(st, lambda, &lin, &nerr, &solved))) return rc;
+      if ((rc = direct(lambda, &lin, &nerr, &solved))) return rc;
       if (!solved) {
         if ((rc = pcg(st, lambda, &pit))) return rc;
         if ((rc = model_decrease(st, &lin))) return rc;
@@ -2318,16 +2331,16 @@ int SolverRun::run(hipStream_t st, const rpgo_solve_problem* pr, rpgo_solve_repo
   int rc;
   stats = Stats{};
   if ((rc = build_incidence(st))) return rc;
-  if ((rc = direct_setup(st, pr->kind, pr->key_i, pr->key_j))) return rc;
+  if ((rc = direct_setup(st, pr))) return rc;
   int lm_it = 0;
   double cost = 0.0;
   int gnc_it = 0;
   double mu = -1.0;
   if (!prm.use_gnc) {
-    if ((rc = nonlinear_solve(st, true, &cost, &lm_it))) return rc;
+    if ((rc = nonlinear_solve(st, pr, true, &cost, &lm_it))) return rc;
   } else {
     // first solve with the initial weights (all 1 or bias_odom / caller weights)
-    if ((rc = nonlinear_solve(st, true, &cost, &lm_it))) return rc;
+    if ((rc = nonlinear_solve(st, pr, true, &cost, &lm_it))) return rc;
     if (prm.init_mu > 0.0) {
       mu = prm.init_mu;
     } else {
@@ -2357,7 +2370,7 @@ int SolverRun::run(hipStream_t st, const rpgo_solve_problem* pr, rpgo_solve_repo
                                                                 w.as<double>());
         RPGO_HIP_CHECK(hipGetLastError());
         int it2;
-        if ((rc = nonlinear_solve(st, !prm.gnc_warm_start, &cost, &it2))) return rc;
+        if ((rc = nonlinear_solve(st, pr, !prm.gnc_warm_start, &cost, &it2))) return rc;
         gnc_it = k + 1;
         RPGO_HIP_CHECK(hipMemsetAsync(sc.as<double>() + 24, 0, sizeof(double), st));
         k_weights_binary<<<grid_for(F, 256, 1 << 20), 256, 0, st>>>(
@@ -2383,7 +2396,7 @@ int SolverRun::run(hipStream_t st, const rpgo_solve_problem* pr, rpgo_solve_repo
     prm.pcg_rel_tol = std::min(prm.pcg_rel_tol, 1e-6);
     int it3;
     polish = true;
-    rc = nonlinear_solve(st, false, &cost, &it3);
+    rc = nonlinear_solve(st, pr, false, &cost, &it3);
     polish = false;
     prm = saved;
     if (rc) return rc;

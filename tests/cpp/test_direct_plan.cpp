@@ -324,6 +324,37 @@ TEST(DirectPlan, LongLists) {
   }
 }
 
+TEST(DirectPlan, PosesHeld) {
+  // a chain 0-1-2, a pair 3-4, poses 5 (prior) and 6 alone; factor 7 joins 4 to 2
+  const std::vector<int32_t> kind = {0, 0, 0, 1, 1, 1, 1, 0}, fi = {0, 2, 3, 1, 5, 4, 6, 4}, fj = {1, 1, 4, 1, 5, 4, 6, 2};
+  const auto held = [&](std::vector<int> off) {
+    return poses_held(7, 8, kind.data(), fi.data(), fj.data(),
+                      [&](int f) { return std::find(off.begin(), off.end(), f) == off.end(); });
+  };
+  EXPECT(held({}));
+  EXPECT(!held({6}));      // pose 6 without its prior
+  EXPECT(!held({4}));
+  EXPECT(held({3}));       // the chain by factor 7
+  EXPECT(held({5}));       // the pair by factor 7
+  EXPECT(held({7}));
+  EXPECT(!held({3, 7}));   // the chain by nothing
+  EXPECT(!held({5, 7}));
+  EXPECT(!held({0}));      // pose 0 cut off
+  EXPECT(!held({2, 5}));   // pose 3 cut off
+  const int32_t none = 0;
+  EXPECT(!poses_held(1, 0, &none, &none, &none, [](int) { return true; }));
+  std::vector<int32_t> k(50000, 0), i(50000), j(50000);  // a long chain in order and reversed, prior last
+  for (int f = 0; f < 49999; ++f) i[f] = f, j[f] = f + 1;
+  k[49999] = 1, i[49999] = j[49999] = 49999;
+  EXPECT(poses_held(50000, 50000, k.data(), i.data(), j.data(), [](int) { return true; }));
+  EXPECT(!poses_held(50000, 50000, k.data(), i.data(), j.data(), [](int f) { return f != 777; }));
+  EXPECT(!poses_held(50000, 50000, k.data(), i.data(), j.data(), [](int f) { return f != 49999; }));
+  std::reverse(i.begin(), i.end() - 1);
+  std::reverse(j.begin(), j.end() - 1);
+  EXPECT(poses_held(50000, 50000, k.data(), j.data(), i.data(), [](int) { return true; }));
+  EXPECT(!poses_held(50000, 50000, k.data(), j.data(), i.data(), [](int f) { return f != 49999; }));
+}
+
 TEST(DirectPlan, Limits) {
   std::vector<std::pair<int, int>> clique;
   for (int a = 0; a < 20; ++a)

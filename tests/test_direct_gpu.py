@@ -202,3 +202,49 @@ def test_residual_decides(ctx, n, stiff, direct):
     print(f"[direct] weakly held {n} {stiff:.0e}: {ra.pcg_iterations} at 1e-6, {rb.pcg_iterations} at 1e-2", flush=True)
     assert np.isfinite(a).all() and rb.pcg_iterations <= 4
     assert (ra.pcg_iterations <= 4) == direct
+
+
+@pytest.mark.parametrize("n, n_lc", [(1000, 0), (1000, 100), (20000, 0), (20000, 2000)])
+def test_free_graph_undamped(ctx, n, n_lc):
+    """Gauss-Newton without a prior: the matrix is singular and its last pivots
+    are noise of either sign, up to 2e-10 of the diagonal at 20,000 poses, so
+    the step is the PCG's without a factorization (its iterations come in
+    eights; a factorization would count one more).  LM whose lambda is lost in
+    the diagonal starts with the PCG too, and never raises the cost."""
+    gr = synth.se3_helix(n_poses=n, n_lc=max(n_lc, 2), outlier_frac=0.0, seed=3)
+    a = problem.solve_arrays(gr, lc_idx=np.arange(n_lc))
+    keep = a[1] == 0
+    g = [a[0]] + [v[keep] for v in a[1:6]]
+    g[0], _, r0 = ctx.solve(*g)
+    assert r0.pcg_iterations <= 4 * (r0.linearizations + 1)  # damped: direct
+    x, _, r = ctx.solve(*g, solver=_capi.SOLVER_GN, lm_max_iterations=1)
+    print(f"[direct] free {n} {n_lc}: {r.pcg_iterations} cost {r0.final_cost:.10g} {r.final_cost:.10g}", flush=True)
+    assert r.pcg_iterations > 0 and r.pcg_iterations % 8 == 0
+    assert np.isfinite(x).all()
+    x, _, r = ctx.solve(*g, lambda_initial=1e-20, lm_max_iterations=1, lm_relative_error_tol=1e-30)
+    assert r.pcg_iterations >= 8 and np.isfinite(x).all() and r.final_cost <= r0.final_cost * (1 + 1e-9)
+    # lambda added as it is (not times the diagonal): the PCG; direct with a prior
+    for damped in (g, a[:6]):
+        x, _, r = ctx.solve(*damped, lm_diagonal_damping=0, lm_max_iterations=1)
+        assert (r.pcg_iterations % 8 == 0) == (damped is g) and np.isfinite(x).all()
+
+
+@pytest.mark.parametrize("use_gnc", [0, 1])
+def test_zero_weight_frees_a_part(ctx, use_gnc):
+    """Two chains, a prior on the first only, joined by one factor: while its
+    weight holds the second chain the Gauss-Newton steps are direct, at weight
+    0 (GNC's initial weights here) they are the PCG's."""
+    edges = [(k, k + 1) for k in range(59) if k != 29] + [(0, 20), (5, 25), (30, 50), (35, 55), (10, 40)]
+    poses, kind, ki, kj, meas, info = _graph(60, edges, 4)
+    link = (kind == 0) & (ki == 10) & (kj == 40)
+    order = np.argsort(link, kind="stable")  # the link last, all others known
+    g = (poses,) + tuple(np.ascontiguousarray(v[order]) for v in (kind, ki, kj, meas, info))
+    kw = dict(solver=_capi.SOLVER_GN, use_gnc=use_gnc, known_inliers=len(kind) - 1 if use_gnc else 0,
+              gnc_max_iterations=0)
+    its = {}
+    for w in (1.0, 1e-3, 0.0):
+        x, _, r = ctx.solve(*g, init_weights=np.r_[np.ones(len(kind) - 1), w], **kw)
+        its[w] = r.pcg_iterations
+        assert np.isfinite(x).all()
+        assert (r.pcg_iterations <= 4 * r.linearizations) == (w > 0.0)
+    print(f"[direct] freed part: {its}", flush=True)

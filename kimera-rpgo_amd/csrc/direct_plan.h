@@ -89,6 +89,7 @@ struct DirectPlan {
   int N = 0;
   int max_d = 0;                    // neighbours of the widest pivot
   int64_t u_len = 0, g_len = 0;     // doubles of all update matrices and panels
+  int64_t steps = 0;                // list entries touched while eliminating, also when refused
   std::vector<int> lvl;             // level offsets into meta
   std::vector<int> lvl_bytes;       // largest panel_bytes of each level
   std::vector<int> lvl_back;        // largest back_bytes
@@ -222,7 +223,8 @@ inline bool build_direct_plan(int N, int F, const int32_t* kind, const int32_t* 
   order.reserve(N);
   std::vector<int32_t> mark(N, -1), elim(N, -1), seen(N, -1), stamp(N, -1), tmp, longs;
   std::vector<int32_t> bucket_off, cand;
-  int64_t steps = 0, u_len = 0;
+  int64_t& steps = P.steps;
+  int64_t u_len = 0;
   int thin_levels = 0;
   int32_t gen = -1;
   const int64_t max_u = std::min(lim.max_u, std::max(lim.u_free, lim.max_u_pose * N));
@@ -230,15 +232,20 @@ inline bool build_direct_plan(int N, int F, const int32_t* kind, const int32_t* 
     if (level >= lim.max_levels) return false;
     int dmin = A.len[alive[0]];
     size_t chain_poses = 0;
+    int64_t degrees = 0;
     for (int v : alive) {
       dmin = std::min(dmin, (int)A.len[v]);
+      degrees += A.len[v];
       chain_poses += A.len[v] <= 2;
     }
     const bool thin = dmin <= 2 && 8 * chain_poses < alive.size();
     thin_levels += thin;
-    // the fill still to come is more than a quarter of what the remaining
-    // poses' present degree would make: give up early when that is too much
-    if (u_len + (int64_t)(alive.size() / 4) * front_update_len(dmin) > max_u) return false;
+    // The update matrices still to come are more than a fifth of one of the mean
+    // degree for every remaining pose (a clique of them makes a third, accepted
+    // graphs 0.29 and more): give up early when that is too much.  With the
+    // smallest degree in its place 50,000 poses with outliers were refused after
+    // twice the list entries.
+    if (u_len + (int64_t)(alive.size() / 5) * front_update_len(degrees / (int64_t)alive.size()) > max_u) return false;
     const int thr = dmin <= 2 && !(thin && thin_levels > kThinLevels) ? 2 : std::max(3 * dmin, dmin + 4);
     // candidates by degree, then index (counting sort)
     bucket_off.assign(thr + 2, 0);

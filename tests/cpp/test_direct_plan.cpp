@@ -324,6 +324,21 @@ TEST(DirectPlan, LongLists) {
   }
 }
 
+// A graph that fills in too much is given up early: random loop closures on a
+// fifth of the poses of a chain end in one clique of several hundred
+TEST(DirectPlan, RefusedEarly) {
+  std::mt19937 rng(3);
+  auto e = chain(20000);
+  for (int k = 0; k < 4000; ++k) {
+    const int a = (int)(rng() % 20000), b = (int)(rng() % 20000);
+    if (a != b) e.push_back({a, b});
+  }
+  DirectPlan P;
+  EXPECT(!plan(20000, e, DirectLimits(), P));
+  std::printf("  refused after %lld list entries\n", (long long)P.steps);
+  EXPECT(P.steps < 100 * 20000);  // 81 a pose; 140 with the smallest degree as the estimate
+}
+
 TEST(DirectPlan, PosesHeld) {
   // a chain 0-1-2, a pair 3-4, poses 5 (prior) and 6 alone; factor 7 joins 4 to 2
   const std::vector<int32_t> kind = {0, 0, 0, 1, 1, 1, 1, 0}, fi = {0, 2, 3, 1, 5, 4, 6, 4}, fj = {1, 1, 4, 1, 5, 4, 6, 2};

@@ -2251,15 +2251,21 @@ int SolverRun::nonlinear_solve(hipStream_t st, const rpgo_solve_problem* pr, boo
   // an undamped step is direct only where the weights hold every pose (so is one
   // damped by lambda itself, which a large diagonal loses much earlier)
   int held = -1;
+  // the largest lambda whose factorization was no use: a matrix that is singular
+  // or too ill-scaled for FP64 is no better with less damping, at the next
+  // linearization either
+  double failed = -1.0;
   const auto direct = [&](double lam, double* lin, double* nerr, bool* solved) -> int {
     *solved = false;
-    if (!direct_ready) return RPGO_OK;
+    if (!direct_ready || lam <= failed) return RPGO_OK;
     if (!(lam > kUndamped) || !prm.lm_diagonal_damping) {
       int rh;
       if ((rh = poses_held_now(st, pr, &held))) return rh;
       if (!held) return RPGO_OK;
     }
-    return direct_step(st, lam, lin, nerr, solved);
+    const int rd = direct_step(st, lam, lin, nerr, solved);
+    if (!*solved) failed = lam;
+    return rd;
   };
   while (it < prm.lm_max_iterations) {
     if ((rc = linearize(st))) return rc;

@@ -248,3 +248,14 @@ def test_zero_weight_frees_a_part(ctx, use_gnc):
         assert np.isfinite(x).all()
         assert (r.pcg_iterations <= 4 * r.linearizations) == (w > 0.0)
     print(f"[direct] freed part: {its}", flush=True)
+
+
+def test_failed_factorization_is_remembered(ctx):
+    """A Gauss-Newton matrix that is singular to FP64 (a prior of 1e-2 under a
+    chain of 1e10) is factored once, not at every step; the PCG's iterations
+    come in eights."""
+    g = _weakly_held(20, 1e10)
+    _, _, r = ctx.solve(*g, solver=_capi.SOLVER_GN, lm_relative_error_tol=0.0, lm_absolute_error_tol=0.0,
+                        lm_max_iterations=3)
+    print(f"[direct] singular: {r.linearizations} linearizations, {r.pcg_iterations} iterations", flush=True)
+    assert r.linearizations == 3 and r.pcg_iterations > 8 and r.pcg_iterations % 8 == 1

@@ -593,6 +593,9 @@ __global__ void __launch_bounds__(256) k_icc_compact(int n, int pos, int best, c
 // (replay_walk).  Exit steps come from one pass over the picks' rows, sizes
 // from their histogram, and every step writes its positions by itself.  The
 // sequential replay of a 4,816-vertex clique took 1.9 ms on one wavefront.
+// The number of picks listed must be the greedy size less one, K, and S_0 must
+// be empty after them; otherwise nothing is read from the list and the size
+// reported is -1.
 // ---------------------------------------------------------------------------
 // Vertices from which this replaces replay_walk: five launches of about 5 us
 // against 48 us for the step-by-step replay at 400 vertices, 7 us at 75
@@ -641,11 +644,12 @@ __global__ void k_rp_init(int n, int* __restrict__ exit_step, int* __restrict__ 
 
 // one wavefront per (word w, 64 picks): for every vertex of S_0's word w the
 // first of these picks whose row lacks it
-__global__ void __launch_bounds__(256) k_rp_exit(int n, int W, int c, int K, const unsigned long long* __restrict__ adj,
+__global__ void __launch_bounds__(256) k_rp_exit(int W, int c, int K, const unsigned long long* __restrict__ adj,
                                                  const unsigned long long* __restrict__ dmask,
-                                                 const int* __restrict__ list, int* __restrict__ exit_step) {
+                                                 const int* __restrict__ list, const int* __restrict__ count,
+                                                 int* __restrict__ exit_step) {
   const int w = blockIdx.x, j = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (64 * j >= K) return;
+  if (64 * j >= K || *count != K) return;
   const unsigned long long s0 = replay_start_word(c, w, W, adj, dmask);
   if (!s0) return;
   const int t = 64 * j + lane;
@@ -662,22 +666,21 @@ __global__ void __launch_bounds__(256) k_rp_exit(int n, int W, int c, int K, con
     if (lane == b && z) first = __builtin_ctzll(z);
   }
   if (((s0 >> lane) & 1ull) && first < 64) atomicMin(&exit_step[64 * w + lane], 64 * j + first);
-  (void)n;
 }
 
+// vertices per exit step; hist[K]: those still there after the last pick
 __global__ void k_rp_hist(int n, int W, int c, int K, const unsigned long long* __restrict__ adj,
                           const unsigned long long* __restrict__ dmask, const int* __restrict__ exit_step,
                           int* __restrict__ hist) {
   const int u = blockIdx.x * blockDim.x + threadIdx.x;
   if (u >= n || !((replay_start_word(c, u >> 6, W, adj, dmask) >> (u & 63)) & 1ull)) return;
-  const int e = exit_step[u];
-  if (e < K) atomicAdd(&hist[e], 1);
+  atomicAdd(&hist[min(exit_step[u], K)], 1);
 }
 
 // sizes: sz[t] = s_t for t = 0 .. K, from s_K = 1 up; res[0] = greedy size,
 // res[1] = s_0.  One workgroup.
-__global__ void __launch_bounds__(1024) k_rp_sizes(int K, const int* __restrict__ hist, int* __restrict__ sz,
-                                                   int* __restrict__ res) {
+__global__ void __launch_bounds__(1024) k_rp_sizes(int K, const int* __restrict__ hist, const int* __restrict__ count,
+                                                   int* __restrict__ sz, int* __restrict__ res) {
   __shared__ int sum[16];
   __shared__ int base;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
@@ -703,7 +706,7 @@ __global__ void __launch_bounds__(1024) k_rp_sizes(int K, const int* __restrict_
     __syncthreads();
   }
   if (tid == 0) {
-    res[0] = K + 1;
+    res[0] = *count == K && hist[K] == 0 ? K + 1 : -1;
     res[1] = base;
   }
 }
@@ -713,11 +716,12 @@ __global__ void __launch_bounds__(1024) k_rp_sizes(int K, const int* __restrict_
 __global__ void __launch_bounds__(256) k_rp_write(int n, int W, int c, int K,
                                                   const unsigned long long* __restrict__ adj,
                                                   const unsigned long long* __restrict__ dmask,
-                                                  const int* __restrict__ list, const int* __restrict__ exit_step,
-                                                  const int* __restrict__ sz, int* __restrict__ out) {
+                                                  const int* __restrict__ list, const int* __restrict__ count,
+                                                  const int* __restrict__ exit_step, const int* __restrict__ sz,
+                                                  int* __restrict__ out) {
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (blockIdx.x == 0 && threadIdx.x == 0) out[0] = c;
-  if (t >= K) return;
+  if (t >= K || *count != K) return;
   int p = sz[t] - 1;
   const int lo = sz[t + 1];
   for (int w = list[t] >> 6; w >= 0 && p >= lo; --w) {
@@ -1345,14 +1349,12 @@ static int clique_scan(rpgo_ctx* ctx, const uint64_t* d_adj_u64, int n, int mode
     k_dmask<<<(W + 255) / 256, 256, 0, st>>>(n, W, win_best, b.deg, b.dmask, nullptr);
     if (par) {
       const int K = best - 1;  // picks
-      int *list = b.replay, *ex = list + n + 1, *hist = ex + n, *sz = hist + n + 1;
+      int *list = b.replay, *count = list + n, *ex = count + 1, *hist = ex + n, *sz = hist + n + 1;
       k_rp_init<<<(n + 256) / 256, 256, 0, st>>>(n, ex, hist);
-      if (K > 0) {
-        k_rp_exit<<<dim3(W, (K + 255) / 256), 256, 0, st>>>(n, W, win, K, adj, b.dmask, list, ex);
-        k_rp_hist<<<(n + 255) / 256, 256, 0, st>>>(n, W, win, K, adj, b.dmask, ex, hist);
-      }
-      k_rp_sizes<<<1, 1024, 0, st>>>(K, hist, sz, d_res);
-      k_rp_write<<<std::max(1, (K + 3) / 4), 256, 0, st>>>(n, W, win, K, adj, b.dmask, list, ex, sz, b.out);
+      if (K > 0) k_rp_exit<<<dim3(W, (K + 255) / 256), 256, 0, st>>>(W, win, K, adj, b.dmask, list, count, ex);
+      k_rp_hist<<<(n + 255) / 256, 256, 0, st>>>(n, W, win, K, adj, b.dmask, ex, hist);
+      k_rp_sizes<<<1, 1024, 0, st>>>(K, hist, count, sz, d_res);
+      k_rp_write<<<std::max(1, (K + 3) / 4), 256, 0, st>>>(n, W, win, K, adj, b.dmask, list, count, ex, sz, b.out);
     } else {
       k_replay<<<1, 64, 0, st>>>(n, W, win, win_best, adj, b.dmask, b.out, d_res);
     }

@@ -164,7 +164,7 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 
 // Where element (row ri, scalar column ci) of the panel stands, less 6 ri
 __device__ __forceinline__ int panel_col(int n, int ci) {
-  const int q = (ci * 43691) >> 18;  // ci / 6, exact below 1 << 16
+  const int q = (ci * 43691) >> 18;  // ci / 6, exact below 49,152
   return 6 * (__mul24(6 * q, n) - 3 * __mul24(q, q - 1) - 5 * q) + ci - 6 * q;
 }
 
@@ -690,6 +690,7 @@ __global__ void k_direct_axpy(long long n, const double* __restrict__ a, double*
 
 // ------------------------------------------------------------------ host
 static_assert(panel_bytes(DirectLimits().max_d + 1, 1) <= kPanelBytes, "one pivot's panel in LDS");
+static_assert(6 * (DirectLimits().max_d + 1) + 16 < 49152, "panel_col's division by six");
 
 // Whether the weights of this nonlinear solve hold every pose (*held: -1 until
 // it is known).  Factors whose weights do not change in a run are looked at once.

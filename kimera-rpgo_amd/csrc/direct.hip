@@ -751,11 +751,6 @@ int SolverRun::direct_setup(hipStream_t st, const rpgo_solve_problem* pr) {
   return RPGO_OK;
 }
 
-// Where every front of the level is small its update rows go to single lanes:
-// a tile of 16x16 is larger than the whole update below three neighbours, and
-// at n = 8 both take 8 us
-static bool small_level(const DirectPlan& P, int l) { return P.lvl_n[l] <= 8; }
-
 // Factor H + lambda damp and substitute forward with b: one launch per level.
 int SolverRun::direct_factor(hipStream_t st, double lambda) {
   const DirectPlan& P = plan;
@@ -766,22 +761,12 @@ int SolverRun::direct_factor(hipStream_t st, double lambda) {
   first, d_meta.as<FrontMeta>(), d_childs.as<FrontChild>(), d_origs.as<FrontOrig>(), d_maps.as<int>(),           \
       d_rows.as<int>(), D.as<double>(), hdiag.as<double>(), b64.as<double>(), Hij.as<double>(), lambda,          \
       prm.lm_diagonal_damping, d_U.as<double>(), d_G.as<double>(), d_bad.as<int>()
-    if (small_level(P, l)) {
-      // a wavefront a front where the level fills the chip by itself: 22,520
-      // fronts 50 us; four wavefronts run a front's three chains of loads side
-      // by side: levels of 100 to 600 fronts 11 -> 7.8 us
-      if (n > 4096) k_front_small<64><<<n, 64, lds, st>>>(RPGO_FRONT_ARGS);
-      else k_front_small<256><<<n, 256, lds, st>>>(RPGO_FRONT_ARGS);
-    } else {
-      // wide fronts of a narrow level share their update tiles among
-      // workgroups, each repeating the panel
-      const int T = (6 * P.lvl_d[l] + 16) / 16, tiles = T * (T + 1) / 2;
-      const auto split = [&](int waves) { return std::max(1, std::min((tiles + waves - 1) / waves, 1024 / n)); };
-      // sixteen wavefronts for the pivots' latency, four where fronts
-      // outnumber half the CUs: levels of 207 to 1,166 fronts 28-45 -> 20-26 us
-      if (n > 128) k_front<256><<<dim3(n, split(4)), 256, lds, st>>>(RPGO_FRONT_ARGS);
-      else k_front<1024><<<dim3(n, split(16)), 1024, lds, st>>>(RPGO_FRONT_ARGS);
-    }
+    const LevelLaunch how = level_launch(P, l);
+    const dim3 grid(n, how.split);
+    if (how.small && how.threads == 64) k_front_small<64><<<grid, 64, lds, st>>>(RPGO_FRONT_ARGS);
+    else if (how.small) k_front_small<256><<<grid, 256, lds, st>>>(RPGO_FRONT_ARGS);
+    else if (how.threads == 256) k_front<256><<<grid, 256, lds, st>>>(RPGO_FRONT_ARGS);
+    else k_front<1024><<<grid, 1024, lds, st>>>(RPGO_FRONT_ARGS);
 #undef RPGO_FRONT_ARGS
   }
   RPGO_HIP_CHECK(hipGetLastError());
@@ -793,7 +778,7 @@ int SolverRun::direct_backward(hipStream_t st, double* out) {
   for (int l = P.levels() - 1; l >= 0; --l) {
     const int first = P.lvl[l], n = P.lvl[l + 1] - first;
     const size_t lds = (size_t)P.lvl_back[l];
-    if (small_level(P, l))
+    if (level_launch(P, l).small)
       k_back<64><<<n, 64, lds, st>>>(first, d_meta.as<FrontMeta>(), d_rows.as<int>(), d_G.as<double>(), out);
     else
       k_back<256><<<n, 256, lds, st>>>(first, d_meta.as<FrontMeta>(), d_rows.as<int>(), d_G.as<double>(), out);
@@ -822,7 +807,7 @@ int SolverRun::direct_refine(hipStream_t st) {
 #define RPGO_FORWARD_ARGS                                                                                     \
   first, d_meta.as<FrontMeta>(), d_childs.as<FrontChild>(), d_maps.as<int>(), d_rows.as<int>(), r.as<double>(), \
       d_G.as<double>(), d_U.as<double>()
-    if (small_level(P, l)) k_front_forward<64><<<n, 64, lds, st>>>(RPGO_FORWARD_ARGS);
+    if (level_launch(P, l).small) k_front_forward<64><<<n, 64, lds, st>>>(RPGO_FORWARD_ARGS);
     else k_front_forward<256><<<n, 256, lds, st>>>(RPGO_FORWARD_ARGS);
 #undef RPGO_FORWARD_ARGS
   }

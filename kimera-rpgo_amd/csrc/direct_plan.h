@@ -102,6 +102,30 @@ struct DirectPlan {
   int levels() const { return (int)lvl.size() - 1; }
 };
 
+// How a level is launched: workgroups of `threads` threads, `split` of them for
+// each front.
+//
+// Where every front of the level is small its update rows go to single lanes: a
+// tile of 16x16 is larger than the whole update below three neighbours, and at
+// n = 8 both take 8 us.  A wavefront a front where the level fills the chip by
+// itself: 22,520 fronts 50 us; four wavefronts run a front's three chains of
+// loads side by side: levels of 100 to 600 fronts 11 -> 7.8 us.
+//
+// Wide fronts of a narrow level share their update tiles among workgroups, each
+// repeating the panel.  Sixteen wavefronts for the pivots' latency, four where
+// fronts outnumber half the CUs: levels of 207 to 1,166 fronts 28-45 -> 20-26 us.
+struct LevelLaunch {
+  bool small;
+  int threads, split;
+};
+
+inline LevelLaunch level_launch(const DirectPlan& P, int l) {
+  const int n = P.lvl[l + 1] - P.lvl[l];
+  if (P.lvl_n[l] <= 8) return {true, n > 4096 ? 64 : 256, 1};
+  const int T = (6 * P.lvl_d[l] + 16) / 16, tiles = T * (T + 1) / 2, waves = n > 128 ? 4 : 16;
+  return {false, 64 * waves, std::max(1, std::min((tiles + waves - 1) / waves, 1024 / n))};
+}
+
 // Limits of a plan: past any of them build_direct_plan returns false and the
 // caller keeps its iterative solve.  Where the line lies: loop closures
 // between random poses (outliers left in the graph) end in one wide clique,

@@ -217,6 +217,13 @@ std::vector<std::pair<int, int>> chain_hub(int N, int seen) {
   return e;
 }
 
+// laps of `lap` poses, joined at every `every`th pose
+std::vector<std::pair<int, int>> laps(int N, int lap, int every) {
+  auto e = chain(N);
+  for (int k = 0; k + lap < N; k += every) e.push_back({k + lap, k});
+  return e;
+}
+
 bool plan(int N, const std::vector<std::pair<int, int>>& edges, const DirectLimits& lim, DirectPlan& P) {
   std::vector<int32_t> kind(edges.size(), 0), fi, fj;
   for (auto& e : edges) {
@@ -271,9 +278,7 @@ TEST(DirectPlan, Shapes) {
   EXPECT(check("clique", 45, clique, 6, rpgo_failures_) > 1);
   check("two chains", 41, two, 3, rpgo_failures_);
   check("no factors", 5, none, 4, rpgo_failures_);
-  auto ladder = chain(120);  // laps of 12 poses, joined at every third pose
-  for (int k = 0; k + 12 < 120; k += 3) ladder.push_back({k + 12, k});
-  check("laps", 120, ladder, 5, rpgo_failures_);
+  check("laps", 120, laps(120, 12, 3), 5, rpgo_failures_);
 }
 
 // Poses around one shared pose: the levels stay logarithmic in the chain (a fan
@@ -322,6 +327,23 @@ TEST(DirectPlan, LongLists) {
     EXPECT(plan(121, hub, lim, A) && plan(121, hub, DirectLimits(), B));
     EXPECT(A.row_pose == B.row_pose && A.maps == B.maps && A.lvl == B.lvl && A.u_len == B.u_len);
   }
+}
+
+// The graph that test_direct_gpu.py solves to run every launch of the front
+// kernels has levels of each kind
+TEST(DirectPlan, LaunchShapes) {
+  DirectPlan P;
+  EXPECT(plan(20000, laps(20000, 100, 5), DirectLimits(), P));
+  int small64 = 0, small256 = 0, front256 = 0, front1024 = 0, split256 = 0, split1024 = 0;
+  for (int l = 0; l < P.levels(); ++l) {
+    const LevelLaunch h = level_launch(P, l);
+    EXPECT(h.split >= 1 && (!h.small || h.split == 1));
+    ++(h.small ? (h.threads == 64 ? small64 : small256) : h.threads == 256 ? front256 : front1024);
+    if (!h.small && h.split > 1) ++(h.threads == 256 ? split256 : split1024);
+    std::printf("  %d fronts of up to %d rows, %d neighbours: %s%d x%d\n", P.lvl[l + 1] - P.lvl[l], P.lvl_n[l],
+                P.lvl_d[l], h.small ? "small " : "", h.threads, h.split);
+  }
+  EXPECT(small64 > 0 && small256 > 0 && front256 > 0 && front1024 > 0 && split256 > 0 && split1024 > 0);
 }
 
 // A graph that fills in too much is given up early: random loop closures on a

@@ -1,9 +1,10 @@
 """The direct linear solve (multifrontal block Cholesky, the default) against
 the PCG (an explicit pcg_segment) on the graph shapes its elimination plan can
-meet: single poses, chains, reversed and repeated factors, stars, several
-components, cliques wide enough for every launch shape of the front kernel
-(64 and 256 threads, split update rows), and the graphs it
-declines (too wide, singular), which run the PCG either way.
+meet: single poses, chains, reversed and repeated factors, stars, hubs, several
+components, cliques, and the graphs it declines (too wide, singular), which run
+the PCG either way.  The 20,000-pose laps have levels of every launch shape (fronts
+of up to 8 rows with 64 and 256 threads, wider ones with 256 and 1,024, one or
+more workgroups a front); the plan's test checks that they do.
 
 Bar: the same iteration counts and poses within 1e-6 m.  Both solve each step
 to at most 1e-9 (PCG) and 1e-10 (direct) of its right-hand side; the graphs'
@@ -82,6 +83,11 @@ def _chain_hub(n, seen):
     return n + 1, _chain(n) + [(k * n // seen, n) for k in range(seen)]
 
 
+def _laps(n, lap, every):
+    """Laps of `lap` poses, joined at every `every`th pose."""
+    return _chain(n) + [(k + lap, k) for k in range(0, n - lap, every)]
+
+
 CASES = {
     "one_pose": (1, [], (0,)),
     "two_poses": (2, [(1, 0)], (1,)),
@@ -93,6 +99,7 @@ CASES = {
     "hub_60_of_200": (*_chain_hub(200, 60), (0,)),
     "hub_300_of_300": (*_chain_hub(300, 300), (0,)),
     "two_components": (41, _chain(20) + [(k, k + 1) for k in range(20, 40)] + [(3, 15)], (0, 20)),
+    "laps_20000": (20000, _laps(20000, 100, 5), (0,)),
     "clique_6": (6, _clique(6), (0,)),
     "clique_11": (11, _flip(_clique(11), 5), (0,)),
     "clique_40": (40, _flip(_clique(40), 6), (0,)),

@@ -113,11 +113,6 @@ __device__ __forceinline__ void p32_from64(const double* p, P32& o) {
   o.t[0] = (float)p[9]; o.t[1] = (float)p[10]; o.t[2] = (float)p[11];
 }
 
-__device__ __forceinline__ void add36(double* acc, const double* x) {
-#pragma unroll
-  for (int e = 0; e < 36; ++e) acc[e] += x[e];
-}
-
 // ---------------------------------------------------------------------------
 // precompute
 // ---------------------------------------------------------------------------

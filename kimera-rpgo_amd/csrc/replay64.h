@@ -188,7 +188,7 @@ struct R64<3> {
     for (int e = 0; e < 9; ++e) o[e] = R[e];
     o[9] = t0; o[10] = t1; o[11] = t2;
   }
-  // entry e of a*b (used by the lane-parallel fold)
+  // entry e of a*b (a lane per entry)
   __device__ static __forceinline__ double compose_entry(const double* a, const double* b, int e) {
     if (e < 9) {
       const int r = e / 3, c = e % 3;
@@ -319,11 +319,6 @@ struct R64<2> {
     const double ry = a[1] * b[2] + a[0] * b[3];
     o[0] = c; o[1] = s;
     o[2] = a[2] + rx; o[3] = a[3] + ry;
-  }
-  __device__ static __forceinline__ double compose_entry(const double* a, const double* b, int e) {
-    double o[4];
-    pose_compose(a, b, o);
-    return o[e];
   }
   __device__ static __forceinline__ void pose_inverse(const double* a, double* o) {
     const double c = a[0], s = a[1];

@@ -328,10 +328,11 @@ int rpgo_pcm_batch_download_adj(rpgo_ctx* ctx, int32_t g, uint64_t* adj_bits);
 /* ------------------------------------------------------------------------
  * Robust solve: GNC-TLS over Levenberg-Marquardt / Gauss-Newton.  The linear
  * step is a sparse block Cholesky solve in FP64 (the reference's own kind of
- * step); graphs whose elimination fills in too much, singular systems and
- * calls that choose a preconditioner (pcg_segment > 0 or pcg_coarse != 0) take
- * a PCG (block-tridiagonal segment preconditioner along the odometry chain
- * plus a rigid-segment coarse level).  Replaces RobustSolver::optimize
+ * step); graphs whose elimination fills in too much, singular or too
+ * ill-scaled systems (residual above pcg_rel_tol), undamped steps of graphs
+ * that no prior holds and calls that choose a preconditioner (pcg_segment > 0
+ * or pcg_coarse != 0) take a PCG (block-tridiagonal segment preconditioner
+ * along the odometry chain plus a rigid-segment coarse level).  Replaces RobustSolver::optimize
  * (src/RobustSolver.cpp:115-306): gtsam::GncOptimizer with known inliers
  * (:105-113, :130-180, :225-275) or plain LevenbergMarquardtOptimizer /
  * GaussNewtonOptimizer (:181-218, :276-296).  SE(3) poses only.

@@ -15,11 +15,11 @@
 // Why not more PCG: the two-level PCG takes 300 to 900 iterations per linear
 // step on dead-reckoned helices (condition number 4e10 at 50,000 poses), each
 // four dependent launches.  The whole factorization is about 0.2 GFLOP and
-// 270 MB there; what bounds it is the chain of dependent levels (83 at 50,000
-// poses with 5,000 loop closures), each about as long as one PCG launch.
-// LM at 50,000 poses 814 -> 44 ms, GNC at 3,000 poses 1,639 -> 294 ms, planar
-// GNC at 500 poses 776 -> 70 ms, eight GNC solves of 200-2,000 poses on four
-// lanes 1,710 -> 229 ms (PCG -> this, wall time of the call).
+// 270 MB there; what bounds it is the chain of dependent levels, 23 to 25 at
+// 50,000 poses with 5,000 loop closures, each 22 to 38 us forward and 9 back.
+// PCG -> this, wall time of the call, on one box: LM at 50,000 poses 698 -> 54
+// ms, GNC at 3,000 poses 1,272 -> 225 ms, planar GNC at 500 poses 674 -> 68 ms,
+// eight GNC solves of 200-2,000 poses on four lanes 1,747 -> 228 ms.
 #include <cmath>
 #include <new>
 

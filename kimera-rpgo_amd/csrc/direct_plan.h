@@ -18,8 +18,8 @@
 // their plans do not change.)  The exact minimum degree
 // (threshold dmin) gives the least fill but, once the graph is a strip of
 // cliques, eats it from its ends in long dependent chains: on a helix of
-// 50,000 poses with 5,000 loop closures 1,148 levels and 320,187 update
-// blocks, against 83 levels and 445,827 blocks with the relaxed threshold.
+// 50,000 poses with 5,000 loop closures 1,115 levels and 330,444 update
+// blocks, against 99 levels and 461,430 blocks with the relaxed threshold.
 // The numeric work is small either way (0.4 M 6x6 products); the number of
 // dependent levels is what a GPU pays for.
 //
@@ -27,8 +27,8 @@
 // less (the end of the elimination: a clique loses a pose at a time), is one
 // front with several pivots: its columns are the same rows, so one workgroup
 // eliminates them from one copy in LDS.  The levels of the fronts are the
-// heights of the merged tree: 69 -> 20 at 3,000 poses with 601 loop closures,
-// 97 -> 23 at 50,000 with 5,000, 22 -> 14 for 500 planar poses.
+// heights of the merged tree: 84 -> 23 at 3,000 poses with 601 loop closures,
+// 99 -> 25 at 50,000 with 5,000, 20 -> 13 for 500 planar poses with 60.
 #pragma once
 
 #include <algorithm>
@@ -134,8 +134,8 @@ inline LevelLaunch level_launch(const DirectPlan& P, int l) {
 // MB of updates) 197 / 417 ms; 5,000, 10 % (162, 370 MB) 387 / 629 ms; with one
 // pivot a front (wide fronts have one either way) 5,000, 20 % (223, 754 MB) 622
 // / 474 ms; 10,000, 10 % (256, 1.7 GB) 803 / 611 ms.
-// Graphs after PCM stay far below in width (50,000 poses: 26, 135 MB; with
-// 10,000 loop closures 58, 514 MB).
+// Graphs after PCM stay far below in width (50,000 poses with 5,000 loop
+// closures: 32, 140 MB; with 10,000 58, 514 MB).
 struct DirectLimits {
   int max_d = 192;                   // a front's column in LDS: 56 KB
   int64_t max_u = 256ll << 20;       // doubles of update matrices (2 GB), and

@@ -35,8 +35,9 @@ constexpr int kDirectFinishMin = 8192;
 // singular systems reaches 1e-9 of the diagonal, a factor of 1e3 below.
 constexpr double kHoldWeight = 1e-6;
 // A step is undamped up to this lambda: lambda damp is lost in the FP64
-// diagonal (LM reaches 1e-20 to 1e-66 in GNC's later solves).  Down to 1e-15 a
-// free graph's direct and PCG steps move it alike, above 1e-16 within a third.
+// diagonal (LM reaches 1e-20 to 1e-66 in GNC's later solves).  Down to 1e-14 a
+// free graph's direct and PCG steps move it alike to a tenth, at 1e-15 to a
+// sixth, at 1e-16 to a third.
 constexpr double kUndamped = 1e-16;
 
 struct GraphKey {

@@ -127,9 +127,9 @@ def test_direct_equals_pcg(ctx, name):
 
 
 def test_gauss_newton_and_no_prior(ctx):
-    """Gauss-Newton with a prior runs the direct path; without one the matrix
-    is singular: the factorization's pivot test hands the step to the PCG, as
-    an explicit pcg_segment does."""
+    """Gauss-Newton with a prior runs the direct path; without one no factor
+    holds the poses, the matrix is singular and the step is the PCG's, as with
+    an explicit pcg_segment."""
     n, edges, _ = CASES["shuffled_130"]
     g = _graph(n, edges, 9)
     a, _, ra = ctx.solve(*g, solver=_capi.SOLVER_GN)
